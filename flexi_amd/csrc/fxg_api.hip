@@ -59,6 +59,11 @@ std::vector<double> build_basis(int N, int nodeType) {
     out[B.L_HatMinus() + a] = (1.0 / w[a]) * Lm[a];
     out[B.L_HatPlus() + a] = (1.0 / w[a]) * Lp[a];
   }
+  for (int i = 0, x = B.PairD(); i < n; ++i)
+    for (int l = i + 1; l < n; ++l) {
+      out[x++] = D[i + n * l];
+      out[x++] = D[l + n * i];
+    }
   return out;
 }
 

@@ -4,7 +4,7 @@
 //   A  k_visc_faces (fxg_visc.hip): per element, the BR1 gradients at its boundary nodes and, for each of its
 //      six faces, the viscous normal flux f_v . (n SurfElem) seen from that element (4 values per
 //      face point, momentum and energy) into the side array FG.
-//   B  k_dg_fused:   per element, the face fluxes of its six sides (Riemann solver with the
+//   B  k_stage (fxg_stage.hip) in FP64, k_dg_fused (below) in FP32-bulk: per element, the face fluxes of its six sides (Riemann solver with the
 //      neighbour's face state, plus 0.5*(own - neighbour) viscous normal fluxes), the BR1
 //      gradients at all nodes (recomputed, never stored), the split-form volume integral,
 //      Ut=-Ut*sJ, the LSERK register update and the new state's face values for the next stage.
@@ -33,44 +33,35 @@ namespace {
 
 // ---------------------------------------------------------------------------------------------
 // Kernel B: the rest of the stage.
-// One LDS array, carved by phase (values in the working precision RF):
+// One LDS array, carved by phase:
 //  staging to the gather of the surface terms: rows of np 0 rho, 1 p, 2 H, 3 u, 4 v, 5 w, 6 T, 7 E,
 //    then the neighbour face states (7 rows of NF: u, v, w, T, rho, p, E) and the surface
 //    contributions (5 rows of NF);
-//  direction loop: rows 0..5 as before, the metric terms Ja^1, Ja^2, Ja^3 of every node in rows
-//    6..14 (written once, from the registers the lifting loaded them into) and the contravariant
-//    viscous flux of the current direction in rows 15..18.
-// At N=7 that is 19 rows of 512 doubles (76 KB): with the side slots and the basis two workgroups
-// still share a CU's 160 KB, and the metric terms are read from memory once per stage. In FP32-bulk
-// (STAGE false) only the current direction's Ja^d is staged (rows 6..8, read from memory in each
-// direction, viscous flux in rows 9..12), so that four workgroups still share a CU.
-template <int N, bool STAGE>
+//  direction loop: rows 0..5 as before, the current direction's Ja^d in rows 6..8 (read from memory in
+//    each direction, so that four workgroups share a CU), its contravariant viscous flux in rows 9..12.
+template <int N>
 struct LdsB {
   static constexpr int np = D<N>::np, NF = D<N>::NF;
-  static constexpr int FACE = 8 * np;                 // neighbour face states, then surface contributions
-  static constexpr int JA = 6 * np;                   // Ja^1..3 (9 rows), or Ja^d (3 rows)
-  static constexpr int FV = (STAGE ? 15 : 9) * np;    // contravariant viscous flux, 4 rows
+  static constexpr int FACE = 8 * np;  // neighbour face states, then surface contributions
+  static constexpr int JA = 6 * np;    // Ja^d (3 rows)
+  static constexpr int FV = 9 * np;    // contravariant viscous flux, 4 rows
   static constexpr int A = 8 * np + 12 * NF, Bm = FV + 4 * np;
   static constexpr int SIZE = A > Bm ? A : Bm;
 };
 
 // The Riemann solver is a template parameter: each instance then carries only its own solver's
-// code, which keeps the kernel within 128 VGPRs (two workgroups per CU at N=7) without spills.
-// In FP32-bulk the LDS arrays are FP32 (38 KB at N=7) and the kernel is held to 64 VGPRs, so
-// four workgroups share a CU (six waves per SIMD below N=7, where 8 would spill, and in the last
-// stage of a step).
+// code. The LDS arrays are FP32 (38 KB at N=7) and the kernel is held to 64 VGPRs, so four workgroups
+// share a CU (six waves per SIMD below N=7, where 8 would spill, and in the last stage of a step).
 // LAM: the last stage of a step, which also forms CALCTIMESTEP's per-element spectral radii of the
-// new state; in FP64 from the metric terms staged in LDS (the same values as the time-step kernel
-// reads), so they are not read from memory a second time.
+// new state.
 template <int N, class RF, int SOLVER, bool BC, bool LAM>
 __global__ __launch_bounds__(D<N>::NT)
-__attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 && !LAM ? 8 : 6) : 1))) void k_dg_fused(const double* U, DevMesh m, const double* __restrict__ FU,
+__attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(const double* U, DevMesh m, const double* __restrict__ FU,
                                                      double* __restrict__ FUnext, const RF* __restrict__ FG,
                                                      Gas gas, double* Ut, RKStage st, RF* __restrict__ Gout,
                                                      const double* __restrict__ bcP) {
   constexpr int n = D<N>::n, nf = D<N>::nf, np = D<N>::np, NT = D<N>::NT, NF = D<N>::NF;
-  constexpr bool STAGE = sizeof(RF) == 8;  // all metric terms staged once (FP64)
-  using L = LdsB<N, STAGE>;
+  using L = LdsB<N>;
   // LDS holds the working precision RF: the values are rounded to RF where they are stored, as
   // they were rounded where they are read. sA rows: 0 rho, 1 p, 2 H, 3 u, 4 v, 5 w, 6 T, 7 E
   __shared__ __align__(16) RF sL[L::SIZE];
@@ -188,17 +179,10 @@ __attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 && !LAM ? 8 : 6) : 
   const int sides = act ? node_sides<N>(i, j, k) : 0;
   RF acc[5] = {0, 0, 0, 0, 0};
   RF fv[12];  // contravariant viscous flux Ja^d . (f,g,h)_v, d-major
-  // FP64: the node's metric terms, read once, held until the surface terms are gathered and then
-  // staged in LDS for the direction loop
-  RF JaK[STAGE ? 9 : 1] = {};
   double sjd = 0.0;
   if (act) {
     RF Ja[9], sj;
     load_metrics<RF>(m, gid, Ja, sj);
-    if constexpr (STAGE) {
-#pragma unroll
-      for (int r = 0; r < 9; ++r) JaK[r] = Ja[r];
-    }
     RF g[12];
     lift_node<N, RF>(t, sA + 3 * np, sB, sNb, Ja, sj, g);  // u,v,w,T rows
     if (Gout) {  // (np, 12, nElems) like the four-kernel path
@@ -243,22 +227,16 @@ __attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 && !LAM ? 8 : 6) : 
   if (act) {
     rho = (RF)sA[t]; pp = (RF)sA[np + t]; HH = (RF)sA[2 * np + t];
     uu = (RF)sA[3 * np + t]; vv = (RF)sA[4 * np + t]; ww = (RF)sA[5 * np + t];
-    if constexpr (STAGE) {
-#pragma unroll
-      for (int r = 0; r < 9; ++r) sJa[r * np + t] = JaK[r];
-    }
   }
   // the register R and the state U of the update are loaded before the last direction (whose
   // arithmetic then hides their latency; fv of the first two directions no longer holds registers)
   double rpre[5] = {0, 0, 0, 0, 0}, upre[5] = {0, 0, 0, 0, 0};
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    RF* sM = sJa + (STAGE ? 3 * d * np : 0);
+    RF* sM = sJa;
     if (act) {
-      if constexpr (!STAGE) {
-        const double* Jg = (d == 0 ? m.Mf : (d == 1 ? m.Mg : m.Mh)) + 3 * gid;
-        sM[t] = (RF)Jg[0]; sM[np + t] = (RF)Jg[1]; sM[2 * np + t] = (RF)Jg[2];
-      }
+      const double* Jg = (d == 0 ? m.Mf : (d == 1 ? m.Mg : m.Mh)) + 3 * gid;
+      sM[t] = (RF)Jg[0]; sM[np + t] = (RF)Jg[1]; sM[2 * np + t] = (RF)Jg[2];
 #pragma unroll
       for (int c = 0; c < 4; ++c) sF[c * np + t] = fv[4 * d + c];
       if (d == 2 && st.mode != 0) {
@@ -339,12 +317,10 @@ __attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 && !LAM ? 8 : 6) : 
     }
   } else {
     // The spectral radii come before the global stores. The compiler puts a wait for every
-    // outstanding vector-memory operation of the wave before the reduction's cross-lane moves (and
-    // before the metric loads' use in FP32-bulk), which after the stores took the time of their
-    // write-back (about 300 us per launch at 32^3 elements, N=7). The reduction goes through LDS
-    // rows, so that the new state and register stay in registers beside it: within 128 VGPRs in
-    // FP64; in FP32-bulk this instance is held to six waves per SIMD (76 VGPRs) instead of eight,
-    // which spilled.
+    // outstanding vector-memory operation of the wave before the reduction's cross-lane moves and
+    // before the metric loads' use, which after the stores took the time of their write-back. The
+    // reduction goes through LDS rows, so that the new state and register stay in registers beside
+    // it; this instance is held to six waves per SIMD (76 VGPRs) instead of eight, which spilled.
     double rn[5] = {0, 0, 0, 0, 0};
     if (act) {
       sjd = m.sJ[gid];
@@ -358,22 +334,14 @@ __attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 && !LAM ? 8 : 6) : 
     double lam[6] = {0, 0, 0, 0, 0, 0};
     int isnan_rho = 0;
     if (act) {
-      if constexpr (STAGE) {
-        double Jk[9];  // Ja^1..3 of the node as staged (the values the time-step kernel reads)
-#pragma unroll
-        for (int r = 0; r < 9; ++r) Jk[r] = (double)sJa[r * np + t];
-        dt_node_lambda(un, gas, sjd, Jk, Jk + 3, Jk + 6, lam, isnan_rho);
-      } else {  // FP32-bulk: the metric terms from memory (not staged in full)
-        dt_node_lambda(un, gas, sjd, m.Mf + 3 * gid, m.Mg + 3 * gid, m.Mh + 3 * gid, lam, isnan_rho);
-      }
+      dt_node_lambda(un, gas, sjd, m.Mf + 3 * gid, m.Mg + 3 * gid, m.Mh + 3 * gid, lam, isnan_rho);
     }
     double mx[6];
     int nanr = 0;
-    // LDS freed by the direction loop: the rows of 6 NP doubles from the start, the partial maxima
-    // and flags in the viscous-flux rows (FP64; not in the metric rows, which other waves may still
-    // be reading above) or right after them (FP32-bulk, whose metric terms come from memory)
+    // LDS freed by the direction loop: rows of 6 NP doubles from the start, then the partial maxima
+    // and flags
     double* sRd = reinterpret_cast<double*>(sL);
-    double* sPart = STAGE ? reinterpret_cast<double*>(sF) : sRd + 6 * np;
+    double* sPart = sRd + 6 * np;
     block_lambda_max_rows<NT, np>(lam, isnan_rho, sRd, sPart, reinterpret_cast<int*>(sPart + 6), t, mx, nanr);
     if (t == 0) {
       st.lamSum[2 * e] = mx[0] + mx[1] + mx[2];
@@ -451,29 +419,33 @@ hipError_t fused_n(const DevMesh& m, const FusedWork& w, const Gas& gas, int rie
   }
   {
     Scope sc(tm, K_DG_FUSED, s);
-    const double* FUc = w.FU[cur];
-    double* FUn = w.FU[1 - cur];
-    const RF* FG = (const RF*)w.FG;
-#define FXG_LAUNCH(SOLV, BCV)                                                                                       \
-  if (st.lamSum)                                                                                                   \
-    hipLaunchKernelGGL((k_dg_fused<N, RF, SOLV, BCV, true>), dim3(K), dim3(NT), 0, s, U, m, FUc, FUn, FG, gas, Ut,  \
-                       st, (RF*)G, w.bcP);                                                                         \
-  else                                                                                                             \
-    hipLaunchKernelGGL((k_dg_fused<N, RF, SOLV, BCV, false>), dim3(K), dim3(NT), 0, s, U, m, FUc, FUn, FG, gas, Ut, \
-                       st, (RF*)G, w.bcP)
-    if (riemann == 1) {
-      if (bc) FXG_LAUNCH(1, true); else FXG_LAUNCH(1, false);
-    } else if (riemann == 3) {
-      if (bc) FXG_LAUNCH(3, true); else FXG_LAUNCH(3, false);
+    if constexpr (sizeof(RF) == 8) {
+      const hipError_t err = launch_stage(m, w, gas, riemann, U, Ut, st, cur, (double*)G, s);
+      if (err != hipSuccess) return err;
     } else {
-      if (bc) FXG_LAUNCH(33, true); else FXG_LAUNCH(33, false);
-    }
+      const double* FUc = w.FU[cur];
+      double* FUn = w.FU[1 - cur];
+      const RF* FG = (const RF*)w.FG;
+#define FXG_LAUNCH(SOLV, BCV)                                                                                       \
+    if (st.lamSum)                                                                                                   \
+      hipLaunchKernelGGL((k_dg_fused<N, RF, SOLV, BCV, true>), dim3(K), dim3(NT), 0, s, U, m, FUc, FUn, FG, gas, Ut,  \
+                         st, (RF*)G, w.bcP);                                                                         \
+    else                                                                                                             \
+      hipLaunchKernelGGL((k_dg_fused<N, RF, SOLV, BCV, false>), dim3(K), dim3(NT), 0, s, U, m, FUc, FUn, FG, gas, Ut, \
+                         st, (RF*)G, w.bcP)
+      if (riemann == 1) {
+        if (bc) FXG_LAUNCH(1, true); else FXG_LAUNCH(1, false);
+      } else if (riemann == 3) {
+        if (bc) FXG_LAUNCH(3, true); else FXG_LAUNCH(3, false);
+      } else {
+        if (bc) FXG_LAUNCH(33, true); else FXG_LAUNCH(33, false);
+      }
 #undef FXG_LAUNCH
+    }
   }
   return hipGetLastError();
 }
 
-// Packs the FLEXI-layout metric terms (3,np,K) x 3 and sJ (np,K) into rows of np per element.
 // Packs the metric terms of the boundary nodes, (3,np,K) x 3 and sJ (np,K), into rows of NB
 // per element in boundary-node order (bnd_rank).
 template <int N>

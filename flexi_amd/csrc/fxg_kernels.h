@@ -17,7 +17,9 @@ struct BasisLayout {
   __host__ __device__ int L_Plus() const { return 3 * n * n + n; }
   __host__ __device__ int L_HatMinus() const { return 3 * n * n + 2 * n; }
   __host__ __device__ int L_HatPlus() const { return 3 * n * n + 3 * n; }
-  __host__ __device__ int size() const { return 3 * n * n + 4 * n; }
+  // the pairs i < l of the split form in the order (0,1), (0,2), ..: D(i,l), D(l,i)
+  __host__ __device__ int PairD() const { return 3 * n * n + 4 * n; }
+  __host__ __device__ int size() const { return 4 * n * n + 3 * n; }
 };
 
 // Device views of one context's arrays (FLEXI layouts unless noted).
@@ -132,6 +134,9 @@ hipError_t launch_visc_faces(const DevMesh& m, bool fp32, const double* U, const
 // for Riemann-type sides, whose Riemann flux is the boundary flux); bcP the walls' pressure and the
 // Riemann-type boundary states' velocity.
 hipError_t launch_bc_ghost(const DevMesh& m, double* FU, double* bcP, const Gas& gas, hipStream_t s);
+// Kernel B of the fused stage in FP64 (fxg_stage.hip).
+hipError_t launch_stage(const DevMesh& m, const FusedWork& w, const Gas& gas, int riemann, const double* U, double* Ut,
+                        const RKStage& st, int cur, double* G, hipStream_t s);
 hipError_t launch_rhs_fused(const DevMesh& m, const FusedWork& w, const Gas& gas, int riemann, int fp32,
                             const double* U, double* Ut, const RKStage& st, bool faces_fresh, int cur,
                             void* G, hipStream_t s, KernelTimer* timer);
