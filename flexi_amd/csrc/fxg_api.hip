@@ -349,7 +349,7 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
   if (c->fused) {
     char* FG;
     if (alloc_owned(c, &c->fw.FU[0], 10 * face) || alloc_owned(c, &c->fw.FU[1], 10 * face) ||
-        alloc_owned(c, &FG, 8 * face * gsz) || alloc_owned(c, &c->fw.Jsoa, fxg::packed_metrics_size(c->N, K)) ||
+        alloc_owned(c, &FG, 8 * face * gsz) ||
         alloc_owned(c, &c->lamSum, 2 * (size_t)K) || alloc_owned(c, &c->lamNan, (size_t)K) ||
         alloc_owned(c, &c->fw.bcP, 4 * (size_t)c->nf * nBC))
       return 1;
@@ -366,12 +366,20 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
 }
 
 int finish_setup(fxg_ctx* c) {
-  if (c->fused) HIPCHECK(fxg::launch_pack_metrics(c->m, c->fw.Jsoa, c->stream));
   if (c->fused) {  // the fused kernels read the side slots of their face points from this table
     unsigned* slot = nullptr;
     if (alloc_owned(c, &slot, (size_t)6 * c->nf * c->K)) return 1;
     HIPCHECK(fxg::launch_slot_table(c->m, slot, c->stream));
     c->m.slotTab = slot;
+    double* aff = nullptr;
+    bool all = false;
+    if (alloc_owned(c, &aff, (size_t)10 * c->K)) return 1;
+    HIPCHECK(fxg::find_const_metrics(c->m, aff, c->w.errOut, all, c->stream));
+    c->m.aff = all ? aff : nullptr;
+    if (!all) {  // the boundary nodes' metric terms, packed for the viscous face kernel
+      if (alloc_owned(c, &c->fw.Jsoa, fxg::packed_metrics_size(c->N, c->K))) return 1;
+      HIPCHECK(fxg::launch_pack_metrics(c->m, c->fw.Jsoa, c->stream));
+    }
   }
   HIPCHECK(hipStreamSynchronize(c->stream));
   return 0;

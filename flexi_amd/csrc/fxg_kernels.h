@@ -54,6 +54,9 @@ struct DevMesh {
   // face_slot of every own face point of every element, (6*(N+1)^2, nElems), or null (then
   // formed from ElemToSide and the inverse S2V2 map)
   const unsigned* slotTab = nullptr;
+  // metric terms of each element, (10, nElems): Ja^1..3 x,y,z and sJ, where every element has the same
+  // values at all of its nodes; null otherwise
+  const double* aff = nullptr;
 };
 
 // Work arrays of one right-hand side evaluation. Face arrays of U are FP64 (U(5,p,q,side));

@@ -21,4 +21,8 @@ int compute_metrics_gpu(int N, int nodeType, int NGeo, int nElems, const double*
                         double* TangVec1, double* TangVec2, double* SurfElem, double* SlaveNS, bool reference,
                         hipStream_t s, std::string& err);
 
+// Whether every element's metric terms (m.Mf, m.Mg, m.Mh, m.sJ) are bitwise the same at all of its nodes, and
+// those values into aff(10, nElems): Ja^1..3 x,y,z and sJ. `flag` is device scratch of one int.
+hipError_t find_const_metrics(const DevMesh& m, double* aff, int* flag, bool& all, hipStream_t s);
+
 }  // namespace fxg

@@ -7,6 +7,7 @@
 // nodes; surface metrics of each master side from the interpolated face metrics.
 #include "fxg_metrics.h"
 
+#include <algorithm>
 #include <vector>
 
 #include "fxg_basis.h"
@@ -276,6 +277,127 @@ __global__ __launch_bounds__(512) void k_metrics_n(const double* __restrict__ XC
     TangVec2[3 * fp + 1] = nv[2] * t1[0] - nv[0] * t1[2];
     TangVec2[3 * fp + 2] = nv[0] * t1[1] - nv[1] * t1[0];
   }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Affine elements (parallelepipeds). Their metric terms are constants of the element: forming them
+// from its edges gives every node exactly the same values, without the curl form's rounding, and
+// lets the stage kernels read ten numbers per element instead of ten per node.
+
+// Largest absolute coordinate of the mesh, as the bits of a double (nonnegative doubles order as integers).
+__global__ __launch_bounds__(256) void k_coord_max(const double* __restrict__ NC, size_t count,
+                                                 unsigned long long* __restrict__ out) {
+  double x = 0.0;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (size_t)gridDim.x * 256) x = fmax(x, fabs(NC[i]));
+  for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_down(x, off, 64));
+  if ((threadIdx.x & 63) == 0) atomicMax(out, (unsigned long long)__double_as_longlong(x));
+}
+
+// One lane per element: half the mean edge vectors of the three directions, edge[9]; clears *ok where a node is
+// further from the affine map of these edges through the first corner's position (taken from the mean
+// of the corners) than the rounding of the mesh's coordinates.
+__global__ __launch_bounds__(256) void k_affine_edges(const double* __restrict__ NC, int ng, int nElems,
+                                                    const unsigned long long* __restrict__ big,
+                                                    double* __restrict__ edge, int* __restrict__ ok) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= nElems) return;
+  const double* x = NC + (size_t)3 * ng * ng * ng * e;
+  const int G = ng - 1;
+  double h[3][3], mid[3];
+  for (int c = 0; c < 3; ++c) {
+    double v[8];
+    for (int q = 0; q < 8; ++q) v[q] = x[c + 3 * vol_id(ng, (q & 1) * G, ((q >> 1) & 1) * G, (q >> 2) * G)];
+    h[0][c] = 0.125 * (((v[1] - v[0]) + (v[3] - v[2])) + ((v[5] - v[4]) + (v[7] - v[6])));
+    h[1][c] = 0.125 * (((v[2] - v[0]) + (v[3] - v[1])) + ((v[6] - v[4]) + (v[7] - v[5])));
+    h[2][c] = 0.125 * (((v[4] - v[0]) + (v[5] - v[1])) + ((v[6] - v[2]) + (v[7] - v[3])));
+    mid[c] = 0.125 * (((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
+  }
+  for (int d = 0; d < 3; ++d)
+    for (int c = 0; c < 3; ++c) edge[(size_t)9 * e + 3 * d + c] = h[d][c];
+  // a node's coordinates and the eight corners' are each off by a few units in the last place of the
+  // largest coordinate of the mesh (box vertices are lo + i*h)
+  const double tol = 16.0 * 2.220446049250313e-16 * __longlong_as_double((long long)*big);
+  bool fine = true;
+  for (int k = 0; k < ng; ++k)
+    for (int j = 0; j < ng; ++j)
+      for (int i = 0; i < ng; ++i) {
+        const double a = 2.0 * i / G - 1.0, b = 2.0 * j / G - 1.0, cc = 2.0 * k / G - 1.0;
+        for (int c = 0; c < 3; ++c)
+          fine = fine && fabs(x[c + 3 * vol_id(ng, i, j, k)] - (mid[c] + a * h[0][c] + b * h[1][c] + cc * h[2][c])) <= tol;
+      }
+  if (!fine) *ok = 0;
+}
+
+// Metric terms of an affine element at all of its nodes and side points: Ja^1 = b x c, Ja^2 = c x a, Ja^3 = a x b
+// of the half edges, 1/J, and the surface metrics as SurfMetricsFromJa forms them.
+__global__ __launch_bounds__(256) void k_affine_fill(const double* __restrict__ edge, int n, DevMesh m,
+                                                   double* __restrict__ Mf, double* __restrict__ Mg,
+                                                   double* __restrict__ Mh, double* __restrict__ sJ,
+                                                   double* __restrict__ NormVec, double* __restrict__ TangVec1,
+                                                   double* __restrict__ TangVec2, double* __restrict__ SurfElem,
+                                                   double* __restrict__ SlaveNS) {
+  const int e = blockIdx.x, t = threadIdx.x, np = n * n * n, nf = n * n;
+  double h[3][3], J[3][3];
+  for (int d = 0; d < 3; ++d)
+    for (int c = 0; c < 3; ++c) h[d][c] = edge[(size_t)9 * e + 3 * d + c];
+  for (int d = 0; d < 3; ++d) {
+    const double *b = h[(d + 1) % 3], *c = h[(d + 2) % 3];
+    for (int x = 0; x < 3; ++x) J[d][x] = b[(x + 1) % 3] * c[(x + 2) % 3] - b[(x + 2) % 3] * c[(x + 1) % 3];
+  }
+  const double sj = 1.0 / (h[0][0] * J[0][0] + h[0][1] * J[0][1] + h[0][2] * J[0][2]);
+  for (int o = t; o < 3 * np; o += 256) {
+    const size_t g = (size_t)3 * np * e + o;
+    const int x = o % 3;
+    Mf[g] = x == 0 ? J[0][0] : (x == 1 ? J[0][1] : J[0][2]);
+    Mg[g] = x == 0 ? J[1][0] : (x == 1 ? J[1][1] : J[1][2]);
+    Mh[g] = x == 0 ? J[2][0] : (x == 1 ? J[2][1] : J[2][2]);
+  }
+  for (int o = t; o < np; o += 256) sJ[(size_t)np * e + o] = sj;
+  const int NormalDirs[7] = {0, 3, 2, 1, 2, 1, 3}, TangDirs[7] = {0, 1, 3, 2, 3, 2, 1};
+  const double NormalSigns[7] = {0, -1., -1., 1., 1., -1., 1.};
+  for (int x = t; x < 6 * nf; x += 256) {
+    const int ls = x / nf + 1, pq = x - (ls - 1) * nf;
+    const int side = m.E2S[2 * (ls - 1) + 12 * e] - 1, flip = m.E2S[2 * (ls - 1) + 1 + 12 * e];
+    const double *Jn = J[NormalDirs[ls] - 1], *Jt = J[TangDirs[ls] - 1];
+    const double ns = NormalSigns[ls];
+    const size_t fp = (size_t)pq + (size_t)nf * side;
+    if (flip != 0) {
+      if (SlaveNS)
+        for (int c = 0; c < 3; ++c) SlaveNS[3 * fp + c] = -ns * Jn[c];
+      continue;
+    }
+    const double se = sqrt(Jn[0] * Jn[0] + Jn[1] * Jn[1] + Jn[2] * Jn[2]);
+    double nv[3], t1[3];
+    for (int c = 0; c < 3; ++c) nv[c] = ns * Jn[c] / se;
+    const double dot = Jt[0] * nv[0] + Jt[1] * nv[1] + Jt[2] * nv[2];
+    for (int c = 0; c < 3; ++c) t1[c] = Jt[c] - dot * nv[c];
+    const double tn = sqrt(t1[0] * t1[0] + t1[1] * t1[1] + t1[2] * t1[2]);
+    SurfElem[fp] = se;
+    for (int c = 0; c < 3; ++c) {
+      t1[c] /= tn;
+      NormVec[3 * fp + c] = nv[c];
+      TangVec1[3 * fp + c] = t1[c];
+    }
+    TangVec2[3 * fp + 0] = nv[1] * t1[2] - nv[2] * t1[1];
+    TangVec2[3 * fp + 1] = nv[2] * t1[0] - nv[0] * t1[2];
+    TangVec2[3 * fp + 2] = nv[0] * t1[1] - nv[1] * t1[0];
+  }
+}
+
+// Whether every element's metric terms are bitwise the same at all of its nodes (else *ok is cleared), and
+// those values, aff(10, nElems). One workgroup per element.
+__global__ __launch_bounds__(256) void k_const_metrics(DevMesh m, int np, double* __restrict__ aff, int* __restrict__ ok) {
+  const size_t e = blockIdx.x, o = (size_t)np * e;
+  const int t = threadIdx.x;
+  bool same = true;
+  for (int x = t; x < 3 * np; x += 256) {
+    const int c = x % 3;
+    same = same && m.Mf[3 * o + x] == m.Mf[3 * o + c] && m.Mg[3 * o + x] == m.Mg[3 * o + c] &&
+           m.Mh[3 * o + x] == m.Mh[3 * o + c];
+  }
+  for (int x = t; x < np; x += 256) same = same && m.sJ[o + x] == m.sJ[o];
+  if (!same) *ok = 0;
+  if (t < 10) aff[10 * e + t] = t < 3 ? m.Mf[3 * o + t] : (t < 6 ? m.Mg[3 * o + t - 3] : (t < 9 ? m.Mh[3 * o + t - 6] : m.sJ[o]));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -573,11 +695,30 @@ int compute_metrics_gpu(int N, int nodeType, int NGeo, int nElems, const double*
     }
     return 0;
   }
-  double *dm = nullptr, *XCLN = nullptr, *dXCLG = nullptr, *detRef = nullptr;
-  hipError_t e = hipMalloc((void**)&dm, M.total * sizeof(double));
+  double *dm = nullptr, *XCLN = nullptr, *dXCLG = nullptr, *detRef = nullptr, *edge = nullptr;
+  // edge vectors, the largest coordinate and the affine flag
+  hipError_t e = hipMalloc((void**)&edge, ((size_t)9 * nElems + 2) * sizeof(double));
+  int affine = 1;
+  if (e == hipSuccess) {
+    unsigned long long* big = reinterpret_cast<unsigned long long*>(edge + (size_t)9 * nElems);
+    int* ok = reinterpret_cast<int*>(big + 1);
+    const unsigned long long zero = 0;
+    e = hipMemcpyAsync(big, &zero, sizeof(zero), hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(ok, &affine, sizeof(int), hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) {
+      const size_t count = (size_t)3 * ngp * nElems;
+      hipLaunchKernelGGL(k_coord_max, dim3((unsigned)std::min<size_t>(1024, (count + 255) / 256)), dim3(256), 0, s,
+                         NodeCoords, count, big);
+      hipLaunchKernelGGL(k_affine_edges, dim3((nElems + 255) / 256), dim3(256), 0, s, NodeCoords, ng, nElems, big, edge, ok);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(&affine, ok, sizeof(int), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+  }
+  if (e == hipSuccess) e = hipMalloc((void**)&dm, M.total * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&XCLN, (size_t)3 * np * nElems * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&dXCLG, (size_t)9 * ngp * nElems * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void**)&detRef, (size_t)nrp * nElems * sizeof(double));
+  if (e == hipSuccess && !affine) e = hipMalloc((void**)&detRef, (size_t)nrp * nElems * sizeof(double));
   if (e == hipSuccess) e = hipMemcpyAsync(dm, h.data(), M.total * sizeof(double), hipMemcpyHostToDevice, s);
   const size_t shGeo = (size_t)6 * ngp * sizeof(double);
   const size_t shN = (size_t)9 * np * sizeof(double);
@@ -589,12 +730,17 @@ int compute_metrics_gpu(int N, int nodeType, int NGeo, int nElems, const double*
     hipLaunchKernelGGL(k_geo, dim3(nElems), dim3(256), shGeo, s, NodeCoords, dm, M, XCLN, dXCLG, xGP);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) {
+  if (e == hipSuccess && affine) {
+    hipLaunchKernelGGL(k_affine_fill, dim3(nElems), dim3(256), 0, s, edge, n, m, Mf, Mg, Mh, sJ, NormVec, TangVec1,
+                       TangVec2, SurfElem, SlaveNS);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess && !affine) {
     const long tot = (long)nrp * nElems;
     hipLaunchKernelGGL(k_jac_ref, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, dXCLG, dm, M, nElems, detRef);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) {
+  if (e == hipSuccess && !affine) {
     // k_metrics_n keeps up to 4 nodes per lane in registers: np <= 4*512
     hipLaunchKernelGGL(k_metrics_n, dim3(nElems), dim3(512), shN, s, XCLN, dXCLG, detRef, dm, M, NGeo, m, Mf, Mg, Mh,
                        sJ, NormVec, TangVec1, TangVec2, SurfElem, SlaveNS);
@@ -605,11 +751,25 @@ int compute_metrics_gpu(int N, int nodeType, int NGeo, int nElems, const double*
   (void)hipFree(XCLN);
   (void)hipFree(dXCLG);
   (void)hipFree(detRef);
+  (void)hipFree(edge);
   if (e != hipSuccess) {
     if (err.empty()) err = std::string("compute_metrics_gpu: ") + hipGetErrorString(e);
     return 1;
   }
   return 0;
+}
+
+hipError_t find_const_metrics(const DevMesh& m, double* aff, int* flag, bool& all, hipStream_t s) {
+  const int np = (m.N + 1) * (m.N + 1) * (m.N + 1);
+  int ok = 1;
+  hipError_t e = hipMemcpyAsync(flag, &ok, sizeof(int), hipMemcpyHostToDevice, s);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_const_metrics, dim3(m.nElems), dim3(256), 0, s, m, np, aff, flag);
+  e = hipGetLastError();
+  if (e == hipSuccess) e = hipMemcpyAsync(&ok, flag, sizeof(int), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  all = ok != 0;
+  return e;
 }
 
 }  // namespace fxg
