@@ -396,14 +396,17 @@ void ctx_free(fxg_ctx* c) {
 }
 
 // One right-hand side (st.mode 0) or LSERK stage. On the fused path `faces_fresh` says that
-// FU[cur] already holds the face states of U (written by the previous stage).
-int rhs(fxg_ctx* c, const double* U, double* Ut, const fxg::RKStage& st, hipStream_t s, bool faces_fresh = false) {
+// FU[cur] already holds the face states of U (written by the previous stage). `keep_grads`: the fused
+// path's right-hand side also stores the lifted gradients in G (96 bytes per node; only the context's
+// own right-hand side is ever asked for them). The four-kernel path goes through G in any case.
+int rhs(fxg_ctx* c, const double* U, double* Ut, const fxg::RKStage& st, hipStream_t s, bool faces_fresh = false,
+        bool keep_grads = true) {
   if (c->nBC > 0 && !c->bcSet) return fail("the mesh has boundary sides: set their conditions with fxg_set_boundaries");
   if (c->bcNeedsData && !c->bcData)
     return fail("boundary types 12/121 need their states: set BCDataPrim with fxg_set_boundary_data");
   if (c->fused) {
     HIPCHECK(fxg::launch_rhs_fused(c->m, c->fw, c->gas, c->p.riemann, c->p.precision == FXG_PREC_FP32_BULK, U, Ut, st,
-                                   faces_fresh, c->cur, st.mode == 0 ? c->w.G : nullptr, s, c->timer));
+                                   faces_fresh, c->cur, st.mode == 0 && keep_grads ? c->w.G : nullptr, s, c->timer));
     if (st.mode != 0) c->cur ^= 1;
     c->faces_of = U;  // FU[cur] now holds the face values of U (updated in place in RK modes)
     return 0;
@@ -806,9 +809,11 @@ int fxg_dg_time_derivative_dev(fxg_ctx* c, double t, const double* U, double* Ut
   (void)t;
   if (!c || !U || !Ut) return fail("NULL argument");
   fxg::RKStage st{0, 0.0, 0.0, nullptr, nullptr};
-  const int rc = rhs(c, U, Ut, st, stream ? (hipStream_t)stream : c->stream);
+  // the gradients of the caller's state cannot be asked for
+  const int rc = rhs(c, U, Ut, st, stream ? (hipStream_t)stream : c->stream, false, false);
   c->faces_of = nullptr;  // the caller's buffer may change before the next call
-  // G now holds the gradients of the caller's state: the context's are recomputed on request
+  // on the four-kernel path G now holds the gradients of the caller's state: the context's are recomputed
+  // on request
   c->rhs_stale = true;
   c->grads_state = nullptr;
   return rc;
