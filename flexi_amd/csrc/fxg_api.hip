@@ -371,6 +371,15 @@ int finish_setup(fxg_ctx* c) {
     if (alloc_owned(c, &slot, (size_t)6 * c->nf * c->K)) return 1;
     HIPCHECK(fxg::launch_slot_table(c->m, slot, c->stream));
     c->m.slotTab = slot;
+    // the neighbours' nodes, for the first stage on a state without face states (node indices are 32-bit; a mesh
+    // with boundary sides forms its ghost states from the face states)
+    if (c->nBC == 0 && (size_t)c->np * c->K < (1ull << 32)) {
+      unsigned* nb = nullptr;
+      if (alloc_owned(c, &nb, (size_t)6 * c->nf * c->K)) return 1;
+      // (the face fluxes, not in use yet, hold the inverse of the slot table meanwhile)
+      HIPCHECK(fxg::launch_neighbour_nodes(c->m, static_cast<unsigned*>(c->fw.FG), nb, c->stream));
+      c->m.nbNode = nb;
+    }
     double* aff = nullptr;
     bool all = false;
     if (alloc_owned(c, &aff, (size_t)10 * c->K)) return 1;

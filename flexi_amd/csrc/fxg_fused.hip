@@ -417,18 +417,19 @@ hipError_t fused_n(const DevMesh& m, const FusedWork& w, const Gas& gas, int rie
                    const RKStage& st, bool faces_fresh, int cur, void* G, hipStream_t s, KernelTimer* tm) {
   const int K = m.nElems;
   constexpr int NT = D<N>::NT;
-  if (!faces_fresh) {
+  const bool bc = m.nBC > 0;
+  if (!faces_fresh && (bc || !m.nbNode)) {
     Scope sc(tm, K_FACES, s);
     hipLaunchKernelGGL((k_faces_of<N>), dim3(K), dim3(NT), 0, s, U, m, w.FU[cur]);
+    faces_fresh = true;
   }
-  const bool bc = m.nBC > 0;
   {
     Scope sc(tm, K_VISC_FACES, s);
     if (bc) {
       const hipError_t err = launch_bc_ghost(m, w.FU[cur], w.bcP, gas, s);
       if (err != hipSuccess) return err;
     }
-    const hipError_t err = launch_visc_faces(m, sizeof(RF) == 4, U, w.Jsoa, w.FU[cur], w.FG, gas, w.gBC, w.bcP, s);
+    const hipError_t err = launch_visc_faces(m, sizeof(RF) == 4, faces_fresh, U, w.Jsoa, w.FU[cur], w.FG, gas, w.gBC, w.bcP, s);
     if (err != hipSuccess) return err;
   }
   {
@@ -492,7 +493,41 @@ __global__ __launch_bounds__(256) void k_slot_table(DevMesh m, size_t total, uns
   slot[g] = face_slot<N>(m, e, x);
 }
 
+template <int N>
+__global__ __launch_bounds__(256) void k_slot_node(DevMesh m, size_t total, unsigned* __restrict__ slotNode) {
+  constexpr int n = N + 1, nf = n * n, NF = 6 * nf;
+  const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (g >= total) return;
+  const int e = (int)(g / NF), x = (int)(g - (size_t)e * NF);
+  const int ls = x / nf + 1, ab = x - (ls - 1) * nf;
+  slotNode[m.slotTab[g]] = (unsigned)(n * nf) * e + vidx<N>(ls, ab % n, ab / n);
+}
+
+template <int N>
+__global__ __launch_bounds__(256) void k_nb_node(DevMesh m, size_t total, const unsigned* __restrict__ slotNode,
+                                               unsigned* __restrict__ nbNode) {
+  const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (g < total) nbNode[g] = slotNode[slot_nbr<N>(m.slotTab[g])];
+}
+
 }  // namespace
+
+hipError_t launch_neighbour_nodes(const DevMesh& m, unsigned* slotNode, unsigned* nbNode, hipStream_t s) {
+  if (!m.slotTab || m.nBC > 0) return hipErrorInvalidValue;
+  const size_t total = (size_t)6 * (m.N + 1) * (m.N + 1) * m.nElems;
+  const dim3 g((unsigned)((total + 255) / 256)), b(256);
+  switch (m.N) {
+#define FXG_CASE(NN)                                                             \
+  case NN:                                                                       \
+    hipLaunchKernelGGL((k_slot_node<NN>), g, b, 0, s, m, total, slotNode);       \
+    hipLaunchKernelGGL((k_nb_node<NN>), g, b, 0, s, m, total, slotNode, nbNode); \
+    break;
+    FXG_CASE(2) FXG_CASE(3) FXG_CASE(4) FXG_CASE(5) FXG_CASE(6) FXG_CASE(7)
+#undef FXG_CASE
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
 
 hipError_t launch_slot_table(const DevMesh& m, unsigned* slot, hipStream_t s) {
   if (m.slotTab) return hipErrorInvalidValue;

@@ -54,6 +54,8 @@ struct DevMesh {
   // face_slot of every own face point of every element, (6*(N+1)^2, nElems), or null (then
   // formed from ElemToSide and the inverse S2V2 map)
   const unsigned* slotTab = nullptr;
+  // node (index in U) of the neighbour at every own face point, same shape; null on meshes with boundary sides
+  const unsigned* nbNode = nullptr;
   // metric terms of each element, (10, nElems): Ja^1..3 x,y,z and sJ, where every element has the same
   // values at all of its nodes; null otherwise
   const double* aff = nullptr;
@@ -125,13 +127,17 @@ hipError_t launch_faces_of(const DevMesh& m, const double* U, double* FU, hipStr
 hipError_t launch_pack_metrics(const DevMesh& m, double* Jsoa, hipStream_t s);
 // Fills slot(6*(N+1)^2, nElems) with face_slot of every own face point (m.slotTab must be null).
 hipError_t launch_slot_table(const DevMesh& m, unsigned* slot, hipStream_t s);
+// Fills nbNode(6*(N+1)^2, nElems) (m.slotTab set, no boundary sides); slotNode is scratch of 2*(N+1)^2*nSides.
+hipError_t launch_neighbour_nodes(const DevMesh& m, unsigned* slotNode, unsigned* nbNode, hipStream_t s);
 bool fused_supported(int N, int nodeType, int split, long long nSides);
 // One stage of the fused path. FU[cur] must hold the face states of U unless faces_fresh is
 // false, in which case they are rebuilt first. In RK modes the new state's faces go to FU[1-cur].
 // G (optional, (np,12,nElems) of the gradient type) receives the lifted gradients.
-// Kernel A of the fused stage (fxg_visc.hip): viscous normal face fluxes into FG (float if fp32).
-hipError_t launch_visc_faces(const DevMesh& m, bool fp32, const double* U, const double* Jsoa, const double* FU,
-                             void* FG, const Gas& gas, void* gBC, const double* bcP, hipStream_t s);
+// Kernel A of the fused stage (fxg_visc.hip): viscous normal face fluxes into FG (float if fp32). Unless
+// faces_fresh (FU holds the face states of U) it reads the neighbours' states from U and fills FU; that form
+// needs m.nbNode.
+hipError_t launch_visc_faces(const DevMesh& m, bool fp32, bool faces_fresh, const double* U, const double* Jsoa,
+                             double* FU, void* FG, const Gas& gas, void* gBC, const double* bcP, hipStream_t s);
 // Boundary sides on the fused path (fxg_visc.hip): the outer slot of each boundary side point gets a
 // face state whose BR1 lifting difference with the inner state is the boundary lifting flux (and,
 // for Riemann-type sides, whose Riemann flux is the boundary flux); bcP the walls' pressure and the
