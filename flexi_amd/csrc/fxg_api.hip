@@ -159,6 +159,9 @@ struct fxg_ctx {
   EventTimer* timer = nullptr;  // non-null while kernel timing is enabled
   // fused Gauss-Lobatto split-form path: face states double-buffered across LSERK stages
   bool fused = false;
+  // weak form in FP64 without boundary sides: the two line kernels instead of the four (reported as
+  // "classic": the path of every form but the split one); its face states are kept like the fused path's
+  bool weak = false;
   fxg::FusedWork fw{};
   int cur = 0;
   // the state whose face values FU[cur] holds (only trusted for the context's own state, which
@@ -346,6 +349,15 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
   const char* pipe = std::getenv("FXG_PIPELINE");
   c->fused = fxg::fused_supported(c->N, p->nodeType, p->splitDG == FXG_SPLITDG_PI, S) &&
              !(pipe && std::strcmp(pipe, "classic") == 0);
+  c->weak = !c->fused && fxg::weak_supported(c->N, p->nodeType, p->splitDG == FXG_SPLITDG_PI,
+                                             p->precision == FXG_PREC_FP32_BULK, nBC, S) &&
+            !(pipe && std::strcmp(pipe, "classic") == 0);
+  if (c->weak) {
+    double* FG;
+    if (alloc_owned(c, &c->fw.FU[0], 10 * face) || alloc_owned(c, &c->fw.FU[1], 10 * face) || alloc_owned(c, &FG, 8 * face))
+      return 1;
+    c->fw.FG = FG;
+  }
   if (c->fused) {
     char* FG;
     if (alloc_owned(c, &c->fw.FU[0], 10 * face) || alloc_owned(c, &c->fw.FU[1], 10 * face) ||
@@ -366,14 +378,14 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
 }
 
 int finish_setup(fxg_ctx* c) {
-  if (c->fused) {  // the fused kernels read the side slots of their face points from this table
+  if (c->fused || c->weak) {  // these kernels read the side slots of their face points from this table
     unsigned* slot = nullptr;
     if (alloc_owned(c, &slot, (size_t)6 * c->nf * c->K)) return 1;
     HIPCHECK(fxg::launch_slot_table(c->m, slot, c->stream));
     c->m.slotTab = slot;
     // the neighbours' nodes, for the first stage on a state without face states (node indices are 32-bit; a mesh
     // with boundary sides forms its ghost states from the face states)
-    if (c->nBC == 0 && (size_t)c->np * c->K < (1ull << 32)) {
+    if (c->fused && c->nBC == 0 && (size_t)c->np * c->K < (1ull << 32)) {
       unsigned* nb = nullptr;
       if (alloc_owned(c, &nb, (size_t)6 * c->nf * c->K)) return 1;
       // (the face fluxes, not in use yet, hold the inverse of the slot table meanwhile)
@@ -385,7 +397,7 @@ int finish_setup(fxg_ctx* c) {
     if (alloc_owned(c, &aff, (size_t)10 * c->K)) return 1;
     HIPCHECK(fxg::find_const_metrics(c->m, aff, c->w.errOut, all, c->stream));
     c->m.aff = all ? aff : nullptr;
-    if (!all) {  // the boundary nodes' metric terms, packed for the viscous face kernel
+    if (c->fused && !all) {  // the boundary nodes' metric terms, packed for the viscous face kernel
       if (alloc_owned(c, &c->fw.Jsoa, fxg::packed_metrics_size(c->N, c->K))) return 1;
       HIPCHECK(fxg::launch_pack_metrics(c->m, c->fw.Jsoa, c->stream));
     }
@@ -407,7 +419,8 @@ void ctx_free(fxg_ctx* c) {
 // One right-hand side (st.mode 0) or LSERK stage. On the fused path `faces_fresh` says that
 // FU[cur] already holds the face states of U (written by the previous stage). `keep_grads`: the fused
 // path's right-hand side also stores the lifted gradients in G (96 bytes per node; only the context's
-// own right-hand side is ever asked for them). The four-kernel path goes through G in any case.
+// own right-hand side is ever asked for them), and so does the weak form's. The four-kernel path goes
+// through G in any case.
 int rhs(fxg_ctx* c, const double* U, double* Ut, const fxg::RKStage& st, hipStream_t s, bool faces_fresh = false,
         bool keep_grads = true) {
   if (c->nBC > 0 && !c->bcSet) return fail("the mesh has boundary sides: set their conditions with fxg_set_boundaries");
@@ -418,6 +431,13 @@ int rhs(fxg_ctx* c, const double* U, double* Ut, const fxg::RKStage& st, hipStre
                                    faces_fresh, c->cur, st.mode == 0 && keep_grads ? c->w.G : nullptr, s, c->timer));
     if (st.mode != 0) c->cur ^= 1;
     c->faces_of = U;  // FU[cur] now holds the face values of U (updated in place in RK modes)
+    return 0;
+  }
+  if (c->weak) {
+    HIPCHECK(fxg::launch_rhs_weak(c->m, c->fw, c->gas, c->p.nodeType, c->p.riemann, U, Ut, st, faces_fresh, c->cur,
+                                  st.mode == 0 && keep_grads ? (double*)c->w.G : nullptr, s, c->timer));
+    if (st.mode != 0) c->cur ^= 1;
+    c->faces_of = U;
     return 0;
   }
   HIPCHECK(fxg::launch_rhs(c->m, c->w, c->gas, c->p.nodeType, c->p.splitDG == FXG_SPLITDG_PI, c->p.riemann,
@@ -804,7 +824,7 @@ int fxg_timestep_lserkw2(fxg_ctx* c, double t, double dt, int nStages, const dou
   if (!c) return fail("ctx is NULL");
   c->lam_of = nullptr;
   c->grads_state = nullptr;
-  if (lserk(c, dt, nStages, RKA, RKb, c->U, c->R, c->stream, c->fused && c->faces_of == c->U, true)) return 1;
+  if (lserk(c, dt, nStages, RKA, RKb, c->U, c->R, c->stream, (c->fused || c->weak) && c->faces_of == c->U, true)) return 1;
   // Ut of the last stage is not kept by either pipeline, the gradients not by the fused one
   c->rhs_stale = true;
   c->last_rhs = 2;
@@ -935,7 +955,7 @@ int fxg_forward_n_steps(fxg_ctx* c, int nSteps, const double* dt, int nStages, c
     if (ckpt && it % checkpointEvery == 0)
       HIPCHECK(hipMemcpyAsync(ckpt + (size_t)(it / checkpointEvery) * vol5, U, vol5 * sizeof(double),
                               hipMemcpyDeviceToDevice, s));
-    if (lserk(c, dt[it], nStages, RKA, RKb, U, c->R, s, it > 0 && c->fused)) {
+    if (lserk(c, dt[it], nStages, RKA, RKb, U, c->R, s, it > 0 && (c->fused || c->weak))) {
       c->faces_of = nullptr;
       return 1;
     }

@@ -146,6 +146,12 @@ hipError_t launch_bc_ghost(const DevMesh& m, double* FU, double* bcP, const Gas&
 // Kernel B of the fused stage in FP64 (fxg_stage.hip).
 hipError_t launch_stage(const DevMesh& m, const FusedWork& w, const Gas& gas, int riemann, const double* U, double* Ut,
                         const RKStage& st, int cur, double* G, hipStream_t s);
+// One right-hand side or stage of the weak form by the two line kernels (fxg_weak.hip), with FU and FG of
+// FusedWork used as on the fused path. G (optional, (np,12,nElems)) receives the lifted gradients.
+bool weak_supported(int N, int nodeType, int split, int fp32, int nBC, long long nSides);
+hipError_t launch_rhs_weak(const DevMesh& m, const FusedWork& w, const Gas& gas, int nodeType, int riemann,
+                           const double* U, double* Ut, const RKStage& st, bool faces_fresh, int cur, double* G,
+                           hipStream_t s, KernelTimer* timer);
 hipError_t launch_rhs_fused(const DevMesh& m, const FusedWork& w, const Gas& gas, int riemann, int fp32,
                             const double* U, double* Ut, const RKStage& st, bool faces_fresh, int cur,
                             void* G, hipStream_t s, KernelTimer* timer);
