@@ -25,7 +25,7 @@
 // splitflux.f90:603-700, riemann.f90:267-855, fillflux.f90:40-215, surfint.t90:471-616,
 // lifting_br1.t90:48-292, flux.f90:149-241.
 #include "fxg_dual.h"
-#include "fxg_elem.h"
+#include "fxg_line.h"
 
 // FXG_ADJ_DUAL=1 takes the Riemann-flux derivatives from dual-number evaluations instead of the
 // hand-written reverse (a cross-check of the reverse; slower).
@@ -302,426 +302,553 @@ __device__ __forceinline__ void rot_state_adjoint(const double* c, const Gas& g,
 }
 
 // ---------------------------------------------------------------------------------------------
-// Roe without entropy fix at N=5,6 (256/384-lane workgroups of 216/343 active lanes): three waves
-// per SIMD at 168 VGPRs with a 20-28 byte spill instead of two at 174-176. (At N=7 a 512-lane
-// workgroup cannot gain a wave that way; at N=3,4 the spill is larger.)
-template <int N, int SOLVER>
-__global__ __launch_bounds__(D<N>::NT)
-__attribute__((amdgpu_waves_per_eu(SOLVER == 3 && (N == 5 || N == 6) ? 3 : 1))) void k_adj_euler(
-    const double* __restrict__ U, DevMesh m, const double* __restrict__ FUa, double* __restrict__ lam,
-    double* __restrict__ ub, double cub, Gas gas, double* __restrict__ out, double* __restrict__ XU,
-    double* __restrict__ Xg, Pending pd) {
-  constexpr int n = D<N>::n, nf = D<N>::nf, np = D<N>::np, NT = D<N>::NT, NF = D<N>::NF;
-  __shared__ double sA[6 * np];   // rho, p, H, u, v, w
-  __shared__ double sMu[5 * np];  // -sJ*lam
-  __shared__ double sM[3 * np];   // Ja^d of the direction loop
-  __shared__ double sLf[5 * NF];  // Riemann adjoint w.r.t. the own face state, per own face point
-  __shared__ unsigned sIdx[NF];
-  __shared__ double sB[3 * n * n + 4 * n];
+// Both element kernels give each lane a line of nodes, as the forward stage kernel does (fxg_stage.hip): a
+// pair's Jacobian serves both of its nodes, so evaluating it once per pair halves it, and the LDS reads
+// per node fall from about 330 to 90 (k_adj_euler) and from 290 to 110 (k_adj_visc), which bound the forms with
+// one lane per node. TGV 16^3, N=5, Roe, parallelepipeds: 134 -> 112 us and 90 -> 61 us per reverse stage (about 430 and 310
+// bytes per node at 3.4 and 4.5 TB/s). Two waves per SIMD: at three the Riemann reverse spills (143 and 88 us).
+
+// The lane's line: direction, end nodes (offset in the element), local sides and side slots of its ends.
+template <int N>
+struct AdjLine {
+  int d, ln, a, b, first, last, ls[2], fp[2];  // fp: own face points
+  unsigned own[2];
+  __device__ __forceinline__ AdjLine(const DevMesh& m, int e, int t) {
+    constexpr int n = N + 1, nf = n * n;
+    d = t / nf; ln = t - d * nf; a = ln % n; b = ln / n;
+    first = d == 0 ? n * ln : (d == 1 ? a + nf * b : ln);
+    last = first + N * (d == 0 ? 1 : (d == 1 ? n : nf));
+    ls[0] = d == 0 ? 5 : (d == 1 ? 2 : 1);
+    ls[1] = d == 0 ? 3 : (d == 1 ? 4 : 6);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      fp[s] = (ls[s] - 1) * nf + ln;
+      own[s] = m.slotTab[(size_t)6 * nf * e + fp[s]];
+    }
+  }
+};
+
+// Sum over a node's face points (up to three) of the NV values kept per own face point, rows of NF,
+// place (2 d + s) nf + ln.
+template <int N, int NV>
+__device__ __forceinline__ void add_faces(const double* sF, int nd, double* x) {
+  constexpr int n = N + 1, nf = n * n, NF = 6 * nf;
+  const int at[3] = {nd % n, (nd / n) % n, nd / nf};
+  const int ln[3] = {nd / n, at[0] + n * at[2], nd % nf};
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    if (at[d] == 0 || at[d] == N) {
+      const double* f = sF + (2 * d + (at[d] == N ? 1 : 0)) * nf + ln[d];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) x[v] += f[v * NF];
+    }
+}
+
+// LDS rows of k_adj_euler: 0 rho/4, 1 H, 2 u, 3 v, 4 w, 5..9 -sJ*lam; general metrics: 10..18 Ja^1..3 / 2. Then
+// five values per own face point.
+template <int N, bool AFF>
+struct LdsAE {
+  static constexpr int ROWS = AFF ? 10 : 19, FACE = ROWS * S<N>::RS, NF = 6 * S<N>::nf, SIZE = FACE + 5 * NF;
+};
+
+template <int N, int SOLVER, bool AFF>
+__global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_euler(
+    const double* __restrict__ U, DevMesh m, const double* __restrict__ basis, const double* __restrict__ FUa,
+    double* __restrict__ lam, double* __restrict__ ub, double cub, Gas gas, double* __restrict__ out,
+    double* __restrict__ XU, double* __restrict__ Xg, Pending pd) {
+  constexpr int n = S<N>::n, nf = S<N>::nf, np = S<N>::np, NL = S<N>::NL, NT = S<N>::NT, RN = S<N>::RN, RS = S<N>::RS;
+  using L = LdsAE<N, AFF>;
+  __shared__ double sL[L::SIZE];
+  double* sF = sL + L::FACE;
   const BasisLayout B{n};
-  const int e = blockIdx.x, t = threadIdx.x;
-  const bool act = t < np;
-  const size_t gid = (size_t)np * e + (act ? t : 0);
-  const int i = t % n, j = (t / n) % n, k = t / (n * n);
-  // Staging. The independent loads (ElemToSide of the lane's first own face point, the basis, the
-  // node's U, sJ, lam, ub and out) are issued together, before the first wait; all stores come
-  // after the loads (a store between two loads makes the second wait for the first's write-back).
-  constexpr int NBAS = 3 * n * n + 4 * n;
-  static_assert(NBAS <= NT, "one basis entry per lane");
-  const int2 sfe = face_side_entry<N>(m, e, t < NF ? t : 0);  // (lanes t >= NF do not use it)
-  const double bas = t < NBAS ? m.basis[t] : 0.0;
-  double c5[5] = {1.0, 1.0, 1.0, 1.0, 1.0}, l0[5] = {0, 0, 0, 0, 0}, u0[5] = {0, 0, 0, 0, 0},
-         o5[5] = {0, 0, 0, 0, 0}, sj = 0.0;
-  if (act) {
+  const int e = blockIdx.x, t = N == 7 ? (threadIdx.x + 64 * (e & 3)) % NT : threadIdx.x;
+  const bool line = t < NL;
+  const AdjLine<N> q(m, e, line ? t : 0);
+  const size_t e0 = (size_t)np * e;
+  const double* je = AFF ? m.aff + 10 * (size_t)e : nullptr;
+  // Staging: the loads of a lane's nodes are issued together, before the first wait; all stores come after.
+  double c5[RN][5], l0[RN][5], u0[RN][5], o5[RN][5], sj[RN];
 #pragma unroll
-    for (int v = 0; v < 5; ++v) c5[v] = U[5 * gid + v];
-    sj = m.sJ[gid];
+  for (int r = 0; r < RN; ++r) {
+    const bool in = t + r * NT < np;
+    const size_t gid = e0 + (in ? t + r * NT : 0);
 #pragma unroll
-    for (int v = 0; v < 5; ++v) l0[v] = lam[5 * gid + v];
-    if (ub) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) u0[v] = ub[5 * gid + v];
+    for (int v = 0; v < 5; ++v) {
+      c5[r][v] = U[5 * gid + v];
+      l0[r][v] = lam[5 * gid + v];
+      u0[r][v] = ub ? ub[5 * gid + v] : 0.0;
+      o5[r][v] = pd.XU ? out[5 * gid + v] : 0.0;
     }
-    if (pd.XU) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) o5[v] = out[5 * gid + v];
-    }
+    sj[r] = AFF ? je[9] : m.sJ[gid];
   }
-  if (t < NBAS) sB[t] = bas;
-  for (int x = t; x < NF; x += NT) {
-    const unsigned own = face_slot_from<N>(m, x == t ? sfe : face_side_entry<N>(m, e, x), x);
-    sIdx[x] = own;
-    if (pd.XU) {  // the neighbours' face parts, staged in sLf (free until the surface phase)
-      const size_t nb = slot_nbr<N>(own);
+  if (pd.XU) {  // the neighbours' face parts of the previous reverse stage, to the nodes through the face rows
+    if (line) {
 #pragma unroll
-      for (int v = 0; v < 5; ++v) sLf[v * NF + x] = pd.XU[5 * nb + v];
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int v = 0; v < 5; ++v)
+          sF[v * L::NF + (2 * q.d + s) * nf + q.ln] = pd.XU[5 * (size_t)slot_nbr<N>(q.own[s]) + v];
     }
+    __syncthreads();
   }
-  if (pd.XU) __syncthreads();  // uniform over the launch
-  if (act) {
-    const Prim q = cons_to_prim(c5, gas);
-    sA[t] = q.rho; sA[np + t] = q.p; sA[2 * np + t] = (c5[4] + q.p) / q.rho;
-    sA[3 * np + t] = q.u; sA[4 * np + t] = q.v; sA[5 * np + t] = q.w;
+#pragma unroll
+  for (int r = 0; r < RN; ++r) {
+    const int nd = t + r * NT;
+    if (nd >= np) continue;
+    const size_t gid = e0 + nd;
+    const Prim p = cons_to_prim(c5[r], gas);
+    double* s = sL + pos<N>(nd % n, (nd / n) % n, nd / nf);
+    s[0] = 0.25 * p.rho; s[RS] = (c5[r][4] + p.p) * p.srho; s[2 * RS] = p.u; s[3 * RS] = p.v; s[4 * RS] = p.w;
     double l5[5];
     if (pd.XU) {
       // the register update of the previous reverse stage: ub += its out + the neighbours' face
-      // parts, rbar = a*(rbar + cub*ub) (rbar lives in lam)
-      double g5[5];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) g5[v] = o5[v];
-      const int sides = node_sides<N>(i, j, k);
-#pragma unroll 1
-      for (int ls = 1; ls <= 6; ++ls) {
-        if (!(sides & (1 << (ls - 1)))) continue;
-        const int x = face_point<N>(ls, i, j, k);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) g5[v] += sLf[v * NF + x];
-      }
+      // parts, rbar = a*lam of that stage
+      add_faces<N, 5>(sF, nd, o5[r]);
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
-        const double r = pd.a * (l0[v] + pd.cub * u0[v]);
-        const double u1 = u0[v] + g5[v];
-        lam[5 * gid + v] = r;
+        const double u1 = u0[r][v] + o5[r][v];
         ub[5 * gid + v] = u1;
-        l5[v] = r + cub * u1;
+        l5[v] = pd.a * l0[r][v] + cub * u1;
       }
     } else {
 #pragma unroll
-      for (int v = 0; v < 5; ++v) l5[v] = l0[v] + (ub ? cub * u0[v] : 0.0);
+      for (int v = 0; v < 5; ++v) l5[v] = l0[r][v] + cub * u0[r][v];
+    }
+    if (ub) {  // lam of this stage, for k_adj_visc and for the update that is still to come
+#pragma unroll
+      for (int v = 0; v < 5; ++v) lam[5 * gid + v] = l5[v];
     }
 #pragma unroll
-    for (int v = 0; v < 5; ++v) sMu[v * np + t] = -sj * l5[v];
+    for (int v = 0; v < 5; ++v) s[(5 + v) * RS] = -sj[r] * l5[v];
+    if constexpr (!AFF) {
+#pragma unroll
+      for (int x = 0; x < 3; ++x) {
+        s[(10 + x) * RS] = 0.5 * m.Mf[3 * gid + x];
+        s[(13 + x) * RS] = 0.5 * m.Mg[3 * gid + x];
+        s[(16 + x) * RS] = 0.5 * m.Mh[3 * gid + x];
+      }
+    }
   }
+  Line<N> lp(q.d, q.a, q.b);
   __syncthreads();
 
-  // own face points: the neighbour's share of the viscous face term, and the Riemann adjoint
-  for (int x = t; x < NF; x += NT) {
-    const int ls = x / nf + 1, ab = x - (ls - 1) * nf;
-    const int id = vidx<N>(ls, ab % n, ab / n);
-    const unsigned own = sIdx[x];
-    const bool master = slot_is_master<N>(own);
-    const unsigned nb = slot_nbr<N>(own);
-    const double lh = minus_side(ls) ? sB[B.L_HatMinus()] : sB[B.L_HatPlus() + N];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) Xg[4 * (size_t)own + c] = -0.5 * lh * sMu[(1 + c) * np + id];
-    double nv[3], t1[3], t2[3];
-    const double se = face_frame<N, double>(m, e, ls, id, own, master, nv, t1, t2);
-    const double ms = master ? 1.0 : -1.0;
-    double lF[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) lF[v] = ms * se * lh * sMu[v * np + id];
-    const double* Uo = U + 5 * ((size_t)np * e + id);
-    const double* Un = FUa + 5 * (size_t)nb;
-#if FXG_ADJ_DUAL
-    // directional derivatives in dual arithmetic (10 evaluations): the reference for the reverse
-    const Dual nd[3] = {nv[0], nv[1], nv[2]}, t1d[3] = {t1[0], t1[1], t1[2]}, t2d[3] = {t2[0], t2[1], t2[2]};
-    const GasT<Dual> gd(gas);
+  // own face points, the two ends of the line: the neighbour's share of the viscous face term, and the Riemann adjoint
+  if (line) {
 #pragma unroll 1
-    for (int k = 0; k < 10; ++k) {
-      Dual a[5], b[5];
+    for (int s = 0; s < 2; ++s) {
+      const unsigned own = s ? q.own[1] : q.own[0];  // (selected: an index into registers goes through scratch)
+      const bool master = slot_is_master<N>(own);
+      const unsigned nb = slot_nbr<N>(own);
+      const int id = s ? q.last : q.first;
+      const double lh = s ? basis[B.L_HatPlus() + N] : basis[B.L_HatMinus()];
+      const double* me = lp.at(sL, s ? N : 0);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) Xg[4 * (size_t)own + c] = -0.5 * lh * me[(6 + c) * RS];
+      double nv[3], t1[3], t2[3];
+      const double* Jd = AFF ? je + 3 * q.d : (q.d == 0 ? m.Mf : (q.d == 1 ? m.Mg : m.Mh)) + 3 * (e0 + id);
+      const double se = face_frame<N, double>(m, Jd, s ? q.ls[1] : q.ls[0], own, master, nv, t1, t2);
+      const double ms = master ? 1.0 : -1.0;
+      double lF[5];
+#pragma unroll
+      for (int v = 0; v < 5; ++v) lF[v] = ms * se * lh * me[(5 + v) * RS];
+      const double* Uo = U + 5 * (e0 + id);
+      const double* Un = FUa ? FUa + 5 * (size_t)nb : U + 5 * (size_t)m.nbNode[(size_t)L::NF * e + (s ? q.fp[1] : q.fp[0])];
+      double* dst = sF + (2 * q.d + s) * nf + q.ln;
+#if FXG_ADJ_DUAL
+      // directional derivatives in dual arithmetic (10 evaluations): the reference for the reverse
+      const Dual nd[3] = {nv[0], nv[1], nv[2]}, t1d[3] = {t1[0], t1[1], t1[2]}, t2d[3] = {t2[0], t2[1], t2[2]};
+      const GasT<Dual> gd(gas);
+#pragma unroll 1
+      for (int k = 0; k < 10; ++k) {
+        Dual a[5], b[5];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+          a[v] = Dual(Uo[v], k == v ? 1.0 : 0.0);
+          b[v] = Dual(Un[v], k == 5 + v ? 1.0 : 0.0);
+        }
+        const RotState<Dual> So = rot_state(a, gas.kappaM1, nd, t1d, t2d);
+        const RotState<Dual> Sn = rot_state(b, gas.kappaM1, nd, t1d, t2d);
+        Dual F[5];
+        if (master) riemann_rot<Dual>(gd, SOLVER, true, So, Sn, F);
+        else riemann_rot<Dual>(gd, SOLVER, true, Sn, So, F);
+        double x = lF[0] * F[0].d + lF[4] * F[4].d;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) x += lF[1 + c] * (nv[c] * F[1].d + t1[c] * F[2].d + t2[c] * F[3].d);
+        if (k < 5) dst[k * L::NF] = x;
+        else XU[5 * (size_t)own + (k - 5)] = x;
+      }
+#else
+      // flux adjoint in the side frame, then the reverse of the Riemann solver and of the rotation
+      double lFr[5];
+      lFr[0] = lF[0];
+      lFr[1] = nv[0] * lF[1] + nv[1] * lF[2] + nv[2] * lF[3];
+      lFr[2] = t1[0] * lF[1] + t1[1] * lF[2] + t1[2] * lF[3];
+      lFr[3] = t2[0] * lF[1] + t2[1] * lF[2] + t2[2] * lF[3];
+      lFr[4] = lF[4];
+      const Prim po = cons_to_prim(Uo, gas), pn = cons_to_prim(Un, gas);
+      const RotState<double> So = rotate<double>(po.rho, Uo[4], po.p, po.u, po.v, po.w, nv, t1, t2);
+      const RotState<double> Sn = rotate<double>(pn.rho, Un[4], pn.p, pn.u, pn.v, pn.w, nv, t1, t2);
+      // the master's state on the left, operands selected rather than branched on (one copy of the
+      // reverse; a wave may hold master and slave points)
+      const RotState<double> SL = master ? So : Sn, SR = master ? Sn : So;
+      RotAdj aL, aR;
+      riemann_rot_vjp<SOLVER>(gas, SL, SR, lFr, aL, aR);
+      const RotAdj ao = master ? aL : aR, an = master ? aR : aL;
+      double gOwn[5], gNb[5];
+      rot_state_adjoint(Uo, gas, nv, t1, t2, ao, gOwn);
+      rot_state_adjoint(Un, gas, nv, t1, t2, an, gNb);
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
-        a[v] = Dual(Uo[v], k == v ? 1.0 : 0.0);
-        b[v] = Dual(Un[v], k == 5 + v ? 1.0 : 0.0);
+        dst[v * L::NF] = gOwn[v];
+        XU[5 * (size_t)own + v] = gNb[v];
       }
-      const RotState<Dual> So = rot_state(a, gas.kappaM1, nd, t1d, t2d);
-      const RotState<Dual> Sn = rot_state(b, gas.kappaM1, nd, t1d, t2d);
-      Dual F[5];
-      if (master) riemann_rot<Dual>(gd, SOLVER, true, So, Sn, F);
-      else riemann_rot<Dual>(gd, SOLVER, true, Sn, So, F);
-      double s = lF[0] * F[0].d + lF[4] * F[4].d;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) s += lF[1 + c] * (nv[c] * F[1].d + t1[c] * F[2].d + t2[c] * F[3].d);
-      if (k < 5) sLf[k * NF + x] = s;
-      else XU[5 * (size_t)own + (k - 5)] = s;
-    }
-#else
-    // flux adjoint in the side frame, then the reverse of the Riemann solver and of the rotation
-    double lFr[5];
-    lFr[0] = lF[0];
-    lFr[1] = nv[0] * lF[1] + nv[1] * lF[2] + nv[2] * lF[3];
-    lFr[2] = t1[0] * lF[1] + t1[1] * lF[2] + t1[2] * lF[3];
-    lFr[3] = t2[0] * lF[1] + t2[1] * lF[2] + t2[2] * lF[3];
-    lFr[4] = lF[4];
-    const Prim po = cons_to_prim(Uo, gas), pn = cons_to_prim(Un, gas);
-    const RotState<double> So = rotate<double>(po.rho, Uo[4], po.p, po.u, po.v, po.w, nv, t1, t2);
-    const RotState<double> Sn = rotate<double>(pn.rho, Un[4], pn.p, pn.u, pn.v, pn.w, nv, t1, t2);
-    // the master's state on the left, operands selected rather than branched on (one copy of the
-    // reverse; a wave may hold master and slave points)
-    const RotState<double> SL = master ? So : Sn, SR = master ? Sn : So;
-    RotAdj aL, aR;
-    riemann_rot_vjp<SOLVER>(gas, SL, SR, lFr, aL, aR);
-    const RotAdj ao = master ? aL : aR, an = master ? aR : aL;
-    double gOwn[5], gNb[5];
-    rot_state_adjoint(Uo, gas, nv, t1, t2, ao, gOwn);
-    rot_state_adjoint(Un, gas, nv, t1, t2, an, gNb);
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-      sLf[v * NF + x] = gOwn[v];
-      XU[5 * (size_t)own + v] = gNb[v];
-    }
 #endif
+    }
   }
 
-  // split-flux adjoint: each pair (i,l) contributes J_s^T (DV(l,i) mu_i + DV(i,l) mu_l) to both
+  // split-flux adjoint: each pair (i,l) contributes J_s^T (D(i,l) mu_i + D(l,i) mu_l) to both
   // nodes' primitive adjoints, J_s the flux Jacobian w.r.t. the pair sums (rho,u,v,w,p,H)
-  double lrho = 0, lu = 0, lv = 0, lw = 0, lp = 0, lH = 0;
-  double rho = 0, uu = 0, vv = 0, ww = 0, pp = 0, HH = 0, mu[5] = {0, 0, 0, 0, 0};
-  if (act) {
-    rho = sA[t]; pp = sA[np + t]; HH = sA[2 * np + t]; uu = sA[3 * np + t]; vv = sA[4 * np + t]; ww = sA[5 * np + t];
+  double acc[6][n];  // rho, u, v, w, p, H
+  if (line) {
 #pragma unroll
-    for (int v = 0; v < 5; ++v) mu[v] = sMu[v * np + t];
-  }
-  const double* DV = sB + B.DVolSurf();
-#pragma unroll 1
-  for (int d = 0; d < 3; ++d) {
-    double m0 = 0, m1 = 0, m2 = 0;
-    if (act) {
-      const double* Jg = (d == 0 ? m.Mf : (d == 1 ? m.Mg : m.Mh)) + 3 * gid;
-      m0 = Jg[0]; m1 = Jg[1]; m2 = Jg[2];
-      sM[t] = m0; sM[np + t] = m1; sM[2 * np + t] = m2;
+    for (int v = 0; v < 6; ++v)
+#pragma unroll
+      for (int i = 0; i < n; ++i) acc[v][i] = 0.0;
+    const double* W = basis + B.PairD() + fresh();
+    lp.again();
+    double* sJ9 = sL + (10 + 3 * q.d) * RS;
+    struct Nd {
+      double r, H, u, v, w, mu[5], j[3];
+    };
+    double mj[3] = {0, 0, 0};
+    if constexpr (AFF) {
+#pragma unroll
+      for (int x = 0; x < 3; ++x) mj[x] = q.d == 0 ? je[x] : (q.d == 1 ? je[3 + x] : je[6 + x]);
     }
-    __syncthreads();
-    if (act) {
-      const int me = d == 0 ? i : (d == 1 ? j : k);
-      const int stride = d == 0 ? 1 : (d == 1 ? n : n * n);
-      const int base = t - me * stride;
+    auto load = [&](int l) {
+      const double* s = lp.at(sL, l);
+      Nd x;
+      x.r = s[0]; x.H = s[RS]; x.u = s[2 * RS]; x.v = s[3 * RS]; x.w = s[4 * RS];
 #pragma unroll
-      for (int l = 0; l <= N; ++l) {
-        if (l == me) continue;
-        const int id = base + l * stride;
-        const double rs = rho + sA[id];
-        const double us = uu + sA[3 * np + id], vs = vv + sA[4 * np + id], ws = ww + sA[5 * np + id];
-        const double Hs = HH + sA[2 * np + id];
-        const double a0 = 0.5 * (m0 + sM[id]), a1 = 0.5 * (m1 + sM[np + id]), a2 = 0.5 * (m2 + sM[2 * np + id]);
-        const double mv = a0 * us + a1 * vs + a2 * ws;
-        const double qq = 0.25 * rs * mv;
-        const double wi = DV[l + n * me], wl = DV[me + n * l];
+      for (int c = 0; c < 5; ++c) x.mu[c] = s[(5 + c) * RS];
+      if constexpr (!AFF) {
+        const double* J = lp.at(sJ9, l);
+        x.j[0] = J[0]; x.j[1] = J[RS]; x.j[2] = J[2 * RS];
+      }
+      return x;
+    };
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const Nd A = load(i);
+#pragma unroll
+      for (int l = i + 1; l < n; ++l) {
+        const Nd C = load(l);
+        const int pr = i * (2 * n - i - 1) / 2 + l - i - 1;
+        const double wi = W[2 * pr], wl = W[2 * pr + 1];
+        double a0, a1, a2;
+        if constexpr (AFF) {
+          a0 = mj[0]; a1 = mj[1]; a2 = mj[2];
+        } else {
+          a0 = A.j[0] + C.j[0]; a1 = A.j[1] + C.j[1]; a2 = A.j[2] + C.j[2];
+        }
+        const double us = A.u + C.u, vs = A.v + C.v, ws = A.w + C.w, Hs = A.H + C.H, rq = A.r + C.r;  // rq: rho sum / 4
+        const double mv = a0 * us + a1 * vs + a2 * ws, qq = rq * mv;
         double vec[5];
 #pragma unroll
-        for (int c = 0; c < 5; ++c) vec[c] = wi * mu[c] + wl * sMu[c * np + id];
-        const double beta = 0.5 * vec[0] + 0.25 * (vec[1] * us + vec[2] * vs + vec[3] * ws) + 0.25 * Hs * vec[4];
-        lrho += mv * beta;
-        lu += a0 * rs * beta + qq * vec[1];
-        lv += a1 * rs * beta + qq * vec[2];
-        lw += a2 * rs * beta + qq * vec[3];
-        lp += a0 * vec[1] + a1 * vec[2] + a2 * vec[3];
-        lH += qq * vec[4];
+        for (int c = 0; c < 5; ++c) vec[c] = wi * A.mu[c] + wl * C.mu[c];
+        const double beta = 2.0 * vec[0] + (vec[1] * us + vec[2] * vs + vec[3] * ws) + Hs * vec[4];  // times 4
+        const double rb = rq * beta;
+        const double x[6] = {0.25 * mv * beta,        a0 * rb + qq * vec[1], a1 * rb + qq * vec[2],
+                             a2 * rb + qq * vec[3],   a0 * vec[1] + a1 * vec[2] + a2 * vec[3], qq * vec[4]};
+#pragma unroll
+        for (int v = 0; v < 6; ++v) {
+          acc[v][i] += x[v];
+          acc[v][l] += x[v];
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
+  }
+  __syncthreads();  // the pair loop's rows are free
+  // the three directions' sums at the nodes, VR variables at a time
+  constexpr int VR = L::ROWS >= 18 ? 6 : 3;
+  double sum[RN][6];
+#pragma unroll
+  for (int v0 = 0; v0 < 6; v0 += VR) {
+    if (line) {
+      lp.again();
+      double* sS = sL + VR * q.d * RS;
+#pragma unroll
+      for (int v = 0; v < VR; ++v)
+#pragma unroll
+        for (int i = 0; i < n; ++i) lp.at(sS, i)[v * RS] = acc[v0 + v][i];
+    }
     __syncthreads();
-  }
-  if (!act) return;
-  const Prim q = cons_to_prim(U + 5 * gid, gas);
-  double lU[5];
-  prim_adjoint(q, U[5 * gid + 4], gas, lrho, lu, lv, lw, lp, 0.0, lH, lU);
-  const int sides = node_sides<N>(i, j, k);
-#pragma unroll 1
-  for (int ls = 1; ls <= 6; ++ls) {
-    if (!(sides & (1 << (ls - 1)))) continue;
-    const int x = face_point<N>(ls, i, j, k);
 #pragma unroll
-    for (int v = 0; v < 5; ++v) lU[v] += sLf[v * NF + x];
+    for (int r = 0; r < RN; ++r) {
+      const int nd = t + r * NT < np ? t + r * NT : 0;
+      const double* s = sL + pos<N>(nd % n, (nd / n) % n, nd / nf);
+#pragma unroll
+      for (int v = 0; v < VR; ++v) sum[r][v0 + v] = s[v * RS] + s[(VR + v) * RS] + s[(2 * VR + v) * RS];
+    }
+    if (v0 + VR < 6) __syncthreads();
   }
 #pragma unroll
-  for (int v = 0; v < 5; ++v) out[5 * gid + v] = lU[v];
+  for (int r = 0; r < RN; ++r) {
+    const int nd = t + r * NT;
+    if (nd >= np) continue;
+    const size_t gid = e0 + nd;
+    double cc[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) cc[v] = U[5 * gid + v];
+    const Prim p = cons_to_prim(cc, gas);
+    double lU[5];
+    prim_adjoint(p, cc[4], gas, sum[r][0], sum[r][1], sum[r][2], sum[r][3], sum[r][4], 0.0, sum[r][5], lU);
+    add_faces<N, 5>(sF, nd, lU);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) out[5 * gid + v] = lU[v];
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
 // XU: the Riemann part of the neighbour's face adjoint (k_adj_euler); the lifting part w.r.t. the
 // neighbour's (u,v,w,T), taken to its conservative variables with its face state, is added here.
-template <int N>
-__global__ __launch_bounds__(D<N>::NT) __attribute__((amdgpu_waves_per_eu(4))) void k_adj_visc(const double* __restrict__ U, DevMesh m,
-                                                     const double* __restrict__ FUa, const double* __restrict__ lam,
-                                                     const double* __restrict__ ub, double cub,
-                                                     const double* __restrict__ Xg, Gas gas, double* __restrict__ out,
-                                                     double* __restrict__ XU) {
-  constexpr int n = D<N>::n, np = D<N>::np, NT = D<N>::NT, NF = D<N>::NF;
-  // sW: u, v, w, T (rows 0-3) and -sJ*lam of momentum and energy (rows 4-7) until the node
-  // values are formed, then the lifting adjoint per reference derivative (rows 4*d + var)
-  __shared__ double sW[12 * np];
-  double* sP = sW;
-  double* sMu = sW + 4 * np;
-  double* sK = sW;
-  __shared__ double sNb[5 * NF];   // neighbour u, v, w, T, rho per own face point
-  __shared__ unsigned sIdx[NF];
-  __shared__ double sB[3 * n * n + 4 * n];
+// LDS rows: 0 u, 1 v, 2 w, 3 T, 4..7 -sJ*lam of momentum and energy, 8..13 exchange between line and node phases
+// (two variables in three directions).
+template <int N, bool AFF>
+__global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(N <= 4 ? 3 : 2))) void k_adj_visc(
+    const double* __restrict__ U, DevMesh m, const double* __restrict__ basis, const double* __restrict__ FUa,
+    const double* __restrict__ lam, const double* __restrict__ Xg, Gas gas, double* __restrict__ out,
+    double* __restrict__ XU) {
+  constexpr int n = S<N>::n, nf = S<N>::nf, np = S<N>::np, NL = S<N>::NL, NT = S<N>::NT, RN = S<N>::RN, RS = S<N>::RS;
+  constexpr int X = 8;
+  __shared__ double sL[14 * RS];
   const BasisLayout B{n};
-  const int e = blockIdx.x, t = threadIdx.x;
-  const bool act = t < np;
-  const size_t gid = (size_t)np * e + (act ? t : 0);
-  // Staging: the independent loads (ElemToSide of the lane's first own face point, the basis, the
-  // node's U, sJ, lam and ub) are issued together, before the first wait.
-  constexpr int NBAS = 3 * n * n + 4 * n;
-  static_assert(NBAS <= NT, "one basis entry per lane");
-  const int2 sfe = face_side_entry<N>(m, e, t < NF ? t : 0);  // (lanes t >= NF do not use it)
-  const double bas = t < NBAS ? m.basis[t] : 0.0;
-  double c5[5] = {1.0, 1.0, 1.0, 1.0, 1.0}, l4[4] = {0, 0, 0, 0}, u4[4] = {0, 0, 0, 0}, sjn = 0.0;
-  if (act) {
+  const int e = blockIdx.x, t = N == 7 ? (threadIdx.x + 64 * (e & 3)) % NT : threadIdx.x;
+  const bool line = t < NL;
+  const AdjLine<N> q(m, e, line ? t : 0);
+  const size_t e0 = (size_t)np * e;
+  const double* je = AFF ? m.aff + 10 * (size_t)e : nullptr;
+  double c5[RN][5], l4[RN][4], sj[RN];
 #pragma unroll
-    for (int v = 0; v < 5; ++v) c5[v] = U[5 * gid + v];
-    sjn = m.sJ[gid];
+  for (int r = 0; r < RN; ++r) {
+    const size_t gid = e0 + (t + r * NT < np ? t + r * NT : 0);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) l4[c] = lam[5 * gid + 1 + c];
-    if (ub) {
+    for (int v = 0; v < 5; ++v) c5[r][v] = U[5 * gid + v];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) u4[c] = ub[5 * gid + 1 + c];
+    for (int c = 0; c < 4; ++c) l4[r][c] = lam[5 * gid + 1 + c];
+    sj[r] = AFF ? je[9] : m.sJ[gid];
+  }
+  double fn[2][5], xg[2][4];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const size_t nb = slot_nbr<N>(q.own[s]);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) fn[s][v] = FUa ? FUa[5 * nb + v] : U[5 * (size_t)m.nbNode[(size_t)6 * nf * e + q.fp[s]] + v];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) xg[s][c] = Xg[4 * nb + c];
+  }
+  int place[RN];
+#pragma unroll
+  for (int r = 0; r < RN; ++r) {
+    const int nd = t + r * NT < np ? t + r * NT : 0;
+    place[r] = pos<N>(nd % n, (nd / n) % n, nd / nf);
+    if (t + r * NT < np) {
+      const Prim p = cons_to_prim(c5[r], gas);
+      double* s = sL + place[r];
+      s[0] = p.u; s[RS] = p.v; s[2 * RS] = p.w; s[3 * RS] = p.T;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s[(4 + c) * RS] = -sj[r] * l4[r][c];
     }
   }
-  if (t < NBAS) sB[t] = bas;
-  Prim q{};
-  if (act) {
-    q = cons_to_prim(c5, gas);
-    sP[t] = q.u; sP[np + t] = q.v; sP[2 * np + t] = q.w; sP[3 * np + t] = q.T;
+  Prim qn[2];  // the neighbours' face states
 #pragma unroll
-    for (int c = 0; c < 4; ++c) sMu[c * np + t] = -sjn * (l4[c] + (ub ? cub * u4[c] : 0.0));
-  }
-  // where rows 8..11 of sW (free until the lifting adjoint is formed) hold NF values, the
-  // neighbours' viscous shares Xg are staged there with the face states, so that the side loop
-  // below reads them from LDS instead of waiting for one load per side
-  constexpr bool XG_LDS = np >= NF;  // N >= 5
-  double* sXg = sW + 8 * np;
-  for (int x = t; x < NF; x += NT) {
-    const unsigned own = face_slot_from<N>(m, x == t ? sfe : face_side_entry<N>(m, e, x), x);
-    sIdx[x] = own;
-    const size_t nb = slot_nbr<N>(own);
-    if constexpr (XG_LDS) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) sXg[c * NF + x] = Xg[4 * nb + c];
-    }
-    const Prim qn = cons_to_prim(FUa + 5 * nb, gas);
-    sNb[x] = qn.u; sNb[NF + x] = qn.v; sNb[2 * NF + x] = qn.w; sNb[3 * NF + x] = qn.T; sNb[4 * NF + x] = qn.rho;
-  }
+  for (int s = 0; s < 2; ++s) qn[s] = cons_to_prim(fn[s], gas);
+  Line<N> lp(q.d, q.a, q.b);
+  const double lhm = basis[B.L_HatMinus()], lhp = basis[B.L_HatPlus() + N];
   __syncthreads();
-  const int i = t % n, j = (t / n) % n, k = t / (n * n);
-  const int sides = act ? node_sides<N>(i, j, k) : 0;
-  double Ja[9], sj = 0;
-  double lq[4] = {0, 0, 0, 0};  // adjoint of u, v, w, T at this node
-  double nu[12];
-  if (act) {
-    load_metrics<double>(m, gid, Ja, sj);
-    double g[12];
-    lift_node<N, double>(t, sP, sB, sNb, Ja, sj, g);
-    // adjoint of the viscous flux vectors fx, fy, fz (momentum and energy rows)
-    double lf[3][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
-    const double* DH = sB + B.D_Hat_T();
+  double jq[2][4];  // BR1 jumps with their sign and weight
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const int me = d == 0 ? i : (d == 1 ? j : k);
-      const int stride = d == 0 ? 1 : (d == 1 ? n : n * n);
-      const int base = t - me * stride;
-      double lc[4] = {0, 0, 0, 0};
-      for (int l = 0; l <= N; ++l) {
-        const double w = DH[me + n * l];
+  for (int s = 0; s < 2; ++s) {
+    const double* o = lp.at(sL, s ? N : 0);
+    const double h = s ? 0.5 * lhp : -0.5 * lhm;
+    jq[s][0] = h * (qn[s].u - o[0]); jq[s][1] = h * (qn[s].v - o[RS]); jq[s][2] = h * (qn[s].w - o[2 * RS]);
+    jq[s][3] = h * (qn[s].T - o[3 * RS]);
+  }
+  // to the nodes: the reference derivatives of u,v,w,T (g) and, from the adjoint of the viscous flux, the
+  // transposed weak derivative of mu along each direction with the face terms at the ends (lc)
+  double g[RN][12], lc[RN][12];  // [d][variable]
 #pragma unroll
-        for (int c = 0; c < 4; ++c) lc[c] += w * sMu[c * np + base + l * stride];
+  for (int h = 0; h < 4; ++h) {
+    const int w0 = 2 * (h & 1);
+    if (line) {
+      const double* M = basis + (h < 2 ? B.D_T() : B.D_Hat_T()) + fresh();
+      lp.again();
+      double* sX = sL + (X + 2 * q.d) * RS;
+      double x[2][n];
+#pragma unroll
+      for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (int l = 0; l < n; ++l) x[w][l] = lp.at(sL, l)[((h < 2 ? 0 : 4) + w0 + w) * RS];
+      double y[2][n];
+#pragma unroll
+      for (int l = 0; l < n; ++l)
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            // D_T(l,i) for the derivative at i; D_Hat_T(i,l) for its transpose
+            const double z = (h < 2 ? M[l + n * i] : M[i + n * l]) * x[w][l];
+            y[w][i] = l == 0 ? z : y[w][i] + z;
+          }
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        if (h < 2) {
+          y[w][0] += jq[0][w0 + w];
+          y[w][N] += jq[1][w0 + w];
+        } else {
+          y[w][0] -= 0.5 * lhm * x[w][0] + xg[0][w0 + w];
+          y[w][N] += 0.5 * lhp * x[w][N] + xg[1][w0 + w];
+        }
+#pragma unroll
+        for (int i = 0; i < n; ++i) lp.at(sX, i)[w * RS] = y[w][i];
       }
-#pragma unroll
-      for (int x = 0; x < 3; ++x)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) lf[x][c] += Ja[3 * d + x] * lc[c];
     }
-#pragma unroll 1
-    for (int ls = 1; ls <= 6; ++ls) {
-      if (!(sides & (1 << (ls - 1)))) continue;
-      const int dir = dir_of(ls);
-      const double sg = normal_sign(ls);
-      const double lh = minus_side(ls) ? sB[B.L_HatMinus()] : sB[B.L_HatPlus() + N];
-      const int x = face_point<N>(ls, i, j, k);
-      const double* xg = Xg + 4 * (size_t)slot_nbr<N>(sIdx[x]);
+    __syncthreads();
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const double a = 0.5 * lh * sMu[c * np + t] + (XG_LDS ? sXg[c * NF + x] : xg[c]);
+    for (int r = 0; r < RN; ++r)
 #pragma unroll
-        for (int r = 0; r < 3; ++r) lf[r][c] += a * sg * Ja[3 * dir + r];
+      for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int w = 0; w < 2; ++w) (h < 2 ? g : lc)[r][4 * d + w0 + w] = sL[(X + 2 * d + w) * RS + place[r]];
+    __syncthreads();
+  }
+  // node lanes: in place of g the adjoint per reference derivative kappa^d = Ja^d . nu, in lq that of u,v,w
+  double lq[RN][4];
+#pragma unroll
+  for (int r = 0; r < RN; ++r) {
+    double Ja[9], sjr = sj[r];
+    if constexpr (AFF) {
+#pragma unroll
+      for (int x = 0; x < 9; ++x) Ja[x] = je[x];
+    } else {
+      double z;
+      load_metrics<double>(m, e0 + (t + r * NT < np ? t + r * NT : 0), Ja, z);
+    }
+    double p[12], lf[3][4];
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        p[4 * x + v] = (Ja[x] * g[r][v] + Ja[3 + x] * g[r][4 + v] + Ja[6 + x] * g[r][8 + v]) * sjr;
+        lf[x][v] = Ja[x] * lc[r][v] + Ja[3 + x] * lc[r][4 + v] + Ja[6 + x] * lc[r][8 + v];
       }
-    }
     // diff_flux adjoint (flux.f90:149-241): stresses, velocities, temperature gradient
     const double mu0 = gas.mu0;
-    const double txx = mu0 * (gas.s43 * g[0] - gas.s23 * g[5] - gas.s23 * g[10]);
-    const double tyy = mu0 * (-gas.s23 * g[0] + gas.s43 * g[5] - gas.s23 * g[10]);
-    const double tzz = mu0 * (-gas.s23 * g[0] - gas.s23 * g[5] + gas.s43 * g[10]);
-    const double txy = mu0 * (g[4] + g[1]), txz = mu0 * (g[8] + g[2]), tyz = mu0 * (g[9] + g[6]);
-    const double u = q.u, v = q.v, w = q.w;
+    const double txx = mu0 * (gas.s43 * p[0] - gas.s23 * p[5] - gas.s23 * p[10]);
+    const double tyy = mu0 * (-gas.s23 * p[0] + gas.s43 * p[5] - gas.s23 * p[10]);
+    const double tzz = mu0 * (-gas.s23 * p[0] - gas.s23 * p[5] + gas.s43 * p[10]);
+    const double txy = mu0 * (p[4] + p[1]), txz = mu0 * (p[8] + p[2]), tyz = mu0 * (p[9] + p[6]);
+    const double* sn = sL + place[r];
+    const double u = sn[0], v = sn[RS], w = sn[2 * RS];
     const double ltxx = -lf[0][0] - u * lf[0][3];
     const double ltxy = -lf[0][1] - v * lf[0][3] - lf[1][0] - u * lf[1][3];
     const double ltxz = -lf[0][2] - w * lf[0][3] - lf[2][0] - u * lf[2][3];
     const double ltyy = -lf[1][1] - v * lf[1][3];
     const double ltyz = -lf[1][2] - w * lf[1][3] - lf[2][1] - v * lf[2][3];
     const double ltzz = -lf[2][2] - w * lf[2][3];
-    lq[0] = -(txx * lf[0][3] + txy * lf[1][3] + txz * lf[2][3]);
-    lq[1] = -(txy * lf[0][3] + tyy * lf[1][3] + tyz * lf[2][3]);
-    lq[2] = -(txz * lf[0][3] + tyz * lf[1][3] + tzz * lf[2][3]);
-    double lg[12];
-    lg[0] = mu0 * (gas.s43 * ltxx - gas.s23 * ltyy - gas.s23 * ltzz);   // du/dx
-    lg[5] = mu0 * (-gas.s23 * ltxx + gas.s43 * ltyy - gas.s23 * ltzz);  // dv/dy
-    lg[10] = mu0 * (-gas.s23 * ltxx - gas.s23 * ltyy + gas.s43 * ltzz); // dw/dz
-    lg[4] = mu0 * ltxy; lg[1] = mu0 * ltxy;                              // du/dy, dv/dx
-    lg[8] = mu0 * ltxz; lg[2] = mu0 * ltxz;                              // du/dz, dw/dx
-    lg[9] = mu0 * ltyz; lg[6] = mu0 * ltyz;                              // dv/dz, dw/dy
-    lg[3] = -gas.lambda * lf[0][3]; lg[7] = -gas.lambda * lf[1][3]; lg[11] = -gas.lambda * lf[2][3];
-    // lifting adjoint: nu = sJ*lg
-#pragma unroll
-    for (int c = 0; c < 12; ++c) nu[c] = sj * lg[c];
-  }
-  __syncthreads();  // sP and sMu are no longer read: sK takes their place
-  if (act) {
-    // reference-derivative adjoint kappa^d = Ja^d . nu
+    lq[r][0] = -(txx * lf[0][3] + txy * lf[1][3] + txz * lf[2][3]);
+    lq[r][1] = -(txy * lf[0][3] + tyy * lf[1][3] + tyz * lf[2][3]);
+    lq[r][2] = -(txz * lf[0][3] + tyz * lf[1][3] + tzz * lf[2][3]);
+    lq[r][3] = 0.0;
+    // nu = sJ times the adjoint of the gradients, [x][u v w T]
+    const double ms = mu0 * sjr, ls = gas.lambda * sjr;
+    const double nu[12] = {ms * (gas.s43 * ltxx - gas.s23 * ltyy - gas.s23 * ltzz), ms * ltxy, ms * ltxz, -ls * lf[0][3],
+                           ms * ltxy, ms * (-gas.s23 * ltxx + gas.s43 * ltyy - gas.s23 * ltzz), ms * ltyz, -ls * lf[1][3],
+                           ms * ltxz, ms * ltyz, ms * (-gas.s23 * ltxx - gas.s23 * ltyy + gas.s43 * ltzz), -ls * lf[2][3]};
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
-      for (int v2 = 0; v2 < 4; ++v2)
-        sK[(4 * d + v2) * np + t] = Ja[3 * d] * nu[v2] + Ja[3 * d + 1] * nu[4 + v2] + Ja[3 * d + 2] * nu[8 + v2];
-    // face corrections 0.5*L_hat*(q_nb - q_own).(n SurfElem): own part here, the neighbour's
-    // part to its conservative variables (its state is the face state FUa of the neighbour slot)
-    // and into its exchange slot
-    const double lhm = sB[B.L_HatMinus()], lhp = sB[B.L_HatPlus() + N];
-#pragma unroll 1
-    for (int ls = 1; ls <= 6; ++ls) {
-      if (!(sides & (1 << (ls - 1)))) continue;
-      const int dir = dir_of(ls);
-      const double s = normal_sign(ls) * 0.5 * (minus_side(ls) ? lhm : lhp);
-      const int x = face_point<N>(ls, i, j, k);
-      double z[4];
+      for (int x = 0; x < 4; ++x)
+        g[r][4 * d + x] = Ja[3 * d] * nu[x] + Ja[3 * d + 1] * nu[4 + x] + Ja[3 * d + 2] * nu[8 + x];
 #pragma unroll
-      for (int v2 = 0; v2 < 4; ++v2) {
-        z[v2] = s * (Ja[3 * dir] * nu[v2] + Ja[3 * dir + 1] * nu[4 + v2] + Ja[3 * dir + 2] * nu[8 + v2]);
-        lq[v2] -= z[v2];
+    for (int x = 0; x < 12; ++x) now(g[r][x]);
+#pragma unroll
+    for (int x = 0; x < 3; ++x) now(lq[r][x]);
+  }
+  // along the lines: transposed derivatives, and the face corrections 0.5*L_hat*(q_nb - q_own).(n SurfElem)
+  // at the ends (own part here, the neighbour's part zn to its exchange slot); back to the nodes in place
+  double zn[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int r = 0; r < RN; ++r)
+      if (t + r * NT < np) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+          for (int w = 0; w < 2; ++w) sL[(X + 2 * d + w) * RS + place[r]] = g[r][4 * d + 2 * h + w];
       }
-      const Prim qn{sNb[4 * NF + x], sNb[x], sNb[NF + x], sNb[2 * NF + x], 0.0, sNb[3 * NF + x]};
+    __syncthreads();
+    if (line) {
+      const double* DT = basis + B.D_T() + fresh();
+      lp.again();
+      double* sX = sL + (X + 2 * q.d) * RS;
+      double x[2][n], y[2][n];
+#pragma unroll
+      for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (int l = 0; l < n; ++l) x[w][l] = lp.at(sX, l)[w * RS];
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        zn[0][2 * h + w] = -0.5 * lhm * x[w][0];
+        zn[1][2 * h + w] = 0.5 * lhp * x[w][N];
+      }
+#pragma unroll
+      for (int l = 0; l < n; ++l)
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            const double z = DT[i + n * l] * x[w][l];
+            y[w][i] = l == 0 ? z : y[w][i] + z;
+          }
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        y[w][0] -= zn[0][2 * h + w];
+        y[w][N] -= zn[1][2 * h + w];
+#pragma unroll
+        for (int i = 0; i < n; ++i) lp.at(sX, i)[w * RS] = y[w][i];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RN; ++r)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        const double* s = sL + (X + w) * RS + place[r];
+        lq[r][2 * h + w] += s[0] + s[2 * RS] + s[4 * RS];
+      }
+  }
+  if (line) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
       double lP[5];
-      prim_adjoint(qn, 0.0, gas, 0.0, z[0], z[1], z[2], 0.0, z[3], 0.0, lP);
-      // in place of the neighbour values of this face point (read above; no other lane has x)
+      prim_adjoint(qn[s], 0.0, gas, 0.0, zn[s][0], zn[s][1], zn[s][2], 0.0, zn[s][3], 0.0, lP);
 #pragma unroll
-      for (int v = 0; v < 5; ++v) sNb[v * NF + x] = lP[v];
+      for (int v = 0; v < 5; ++v) XU[5 * (size_t)q.own[s] + v] += lP[v];
     }
   }
-  __syncthreads();
-  // into the neighbour's exchange slots, one lane per own face point: the read-modify-writes of
-  // a node's sides then do not wait for each other's stores
-  for (int x = t; x < NF; x += NT) {
-    const unsigned own = sIdx[x];
 #pragma unroll
-    for (int v = 0; v < 5; ++v) XU[5 * (size_t)own + v] += sNb[v * NF + x];
+  for (int r = 0; r < RN; ++r) {
+    if (t + r * NT >= np) continue;
+    const size_t gid = e0 + t + r * NT;
+    const Prim p = cons_to_prim(c5[r], gas);
+    double lU[5];
+    prim_adjoint(p, c5[r][4], gas, 0.0, lq[r][0], lq[r][1], lq[r][2], 0.0, lq[r][3], 0.0, lU);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) out[5 * gid + v] += lU[v];
   }
-  if (!act) return;
-  // transposed line derivatives: dq/dxi_d at node i = sum_l D_T(l,i) q_l
-  const double* DT = sB + B.D_T();
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const int me = d == 0 ? i : (d == 1 ? j : k);
-    const int stride = d == 0 ? 1 : (d == 1 ? n : n * n);
-    const int base = t - me * stride;
-    for (int l = 0; l <= N; ++l) {
-      const double w = DT[me + n * l];
-#pragma unroll
-      for (int v2 = 0; v2 < 4; ++v2) lq[v2] += w * sK[(4 * d + v2) * np + base + l * stride];
-    }
-  }
-  double lU[5];
-  prim_adjoint(q, U[5 * gid + 4], gas, 0.0, lq[0], lq[1], lq[2], 0.0, lq[3], 0.0, lU);
-#pragma unroll
-  for (int v = 0; v < 5; ++v) out[5 * gid + v] += lU[v];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -732,7 +859,7 @@ __global__ __launch_bounds__(D<N>::NT) void k_adj_gather(DevMesh m, const double
   constexpr int n = D<N>::n, np = D<N>::np, NT = D<N>::NT, NF = D<N>::NF;
   __shared__ unsigned sIdx[NF];
   const int e = blockIdx.x, t = threadIdx.x;
-  for (int x = t; x < NF; x += NT) sIdx[x] = face_slot<N>(m, e, x);
+  for (int x = t; x < NF; x += NT) sIdx[x] = face_slot_tab<N>(m, e, x);
   __syncthreads();
   if (t >= np) return;
   const int i = t % n, j = (t / n) % n, k = t / (n * n);
@@ -752,15 +879,15 @@ __global__ __launch_bounds__(D<N>::NT) void k_adj_gather(DevMesh m, const double
 }
 
 // The register update of a reverse LSERK stage (the last one of a chain; the others are applied
-// by the next stage's k_adj_euler): ub += out + the neighbours' face parts, rbar = a*(rbar + cub*ub).
+// by the next stage's k_adj_euler): ub += out + the neighbours' face parts, rbar = a*lam, in place of lam.
 template <int N>
 __global__ __launch_bounds__(D<N>::NT) void k_adj_stage_update(DevMesh m, const double* __restrict__ XU,
                                                              const double* __restrict__ out, double* __restrict__ ub,
-                                                             double* __restrict__ rbar, double cub, double a) {
+                                                             double* __restrict__ rbar, double a) {
   constexpr int n = D<N>::n, np = D<N>::np, NT = D<N>::NT, NF = D<N>::NF;
   __shared__ unsigned sIdx[NF];
   const int e = blockIdx.x, t = threadIdx.x;
-  for (int x = t; x < NF; x += NT) sIdx[x] = face_slot<N>(m, e, x);
+  for (int x = t; x < NF; x += NT) sIdx[x] = face_slot_tab<N>(m, e, x);
   __syncthreads();
   if (t >= np) return;
   const int i = t % n, j = (t / n) % n, k = t / (n * n);
@@ -779,7 +906,7 @@ __global__ __launch_bounds__(D<N>::NT) void k_adj_stage_update(DevMesh m, const 
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
     const double u0 = ub[5 * gid + v];
-    rbar[5 * gid + v] = a * (rbar[5 * gid + v] + cub * u0);
+    rbar[5 * gid + v] = a * rbar[5 * gid + v];
     ub[5 * gid + v] = u0 + g5[v];
   }
 }
@@ -790,25 +917,31 @@ __global__ __launch_bounds__(256) void k_axpy(size_t n, double a, const double* 
   if (i < n) y[i] += a * x[i];
 }
 
-// The transposed-Jacobian parts of one right-hand side at U (face states FU): out = the element's
+// The transposed-Jacobian parts of one right-hand side at U (FU: its face states, or null: the neighbours'
+// states are read from U through m.nbNode): out = the element's
 // own parts, XU = the parts of the neighbours' face nodes. lam (+ cub*ub when ub is given) is the
 // adjoint of Ut; with pd.XU a previous stage's register update is applied first (k_adj_euler).
+template <int N, bool AFF>
+hipError_t adj_parts_n(const DevMesh& m, const AdjointWork& w, const Gas& gas, int riemann, const double* U,
+                       const double* FU, double* lam, double* ub, double cub, double* out, double* XU, Pending pd,
+                       hipStream_t s) {
+  const dim3 g(m.nElems), b(S<N>::NT);
+#define FXG_LAUNCH(SOLV)                                                                                        \
+  hipLaunchKernelGGL((k_adj_euler<N, SOLV, AFF>), g, b, 0, s, U, m, m.basis, FU, lam, ub, cub, gas, out, XU, w.Xg, pd)
+  if (riemann == 1) FXG_LAUNCH(1);
+  else if (riemann == 3) FXG_LAUNCH(3);
+  else FXG_LAUNCH(33);
+#undef FXG_LAUNCH
+  hipLaunchKernelGGL((k_adj_visc<N, AFF>), g, b, 0, s, U, m, m.basis, FU, (const double*)lam, (const double*)w.Xg, gas,
+                     out, XU);
+  return hipGetLastError();
+}
 template <int N>
 hipError_t adj_parts(const DevMesh& m, const AdjointWork& w, const Gas& gas, int riemann, const double* U,
                      const double* FU, double* lam, double* ub, double cub, double* out, double* XU, Pending pd,
                      hipStream_t s) {
-  const int K = m.nElems;
-  constexpr int NT = D<N>::NT;
-  if (riemann == 1)
-    hipLaunchKernelGGL((k_adj_euler<N, 1>), dim3(K), dim3(NT), 0, s, U, m, FU, lam, ub, cub, gas, out, XU, w.Xg, pd);
-  else if (riemann == 3)
-    hipLaunchKernelGGL((k_adj_euler<N, 3>), dim3(K), dim3(NT), 0, s, U, m, FU, lam, ub, cub, gas, out, XU, w.Xg, pd);
-  else
-    hipLaunchKernelGGL((k_adj_euler<N, 33>), dim3(K), dim3(NT), 0, s, U, m, FU, lam, ub, cub, gas, out, XU, w.Xg,
-                       pd);
-  hipLaunchKernelGGL((k_adj_visc<N>), dim3(K), dim3(NT), 0, s, U, m, FU, (const double*)lam, (const double*)ub, cub,
-                     (const double*)w.Xg, gas, out, XU);
-  return hipGetLastError();
+  return m.aff ? adj_parts_n<N, true>(m, w, gas, riemann, U, FU, lam, ub, cub, out, XU, pd, s)
+               : adj_parts_n<N, false>(m, w, gas, riemann, U, FU, lam, ub, cub, out, XU, pd, s);
 }
 
 template <int N>
@@ -818,9 +951,9 @@ hipError_t adj_gather(const DevMesh& m, const double* XU, double* out, hipStream
 }
 
 template <int N>
-hipError_t adj_update(const DevMesh& m, const double* XU, const double* out, double* ub, double* rbar, double cub,
-                      double a, hipStream_t s) {
-  hipLaunchKernelGGL((k_adj_stage_update<N>), dim3(m.nElems), dim3(D<N>::NT), 0, s, m, XU, out, ub, rbar, cub, a);
+hipError_t adj_update(const DevMesh& m, const double* XU, const double* out, double* ub, double* rbar, double a,
+                      hipStream_t s) {
+  hipLaunchKernelGGL((k_adj_stage_update<N>), dim3(m.nElems), dim3(D<N>::NT), 0, s, m, XU, out, ub, rbar, a);
   return hipGetLastError();
 }
 
@@ -839,11 +972,10 @@ hipError_t adj_update(const DevMesh& m, const double* XU, const double* out, dou
 
 hipError_t launch_rhs_vjp(const DevMesh& m, const AdjointWork& w, const Gas& gas, int riemann, const double* U,
                           const double* lam, double* out, hipStream_t s) {
-  hipError_t err = launch_faces_of(m, U, w.FUa, s);
-  if (err != hipSuccess) return err;
+  if (!m.nbNode) return hipErrorInvalidValue;
   double* lw = const_cast<double*>(lam);  // read only without a pending update
-#define FXG_PARTS(NN) adj_parts<NN>(m, w, gas, riemann, U, w.FUa, lw, nullptr, 0.0, out, w.XU[0], Pending{}, s)
-  err = [&]() -> hipError_t { FXG_ADJ_SWITCH(FXG_PARTS) }();
+#define FXG_PARTS(NN) adj_parts<NN>(m, w, gas, riemann, U, nullptr, lw, nullptr, 0.0, out, w.XU[0], Pending{}, s)
+  const hipError_t err = [&]() -> hipError_t { FXG_ADJ_SWITCH(FXG_PARTS) }();
 #undef FXG_PARTS
   if (err != hipSuccess) return err;
 #define FXG_GATHER(NN) adj_gather<NN>(m, w.XU[0], out, s)
@@ -854,19 +986,14 @@ hipError_t launch_rhs_vjp(const DevMesh& m, const AdjointWork& w, const Gas& gas
 hipError_t launch_adjoint_stage(const DevMesh& m, const AdjointWork& w, const Gas& gas, int riemann, const double* U,
                                 const double* FU, double* rbar, double* ubar, double cub, double a, double* out,
                                 AdjointChain& ch, hipStream_t s) {
-  if (!FU) {
-    const hipError_t err = launch_faces_of(m, U, w.FUa, s);
-    if (err != hipSuccess) return err;
-    FU = w.FUa;
-  }
-  const Pending pd{ch.pending ? w.XU[ch.cur] : nullptr, ch.cub, ch.a};
+  if (!FU && !m.nbNode) return hipErrorInvalidValue;
+  const Pending pd{ch.pending ? w.XU[ch.cur] : nullptr, ch.a};
   const int nxt = ch.pending ? 1 - ch.cur : ch.cur;
 #define FXG_PARTS(NN) adj_parts<NN>(m, w, gas, riemann, U, FU, rbar, ubar, cub, out, w.XU[nxt], pd, s)
   const hipError_t err = [&]() -> hipError_t { FXG_ADJ_SWITCH(FXG_PARTS) }();
 #undef FXG_PARTS
   ch.cur = nxt;
   ch.pending = true;
-  ch.cub = cub;
   ch.a = a;
   return err;
 }
@@ -875,7 +1002,7 @@ hipError_t launch_adjoint_flush(const DevMesh& m, const AdjointWork& w, double* 
                                 const double* out, AdjointChain& ch, hipStream_t s) {
   if (!ch.pending) return hipSuccess;
   ch.pending = false;
-#define FXG_UPDATE(NN) adj_update<NN>(m, w.XU[ch.cur], out, ubar, rbar, ch.cub, ch.a, s)
+#define FXG_UPDATE(NN) adj_update<NN>(m, w.XU[ch.cur], out, ubar, rbar, ch.a, s)
   FXG_ADJ_SWITCH(FXG_UPDATE)
 #undef FXG_UPDATE
 }

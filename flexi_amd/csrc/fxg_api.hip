@@ -481,10 +481,11 @@ int ensure_adjoint(fxg_ctx* c) {
   if (!c->fused || c->p.precision != FXG_PREC_FP64 || c->nBC > 0)
     return fail("the discrete adjoint is built for the FP64 Gauss-Lobatto split form (N 2..7) on meshes without "
                 "boundary sides");
-  if (c->aw.FUa) return 0;
+  if (!c->m.nbNode) return fail("the discrete adjoint needs fewer than 2^32 nodes");
+  if (c->adjTmp) return 0;
   const size_t face = (size_t)c->nf * c->S, vol = (size_t)c->np * c->K;
-  if (alloc_owned(c, &c->aw.FUa, 10 * face) || alloc_owned(c, &c->aw.XU[0], 10 * face) ||
-      alloc_owned(c, &c->aw.XU[1], 10 * face) || alloc_owned(c, &c->aw.Xg, 8 * face) ||
+  if (alloc_owned(c, &c->aw.XU[0], 10 * face) || alloc_owned(c, &c->aw.XU[1], 10 * face) ||
+      alloc_owned(c, &c->aw.Xg, 8 * face) ||
       alloc_owned(c, &c->adjTmp, 5 * vol))
     return 1;
   return 0;

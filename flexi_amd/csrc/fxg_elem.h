@@ -52,25 +52,15 @@ __device__ __forceinline__ int face_point(int ls, int i, int j, int k) {
   }
 }
 
-// Side-array slot of own face point x of element e: ((side*2 + slot)*nf + pq), slot 0 master.
-// In two steps for callers that issue other loads between them: the ElemToSide entry (side, flip)
-// of the point's local side, then the slot through the inverse S2V2 map.
-template <int N>
-__device__ __forceinline__ int2 face_side_entry(const DevMesh& m, int e, int x) {
-  constexpr int nf = (N + 1) * (N + 1);
-  const int ls = x / nf + 1;
-  return make_int2(m.E2S[2 * (ls - 1) + 12 * e] - 1, m.E2S[2 * (ls - 1) + 1 + 12 * e]);
-}
-template <int N>
-__device__ __forceinline__ unsigned face_slot_from(const DevMesh& m, int2 sf, int x) {
-  constexpr int n = N + 1, nf = n * n;
-  const int ls = x / nf + 1, ab = x - (ls - 1) * nf;
-  const int* pq = m.v2s2 + 2 * (ab + nf * (sf.y + 5 * (ls - 1)));
-  return (unsigned)(((size_t)sf.x * 2 + (sf.y ? 1 : 0)) * nf + pq[0] + n * pq[1]);
-}
+// Side-array slot of own face point x of element e: ((side*2 + slot)*nf + pq), slot 0 master; from the
+// ElemToSide entry (side, flip) of the point's local side and the inverse S2V2 map.
 template <int N>
 __device__ __forceinline__ unsigned face_slot(const DevMesh& m, int e, int x) {
-  return face_slot_from<N>(m, face_side_entry<N>(m, e, x), x);
+  constexpr int n = N + 1, nf = n * n;
+  const int ls = x / nf + 1, ab = x - (ls - 1) * nf;
+  const int side = m.E2S[2 * (ls - 1) + 12 * e] - 1, flip = m.E2S[2 * (ls - 1) + 1 + 12 * e];
+  const int* pq = m.v2s2 + 2 * (ab + nf * (flip + 5 * (ls - 1)));
+  return (unsigned)(((size_t)side * 2 + (flip ? 1 : 0)) * nf + pq[0] + n * pq[1]);
 }
 // The same from the table of the fused path (m.slotTab, filled by launch_slot_table): one load
 // instead of ElemToSide followed by the inverse S2V2 map.
@@ -164,21 +154,18 @@ __device__ __forceinline__ void load_metrics(const double* Je, int t, RF* Ja, RF
   sj = (RF)Je[9 * np + t];
 }
 
-// Geometry of own face point (local side ls, boundary node id), the same arithmetic as the surface
+// Geometry of own face point (local side ls, Jd: the metric terms Ja^dir of its node), the same arithmetic as the surface
 // phase of the fused stage kernel: the master normal nv, SurfElem (returned) and a tangential
 // basis (Gram-Schmidt of the coordinate axis least aligned with n, t2 = n x t1). With
 // ownFaceMetric the own boundary metric NormalSign*Ja^{NormalDir} gives n*SurfElem (times -1 on a
 // slave side for the master normal); otherwise the side's NormVec/SurfElem are used for both
 // sides, as FLEXI does.
 template <int N, class RF>
-__device__ __forceinline__ double face_frame(const DevMesh& m, int e, int ls, int id, unsigned own, bool master, RF* nv,
+__device__ __forceinline__ double face_frame(const DevMesh& m, const double* Jd, int ls, unsigned own, bool master, RF* nv,
                                              RF* t1, RF* t2) {
-  constexpr int np = D<N>::np;
   double se;
   if (m.ownFaceMetric) {
-    const int dir = dir_of(ls);
     const double sgn = normal_sign(ls), ms = master ? 1.0 : -1.0;
-    const double* Jd = (dir == 0 ? m.Mf : (dir == 1 ? m.Mg : m.Mh)) + 3 * ((size_t)np * e + id);
     const double ns0 = sgn * Jd[0], ns1 = sgn * Jd[1], ns2 = sgn * Jd[2];
     se = sqrt(ns0 * ns0 + ns1 * ns1 + ns2 * ns2);
     const double mse = ms / se;
