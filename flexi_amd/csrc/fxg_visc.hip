@@ -4,30 +4,26 @@
 // energy) into the side array FG (lifting_br1.t90:48-181, flux.f90:149-241). A translation unit
 // of its own, so that its code does not change the register allocation of k_dg_fused.
 #include "fxg_bc.h"
-#include "fxg_elem.h"
+#include "fxg_line.h"
 
 namespace fxg {
 namespace {
 
-// FP64 stages the element's U in LDS with contiguous lanes (held to 80 VGPRs at N=7, 52 KB:
-// three workgroups per CU); FP32-bulk converts U from global memory directly and is held to 64
-// VGPRs (18 KB: four workgroups per CU, 0.42 ms instead of 0.53 ms at 32^3, N=7). On meshes with
-// boundary sides (BC) it also keeps the gradients of the boundary face points for k_bc_visc.
-// AFF: every element's metric terms are the same at all of its nodes (m.aff); they then come as ten uniform
-// values of the element instead of rows of Jsoa (46 bytes per node of 143 at N=7; 32^3: 0.47 -> 0.42 ms in
-// FP64, 0.42 -> 0.31 in FP32-bulk).
+// FP32-bulk, one lane per boundary node. U is converted from global memory directly and the kernel is
+// held to 64 VGPRs (18 KB: four workgroups per CU). On meshes with boundary sides (BC) it also keeps the
+// gradients of the boundary face points for k_bc_visc. AFF: every element's metric terms are the same at all
+// of its nodes (m.aff); they then come as ten uniform values of the element instead of rows of Jsoa (46 bytes
+// per node of 143 at N=7; 32^3: 0.42 -> 0.31 ms).
 // FIRST: no stage has left the face states of U (a right-hand side alone, the first stage of a step on
 // a caller's state): the neighbours' states come from their nodes in U and the own face states are
 // written to FU for the stage kernel. Replaces a pass of its own over U (k_faces_of, 64 bytes per node at
-// N=7 and one launch; right-hand side at 32^3, N=7: 1.38 -> 1.30 ms).
+// N=7 and one launch; right-hand side at 32^3, N=7, FP64: 1.38 -> 1.30 ms).
 template <int N, class RF, bool BC, bool AFF, bool FIRST>
 __global__ __launch_bounds__(D<N>::NT)
-__attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 ? 8 : 6) : (N == 7 ? 6 : 1)))) void k_visc_faces(
+__attribute__((amdgpu_waves_per_eu(N == 7 ? 8 : 6))) void k_visc_faces(
     const double* __restrict__ U, DevMesh m, const double* __restrict__ Jsoa, double* __restrict__ FU,
     RF* __restrict__ FG, Gas gas, RF* __restrict__ gBC) {
   constexpr int n = D<N>::n, np = D<N>::np, NT = D<N>::NT, NF = D<N>::NF;
-  constexpr bool raw = sizeof(RF) == 8;
-  __shared__ double sRaw[raw ? 5 * np : 1];  // the element's U as stored, loaded with contiguous lanes
   __shared__ RF sP[4 * np];        // u, v, w, T
   __shared__ RF sNb[4 * NF];       // neighbour u, v, w, T per own face point
   __shared__ unsigned sIdx[NF];
@@ -38,10 +34,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 ? 8 : 6) : (N == 7 
   constexpr int NBAS = 3 * n * n + 4 * n;
   static_assert(NBAS <= NT, "one basis entry per lane");
   constexpr int RS = (NF + NT - 1) / NT;  // own face points per lane
-  constexpr int RU = raw ? (5 * np + NT - 1) / NT : 5;
   // Every global load of the staging is issued before the first wait, instead of one wait per
-  // loop of loads: the side slots first (the neighbour states depend on them), then U (FP64: the
-  // element's values with contiguous lanes; FP32-bulk: the lane's node) and the basis.
+  // loop of loads: the side slots first (the neighbour states depend on them), then U and the basis.
   unsigned own[RS], nbr[RS];
 #pragma unroll
   for (int r = 0; r < RS; ++r) {
@@ -49,16 +43,9 @@ __attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 ? 8 : 6) : (N == 7 
     own[r] = x < NF ? face_slot_tab<N>(m, e, x) : 0u;
     nbr[r] = FIRST && x < NF ? m.nbNode[(size_t)NF * e + x] : 0u;
   }
-  double ul[RU];
+  double ul[5];
 #pragma unroll
-  for (int r = 0; r < RU; ++r) {
-    if constexpr (raw) {
-      const int x = t + r * NT;
-      ul[r] = x < 5 * np ? Ue[x] : 0.0;
-    } else {
-      ul[r] = t < np ? Ue[5 * t + r] : 1.0;
-    }
-  }
+  for (int r = 0; r < 5; ++r) ul[r] = t < np ? Ue[5 * t + r] : 1.0;
   const double bas = t < NBAS ? m.basis[t] : 0.0;
   double cn[RS][5];
 #pragma unroll
@@ -67,11 +54,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 ? 8 : 6) : (N == 7 
 #pragma unroll
     for (int v = 0; v < 5; ++v) cn[r][v] = t + r * NT < NF ? c[v] : 1.0;
   }
-  if constexpr (raw) {
-#pragma unroll
-    for (int r = 0; r < RU; ++r)
-      if (t + r * NT < 5 * np) sRaw[t + r * NT] = ul[r];
-  } else if (t < np) {
+  if (t < np) {
     const Prim q = cons_to_prim(ul, gas);
     sP[t] = q.u; sP[np + t] = q.v; sP[2 * np + t] = q.w; sP[3 * np + t] = q.T;
   }
@@ -93,18 +76,11 @@ __attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 ? 8 : 6) : (N == 7 
       if (x < NF) {
         const int ls = x / (n * n) + 1, ab = x - (ls - 1) * n * n;
         const int id = vidx<N>(ls, ab % n, ab / n);
-        const double* c = raw ? sRaw + 5 * id : Ue + 5 * id;
+        const double* c = Ue + 5 * id;
 #pragma unroll
         for (int v = 0; v < 5; ++v) FU[5 * (size_t)own[r] + v] = c[v];
       }
     }
-  }
-  if (raw) {
-    if (t < np) {
-      const Prim q = cons_to_prim(sRaw + 5 * t, gas);
-      sP[t] = q.u; sP[np + t] = q.v; sP[2 * np + t] = q.w; sP[3 * np + t] = q.T;
-    }
-    __syncthreads();
   }
   // one lane per boundary node, in boundary-rank order (the Jsoa rows): lanes 0..NB-1, so the
   // waves beyond NB/64 end here instead of idling through the lifting
@@ -147,6 +123,195 @@ __attribute__((amdgpu_waves_per_eu(sizeof(RF) == 4 ? (N == 7 ? 8 : 6) : (N == 7 
         for (int c = 0; c < 12; ++c) gb[c] = g[c];
       }
     }
+  }
+}
+
+// FP64: the same with one lane per line of nodes (fxg_line.h), as in the stage kernel. The form above, one lane
+// per boundary node, reads 120 values per boundary node from LDS and leaves two of five lanes idle; here a
+// line is read once per variable, the gradients come together in the node phase, and the ends of the lines are
+// the face points. 10 LDS rows: four workgroups of four waves per CU at N=7. Parallelepipeds: 32^3, N=7
+// 0.42 -> 0.33 ms (94 bytes per node at 4.8 TB/s, the copy rate), N=5, 24^3 0.108 -> 0.079, N=3, 32^3 0.089 ->
+// 0.068; general: N=7, 32^3 0.48 -> 0.44, N=5, 24^3 0.129 -> 0.105.
+// LDS rows: 0 u, 1 v, 2 w, 3 T; 4..9 exchange between line and node phases (two variables in three directions).
+template <int N, bool BC, bool AFF, bool FIRST>
+__global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(3))) void k_visc_lines(
+    const double* __restrict__ U, DevMesh m, const double* __restrict__ basis, const double* __restrict__ Jsoa,
+    double* __restrict__ FU, double* __restrict__ FG, Gas gas, double* __restrict__ gBC) {
+  constexpr int n = S<N>::n, nf = S<N>::nf, np = S<N>::np, NL = S<N>::NL, NT = S<N>::NT, RN = S<N>::RN, RS = S<N>::RS;
+  constexpr int X = 4, NF = 6 * nf;
+  __shared__ double sL[10 * RS];
+  const BasisLayout B{n};
+  const int e = blockIdx.x, t = N == 7 ? (threadIdx.x + 64 * (e & 3)) % NT : threadIdx.x;
+  const bool line = t < NL;
+  const int tl = line ? t : 0;
+  const int d = tl / nf, ln = tl - d * nf, la = ln % n, lb = ln / n;
+  const size_t fp0 = (size_t)NF * e + ((d == 0 ? 5 : (d == 1 ? 2 : 1)) - 1) * nf + ln;
+  const size_t fp1 = (size_t)NF * e + ((d == 0 ? 3 : (d == 1 ? 4 : 6)) - 1) * nf + ln;
+  const unsigned own0 = m.slotTab[fp0], own1 = m.slotTab[fp1];
+  const size_t e0 = (size_t)np * e;
+  const double* je = AFF ? m.aff + 10 * (size_t)e : nullptr;
+  double c[RN][5];
+#pragma unroll
+  for (int r = 0; r < RN; ++r)
+#pragma unroll
+    for (int v = 0; v < 5; ++v) c[r][v] = t + r * NT < np ? U[5 * (e0 + t + r * NT) + v] : 1.0;
+  double nb[2][5];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const double* b = FIRST ? U + 5 * (size_t)m.nbNode[s ? fp1 : fp0] : FU + 5 * (size_t)slot_nbr<N>(s ? own1 : own0);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) nb[s][v] = b[v];
+  }
+  int place[RN];
+#pragma unroll
+  for (int r = 0; r < RN; ++r) {
+    const int nd = t + r * NT < np ? t + r * NT : 0;
+    place[r] = pos<N>(nd % n, (nd / n) % n, nd / nf);
+    if (t + r * NT < np) {
+      const Prim q = cons_to_prim(c[r], gas);
+      double* s = sL + place[r];
+      s[0] = q.u; s[RS] = q.v; s[2 * RS] = q.w; s[3 * RS] = q.T;
+      if constexpr (FIRST) {  // the state itself, to the ends of the lines
+#pragma unroll
+        for (int v = 0; v < 5; ++v) s[(X + v) * RS] = c[r][v];
+      }
+    }
+  }
+  const Prim q0 = cons_to_prim(nb[0], gas), q1 = cons_to_prim(nb[1], gas);
+  Line<N> lp(d, la, lb);
+  __syncthreads();
+  double jq[2][4];  // BR1 jumps with their sign and weight
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const double* o = lp.at(sL, s ? N : 0);
+    const Prim& q = s ? q1 : q0;
+    const double h = s ? 0.5 * basis[B.L_HatPlus() + N] : -0.5 * basis[B.L_HatMinus()];
+    jq[s][0] = h * (q.u - o[0]); jq[s][1] = h * (q.v - o[RS]); jq[s][2] = h * (q.w - o[2 * RS]);
+    jq[s][3] = h * (q.T - o[3 * RS]);
+  }
+  if constexpr (FIRST) {  // the own face states, for the stage kernel
+    if (line) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const double* o = lp.at(sL, s ? N : 0) + X * RS;
+        double* dst = FU + 5 * (size_t)(s ? own1 : own0);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) dst[v] = o[v * RS];
+      }
+    }
+    __syncthreads();
+  }
+  double g[RN][12];  // reference derivatives, then contravariant viscous fluxes: [d][u v w T]
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (line) {
+      const double* DT = basis + B.D_T() + fresh();
+      lp.again();
+      double* sX = sL + (X + 2 * d) * RS;
+      double q[2][n];
+#pragma unroll
+      for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (int l = 0; l < n; ++l) q[w][l] = lp.at(sL, l)[(2 * h + w) * RS];
+#pragma unroll
+      for (int i = 0; i < n; ++i)
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          double a = DT[n * i] * q[w][0];
+#pragma unroll
+          for (int l = 1; l < n; ++l) a += DT[l + n * i] * q[w][l];
+          if (i == 0) a += jq[0][2 * h + w];
+          if (i == N) a += jq[1][2 * h + w];
+          lp.at(sX, i)[w * RS] = a;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RN; ++r)
+#pragma unroll
+      for (int x = 0; x < 3; ++x)
+#pragma unroll
+        for (int w = 0; w < 2; ++w) g[r][4 * x + 2 * h + w] = sL[(X + 2 * x + w) * RS + place[r]];
+    if (h == 0) __syncthreads();
+  }
+  const GasT<double> gt(gas);
+#pragma unroll
+  for (int r = 0; r < RN; ++r) {
+    const int nd = t + r * NT < np ? t + r * NT : 0;
+    double Ja[9], sj;
+    if constexpr (AFF) {
+      const double* jn = je + fresh();
+#pragma unroll
+      for (int x = 0; x < 9; ++x) Ja[x] = jn[x];
+      sj = jn[9];
+    } else {
+      // those of the boundary nodes, packed; the interior nodes' fluxes are not needed
+      constexpr int NB = Bnd<N>::NB;
+      const int i = nd % n, j = (nd / n) % n, k = nd / nf;
+      const bool bn = node_sides<N>(i, j, k) != 0;
+      const double* Je = Jsoa + (size_t)10 * NB * e + (bn ? bnd_rank<N>(i, j, k) : 0);
+#pragma unroll
+      for (int x = 0; x < 9; ++x) Ja[x] = bn ? Je[x * NB] : 0.0;
+      sj = bn ? Je[9 * NB] : 0.0;
+    }
+    double p[12];
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        p[4 * x + v] = (Ja[x] * g[r][v] + Ja[3 + x] * g[r][4 + v] + Ja[6 + x] * g[r][8 + v]) * sj;
+    if constexpr (BC) {
+      // boundary sides: keep the gradients at their face points for k_bc_visc
+      if (t + r * NT < np) {
+        const int i = nd % n, j = (nd / n) % n, k = nd / nf, sides = node_sides<N>(i, j, k);
+#pragma unroll 1
+        for (int ls = 1; ls <= 6; ++ls) {
+          if (!(sides & (1 << (ls - 1)))) continue;
+          const unsigned own = m.slotTab[(size_t)NF * e + face_point<N>(ls, i, j, k)];
+          if ((int)(own / (2u * (unsigned)nf)) >= m.nBC) continue;
+          double* gb = gBC + 12 * slot_side_point<N>(own);
+#pragma unroll
+          for (int x = 0; x < 12; ++x) gb[x] = p[x];
+        }
+      }
+    }
+    double fx[4], fy[4], fz[4];
+    const double* s = sL + place[r];
+    diff_flux<double>(gt, s[0], s[RS], s[2 * RS], p, p + 4, p + 8, fx, fy, fz);
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        g[r][4 * x + v] = Ja[3 * x] * fx[v] + Ja[3 * x + 1] * fy[v] + Ja[3 * x + 2] * fz[v];
+#pragma unroll
+    for (int x = 0; x < 12; ++x) now(g[r][x]);
+  }
+  // to the ends of the lines: n SurfElem there is NormalSign Ja^d
+  double f[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int r = 0; r < RN; ++r)
+      if (t + r * NT < np) {
+#pragma unroll
+        for (int x = 0; x < 3; ++x)
+#pragma unroll
+          for (int w = 0; w < 2; ++w) sL[(X + 2 * x + w) * RS + place[r]] = g[r][4 * x + 2 * h + w];
+      }
+    __syncthreads();
+    const double* sX = sL + (X + 2 * d) * RS;
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      f[0][2 * h + w] = -lp.at(const_cast<double*>(sX), 0)[w * RS];
+      f[1][2 * h + w] = lp.at(const_cast<double*>(sX), N)[w * RS];
+    }
+    if (h == 0) __syncthreads();
+  }
+  if (!line) return;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    FG[4 * (size_t)own0 + v] = f[0][v];
+    FG[4 * (size_t)own1 + v] = f[1][v];
   }
 }
 
@@ -259,22 +424,23 @@ hipError_t launch_visc_faces(const DevMesh& m, bool fp32, bool faces_fresh, cons
   const bool bc = m.nBC > 0;
   if (!faces_fresh && !m.nbNode) return hipErrorInvalidValue;
   switch (m.N) {
-#define FXG_LAUNCH2(NN, RF, BC, AFF, FIRST)                                                                       \
-  hipLaunchKernelGGL((k_visc_faces<NN, RF, BC, AFF, FIRST>), dim3(m.nElems), dim3(D<NN>::NT), 0, s, U, m, Jsoa, FU, \
-                     (RF*)FG, gas, (RF*)gBC)
-#define FXG_LAUNCH(NN, RF)                                                                                       \
-  do {                                                                                                           \
-    if (bc) { if (m.aff) FXG_LAUNCH2(NN, RF, true, true, false); else FXG_LAUNCH2(NN, RF, true, false, false); }  \
-    else if (faces_fresh) { if (m.aff) FXG_LAUNCH2(NN, RF, false, true, false); else FXG_LAUNCH2(NN, RF, false, false, false); } \
-    else { if (m.aff) FXG_LAUNCH2(NN, RF, false, true, true); else FXG_LAUNCH2(NN, RF, false, false, true); }    \
+#define FXG_LAUNCH2(NN, BC, AFF, FIRST)                                                                            \
+  do {                                                                                                             \
+    if (fp32)                                                                                                      \
+      hipLaunchKernelGGL((k_visc_faces<NN, float, BC, AFF, FIRST>), dim3(m.nElems), dim3(D<NN>::NT), 0, s, U, m,    \
+                         Jsoa, FU, (float*)FG, gas, (float*)gBC);                                                  \
+    else                                                                                                           \
+      hipLaunchKernelGGL((k_visc_lines<NN, BC, AFF, FIRST>), dim3(m.nElems), dim3(S<NN>::NT), 0, s, U, m, m.basis, \
+                         Jsoa, FU, (double*)FG, gas, (double*)gBC);                                                      \
   } while (0)
-#define FXG_CASE(NN)                                              \
-  case NN:                                                        \
-    if (fp32) FXG_LAUNCH(NN, float); else FXG_LAUNCH(NN, double); \
+#define FXG_CASE(NN)                                                                                               \
+  case NN:                                                                                                         \
+    if (bc) { if (m.aff) FXG_LAUNCH2(NN, true, true, false); else FXG_LAUNCH2(NN, true, false, false); }            \
+    else if (faces_fresh) { if (m.aff) FXG_LAUNCH2(NN, false, true, false); else FXG_LAUNCH2(NN, false, false, false); } \
+    else { if (m.aff) FXG_LAUNCH2(NN, false, true, true); else FXG_LAUNCH2(NN, false, false, true); }              \
     break;
     FXG_CASE(2) FXG_CASE(3) FXG_CASE(4) FXG_CASE(5) FXG_CASE(6) FXG_CASE(7)
 #undef FXG_CASE
-#undef FXG_LAUNCH
 #undef FXG_LAUNCH2
     default: return hipErrorInvalidValue;
   }
