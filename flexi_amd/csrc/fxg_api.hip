@@ -392,12 +392,14 @@ int finish_setup(fxg_ctx* c) {
       HIPCHECK(fxg::launch_neighbour_nodes(c->m, static_cast<unsigned*>(c->fw.FG), nb, c->stream));
       c->m.nbNode = nb;
     }
-    double* aff = nullptr;
-    bool all = false;
-    if (alloc_owned(c, &aff, (size_t)10 * c->K)) return 1;
-    HIPCHECK(fxg::find_const_metrics(c->m, aff, c->w.errOut, all, c->stream));
-    c->m.aff = all ? aff : nullptr;
-    if (c->fused && !all) {  // the boundary nodes' metric terms, packed for the viscous face kernel
+    if (c->p.precision == FXG_PREC_FP64) {
+      double* aff = nullptr;
+      bool all = false;
+      if (alloc_owned(c, &aff, (size_t)10 * c->K)) return 1;
+      HIPCHECK(fxg::find_const_metrics(c->m, aff, c->w.errOut, all, c->stream));
+      c->m.aff = all ? aff : nullptr;
+    }
+    if (c->fused && !c->m.aff) {  // the boundary nodes' metric terms, packed for the viscous face kernel
       if (alloc_owned(c, &c->fw.Jsoa, fxg::packed_metrics_size(c->N, c->K))) return 1;
       HIPCHECK(fxg::launch_pack_metrics(c->m, c->fw.Jsoa, c->stream));
     }
@@ -584,8 +586,11 @@ int fxg_create_from_nodes(const fxg_params* p, int nElems, int nSides, const int
     const size_t face = (size_t)c->nf * nSides;
     if (alloc_owned(c, &slaveNS, 3 * face) || alloc_owned(c, &c->w.FluxS, 5 * face)) { ctx_free(c); return 1; }
   }
+  // (FP32-bulk keeps each node's own rounding of the terms: any other would change which of its sums round
+  // up, and with that its results by an ulp of FP32 at some nodes)
+  const bool flat = p->precision == FXG_PREC_FP64;
   if (fxg::compute_metrics_gpu(c->N, p->nodeType, NGeo, nElems, dNC, c->m, c->Mf, c->Mg, c->Mh, c->sJ, c->xGP, c->NV,
-                               c->T1, c->T2, c->SE, slaveNS, !own, c->stream, err)) {
+                               c->T1, c->T2, c->SE, slaveNS, !own, flat, c->stream, err)) {
     fail(err); ctx_free(c); return 1;
   }
   c->m.slaveNS = slaveNS;

@@ -53,8 +53,8 @@ struct LdsB {
 // code. The LDS arrays are FP32 (38 KB at N=7) and the kernel is held to 64 VGPRs, so four workgroups
 // share a CU (six waves per SIMD below N=7, where 8 would spill, and in the last stage of a step).
 // LAM: the last stage of a step, which also forms CALCTIMESTEP's per-element spectral radii of the
-// new state. AFF: the metric terms are the same at all nodes of an element (m.aff).
-template <int N, class RF, int SOLVER, bool BC, bool LAM, bool AFF>
+// new state.
+template <int N, class RF, int SOLVER, bool BC, bool LAM>
 __global__ __launch_bounds__(D<N>::NT)
 __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(const double* U, DevMesh m, const double* __restrict__ FU,
                                                      double* __restrict__ FUnext, const RF* __restrict__ FG,
@@ -118,8 +118,7 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
       // own outward normal times SurfElem from the own metric terms at the boundary node
       const int dir = dir_of(ls);
       const double sgn = normal_sign(ls);
-      const double* Jd = AFF ? m.aff + 10 * (size_t)e + 3 * dir
-                             : (dir == 0 ? m.Mf : (dir == 1 ? m.Mg : m.Mh)) + 3 * ((size_t)np * e + id);
+      const double* Jd = (dir == 0 ? m.Mf : (dir == 1 ? m.Mg : m.Mh)) + 3 * ((size_t)np * e + id);
       const double ns0 = sgn * Jd[0], ns1 = sgn * Jd[1], ns2 = sgn * Jd[2];
       se = sqrt(ns0 * ns0 + ns1 * ns1 + ns2 * ns2);
       const double mse = ms / se;
@@ -183,14 +182,7 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
   double sjd = 0.0;
   if (act) {
     RF Ja[9], sj;
-    if constexpr (AFF) {
-      const double* je = m.aff + 10 * (size_t)e;
-#pragma unroll
-      for (int r = 0; r < 9; ++r) Ja[r] = (RF)je[r];
-      sj = (RF)je[9];
-    } else {
-      load_metrics<RF>(m, gid, Ja, sj);
-    }
+    load_metrics<RF>(m, gid, Ja, sj);
     RF g[12];
     lift_node<N, RF>(t, sA + 3 * np, sB, sNb, Ja, sj, g);  // u,v,w,T rows
     if (Gout) {  // (np, 12, nElems) like the four-kernel path
@@ -243,10 +235,8 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
   for (int d = 0; d < 3; ++d) {
     RF* sM = sJa;
     if (act) {
-      if constexpr (!AFF) {
-        const double* Jg = (d == 0 ? m.Mf : (d == 1 ? m.Mg : m.Mh)) + 3 * gid;
-        sM[t] = (RF)Jg[0]; sM[np + t] = (RF)Jg[1]; sM[2 * np + t] = (RF)Jg[2];
-      }
+      const double* Jg = (d == 0 ? m.Mf : (d == 1 ? m.Mg : m.Mh)) + 3 * gid;
+      sM[t] = (RF)Jg[0]; sM[np + t] = (RF)Jg[1]; sM[2 * np + t] = (RF)Jg[2];
 #pragma unroll
       for (int c = 0; c < 4; ++c) sF[c * np + t] = fv[4 * d + c];
       if (d == 2 && st.mode != 0) {
@@ -259,8 +249,7 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
     }
     __syncthreads();
     if (act) {
-      const double* je = m.aff + (AFF ? 10 * (size_t)e + 3 * d : 0);
-      const RF m0 = AFF ? (RF)je[0] : sM[t], m1 = AFF ? (RF)je[1] : sM[np + t], m2 = AFF ? (RF)je[2] : sM[2 * np + t];
+      const RF m0 = sM[t], m1 = sM[np + t], m2 = sM[2 * np + t];
       const int me = d == 0 ? i : (d == 1 ? j : k);
       const int stride = d == 0 ? 1 : (d == 1 ? n : n * n);
       const int base = t - me * stride;
@@ -277,8 +266,7 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
         // Pirozzoli two-point flux with the metric average a = b/2 (SplitVolumeFluxPI,
         // splitflux.f90:603-666), weighted by DV: with b = Ja_i + Ja_l, h = DV/2, Qh = h rs (b.u_sum)/4
         // and P = h p_sum, DV*F = (2 Qh, Qh u_sum + b P, Qh H_sum)
-        const RF b0 = m0 + (AFF ? m0 : (RF)sM[id]), b1 = m1 + (AFF ? m1 : (RF)sM[np + id]),
-                 b2 = m2 + (AFF ? m2 : (RF)sM[2 * np + id]);
+        const RF b0 = m0 + (RF)sM[id], b1 = m1 + (RF)sM[np + id], b2 = m2 + (RF)sM[2 * np + id];
         const RF mb = b0 * us + b1 * vs + b2 * ws;  // 2 (a . u_sum)
         const RF h = (RF)DVh[l + n * me];
         const RF Qh = h * (RF(0.25) * rs * mb);
@@ -301,7 +289,7 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
   double un[5] = {0, 0, 0, 0, 0};
   if constexpr (!LAM) {
     if (act) {
-      sjd = AFF ? m.aff[10 * (size_t)e + 9] : m.sJ[gid];
+      sjd = m.sJ[gid];
       double ut[5];
 #pragma unroll
       for (int v = 0; v < 5; ++v) ut[v] = (-(double)acc[v]) * sjd;
@@ -335,7 +323,7 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
     // it; this instance is held to six waves per SIMD (76 VGPRs) instead of eight, which spilled.
     double rn[5] = {0, 0, 0, 0, 0};
     if (act) {
-      sjd = AFF ? m.aff[10 * (size_t)e + 9] : m.sJ[gid];
+      sjd = m.sJ[gid];
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
         const double ut = (-(double)acc[v]) * sjd;
@@ -346,9 +334,7 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
     double lam[6] = {0, 0, 0, 0, 0, 0};
     int isnan_rho = 0;
     if (act) {
-      const double* je = m.aff + 10 * (size_t)e;
-      dt_node_lambda(un, gas, sjd, AFF ? je : m.Mf + 3 * gid, AFF ? je + 3 : m.Mg + 3 * gid, AFF ? je + 6 : m.Mh + 3 * gid,
-                     lam, isnan_rho);
+      dt_node_lambda(un, gas, sjd, m.Mf + 3 * gid, m.Mg + 3 * gid, m.Mh + 3 * gid, lam, isnan_rho);
     }
     double mx[6];
     int nanr = 0;
@@ -441,13 +427,12 @@ hipError_t fused_n(const DevMesh& m, const FusedWork& w, const Gas& gas, int rie
       const double* FUc = w.FU[cur];
       double* FUn = w.FU[1 - cur];
       const RF* FG = (const RF*)w.FG;
-#define FXG_LAUNCH2(SOLV, BCV, LAM, AFF)                                                                              \
-      hipLaunchKernelGGL((k_dg_fused<N, RF, SOLV, BCV, LAM, AFF>), dim3(K), dim3(NT), 0, s, U, m, FUc, FUn, FG, gas, \
+#define FXG_LAUNCH2(SOLV, BCV, LAM)                                                                              \
+      hipLaunchKernelGGL((k_dg_fused<N, RF, SOLV, BCV, LAM>), dim3(K), dim3(NT), 0, s, U, m, FUc, FUn, FG, gas, \
                          Ut, st, (RF*)G, w.bcP)
 #define FXG_LAUNCH(SOLV, BCV)                                                                                   \
       do {                                                                                                      \
-        if (st.lamSum) { if (m.aff) FXG_LAUNCH2(SOLV, BCV, true, true); else FXG_LAUNCH2(SOLV, BCV, true, false); } \
-        else { if (m.aff) FXG_LAUNCH2(SOLV, BCV, false, true); else FXG_LAUNCH2(SOLV, BCV, false, false); }     \
+        if (st.lamSum) FXG_LAUNCH2(SOLV, BCV, true); else FXG_LAUNCH2(SOLV, BCV, false);                         \
       } while (0)
       if (riemann == 1) {
         if (bc) FXG_LAUNCH(1, true); else FXG_LAUNCH(1, false);

@@ -57,7 +57,7 @@ struct DevMesh {
   // node (index in U) of the neighbour at every own face point, same shape; null on meshes with boundary sides
   const unsigned* nbNode = nullptr;
   // metric terms of each element, (10, nElems): Ja^1..3 x,y,z and sJ, where every element has the same
-  // values at all of its nodes; null otherwise
+  // values at all of its nodes (FP64 only); null otherwise
   const double* aff = nullptr;
 };
 

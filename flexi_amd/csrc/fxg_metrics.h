@@ -14,12 +14,13 @@ namespace fxg {
 // slave element's own n*SurfElem of every inner side point, (3,0:N,0:N,nSides), oriented as the
 // master's normal. `m` supplies ElemToSide and S2V2. With `reference`, the metrics.f90 operation
 // order (absolute coordinates, one-dimensional basis changes in sequence, no FMA contraction;
-// SlaveNS must be null); otherwise coordinates relative to each element's first node. Returns
-// nonzero and sets `err` on failure.
+// SlaveNS must be null); otherwise coordinates relative to each element's first node, and with `flat` the
+// terms of a mesh of parallelepipeds exactly constant in each element. Returns nonzero and sets `err` on
+// failure.
 int compute_metrics_gpu(int N, int nodeType, int NGeo, int nElems, const double* NodeCoords, const DevMesh& m,
                         double* Mf, double* Mg, double* Mh, double* sJ, double* xGP, double* NormVec,
                         double* TangVec1, double* TangVec2, double* SurfElem, double* SlaveNS, bool reference,
-                        hipStream_t s, std::string& err);
+                        bool flat, hipStream_t s, std::string& err);
 
 // Whether every element's metric terms (m.Mf, m.Mg, m.Mh, m.sJ) are bitwise the same at all of its nodes, and
 // those values into aff(10, nElems): Ja^1..3 x,y,z and sJ. `flag` is device scratch of one int.

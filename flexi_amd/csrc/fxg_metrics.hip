@@ -628,7 +628,7 @@ __global__ __launch_bounds__(512) void k_metrics_ref(const double* __restrict__ 
 int compute_metrics_gpu(int N, int nodeType, int NGeo, int nElems, const double* NodeCoords, const DevMesh& m,
                         double* Mf, double* Mg, double* Mh, double* sJ, double* xGP, double* NormVec,
                         double* TangVec1, double* TangVec2, double* SurfElem, double* SlaveNS, bool reference,
-                        hipStream_t s, std::string& err) {
+                        bool flat, hipStream_t s, std::string& err) {
   using namespace basis;
   MetricMats M(N, NGeo);
   const int n = N + 1, ng = NGeo + 1, NGeoRef = 3 * NGeo;
@@ -698,8 +698,8 @@ int compute_metrics_gpu(int N, int nodeType, int NGeo, int nElems, const double*
   double *dm = nullptr, *XCLN = nullptr, *dXCLG = nullptr, *detRef = nullptr, *edge = nullptr;
   // edge vectors, the largest coordinate and the affine flag
   hipError_t e = hipMalloc((void**)&edge, ((size_t)9 * nElems + 2) * sizeof(double));
-  int affine = 1;
-  if (e == hipSuccess) {
+  int affine = flat;
+  if (e == hipSuccess && flat) {
     unsigned long long* big = reinterpret_cast<unsigned long long*>(edge + (size_t)9 * nElems);
     int* ok = reinterpret_cast<int*>(big + 1);
     const unsigned long long zero = 0;

@@ -11,14 +11,12 @@ namespace {
 
 // FP32-bulk, one lane per boundary node. U is converted from global memory directly and the kernel is
 // held to 64 VGPRs (18 KB: four workgroups per CU). On meshes with boundary sides (BC) it also keeps the
-// gradients of the boundary face points for k_bc_visc. AFF: every element's metric terms are the same at all
-// of its nodes (m.aff); they then come as ten uniform values of the element instead of rows of Jsoa (46 bytes
-// per node of 143 at N=7; 32^3: 0.42 -> 0.31 ms).
+// gradients of the boundary face points for k_bc_visc.
 // FIRST: no stage has left the face states of U (a right-hand side alone, the first stage of a step on
 // a caller's state): the neighbours' states come from their nodes in U and the own face states are
 // written to FU for the stage kernel. Replaces a pass of its own over U (k_faces_of, 64 bytes per node at
 // N=7 and one launch; right-hand side at 32^3, N=7, FP64: 1.38 -> 1.30 ms).
-template <int N, class RF, bool BC, bool AFF, bool FIRST>
+template <int N, class RF, bool BC, bool FIRST>
 __global__ __launch_bounds__(D<N>::NT)
 __attribute__((amdgpu_waves_per_eu(N == 7 ? 8 : 6))) void k_visc_faces(
     const double* __restrict__ U, DevMesh m, const double* __restrict__ Jsoa, double* __restrict__ FU,
@@ -91,15 +89,11 @@ __attribute__((amdgpu_waves_per_eu(N == 7 ? 8 : 6))) void k_visc_faces(
   const int sides = node_sides<N>(i, j, k);
   const GasT<RF> gt(gas);
   // metric terms of the boundary nodes only, rows of NB per element (Jsoa layout)
-  // (AFF: through vector registers like the rows, an opaque zero keeps them from the scalar ones, which
-  // cost a spill at the register caps)
-  int z = 0;
-  if constexpr (AFF) asm volatile("" : "+v"(z));
-  const double* Je = AFF ? m.aff + (size_t)10 * e + z : Jsoa + (size_t)10 * NB * e;
+  const double* Je = Jsoa + (size_t)10 * NB * e;
   RF Ja[9], sj;
 #pragma unroll
-  for (int r = 0; r < 9; ++r) Ja[r] = (RF)Je[AFF ? r : r * NB + t];
-  sj = (RF)Je[AFF ? 9 : 9 * NB + t];
+  for (int r = 0; r < 9; ++r) Ja[r] = (RF)Je[r * NB + t];
+  sj = (RF)Je[9 * NB + t];
   RF g[12];
   lift_node<N, RF>(nd, sP, sB, sNb, Ja, sj, g);
   RF fx[4], fy[4], fz[4];
@@ -427,7 +421,7 @@ hipError_t launch_visc_faces(const DevMesh& m, bool fp32, bool faces_fresh, cons
 #define FXG_LAUNCH2(NN, BC, AFF, FIRST)                                                                            \
   do {                                                                                                             \
     if (fp32)                                                                                                      \
-      hipLaunchKernelGGL((k_visc_faces<NN, float, BC, AFF, FIRST>), dim3(m.nElems), dim3(D<NN>::NT), 0, s, U, m,    \
+      hipLaunchKernelGGL((k_visc_faces<NN, float, BC, FIRST>), dim3(m.nElems), dim3(D<NN>::NT), 0, s, U, m,    \
                          Jsoa, FU, (float*)FG, gas, (float*)gBC);                                                  \
     else                                                                                                           \
       hipLaunchKernelGGL((k_visc_lines<NN, BC, AFF, FIRST>), dim3(m.nElems), dim3(S<NN>::NT), 0, s, U, m, m.basis, \
