@@ -400,8 +400,15 @@ int finish_setup(fxg_ctx* c) {
       c->m.aff = all ? aff : nullptr;
     }
     if (c->fused && !c->m.aff) {  // the boundary nodes' metric terms, packed for the viscous face kernel
-      if (alloc_owned(c, &c->fw.Jsoa, fxg::packed_metrics_size(c->N, c->K))) return 1;
-      HIPCHECK(fxg::launch_pack_metrics(c->m, c->fw.Jsoa, c->stream));
+      const bool bulk = c->p.precision == FXG_PREC_FP32_BULK;
+      char* Jsoa;
+      if (alloc_owned(c, &Jsoa, fxg::packed_metrics_size(c->N, c->K) * (bulk ? sizeof(float) : sizeof(double)))) return 1;
+      c->fw.Jsoa = Jsoa;
+      const size_t points = (size_t)6 * c->nf * c->K;
+      if (bulk && (alloc_owned(c, &c->fw.Jnode, (size_t)9 * c->np * c->K) || alloc_owned(c, &c->fw.faceNv, 3 * points) ||
+                   alloc_owned(c, &c->fw.faceSe, points)))
+        return 1;
+      HIPCHECK(fxg::launch_pack_metrics(c->m, c->fw, bulk, c->stream));
     }
   }
   HIPCHECK(hipStreamSynchronize(c->stream));

@@ -54,12 +54,17 @@ struct LdsB {
 // share a CU (six waves per SIMD below N=7, where 8 would spill, and in the last stage of a step).
 // LAM: the last stage of a step, which also forms CALCTIMESTEP's per-element spectral radii of the
 // new state.
+// The metric terms come rounded and packed, Jnode (36 bytes per node, coalesced rows), the face points' normals and
+// SurfElem from faceNv, faceSe (15 bytes per node at N=7): 32^3, N=7 1.28 ms with the FP64 nodal arrays (72 bytes
+// per node, twice, and a root and a division per face point), 1.13 ms now, some 290 bytes per node at 4.4 TB/s.
 template <int N, class RF, int SOLVER, bool BC, bool LAM>
 __global__ __launch_bounds__(D<N>::NT)
 __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(const double* U, DevMesh m, const double* __restrict__ FU,
                                                      double* __restrict__ FUnext, const RF* __restrict__ FG,
                                                      Gas gas, double* Ut, RKStage st, RF* __restrict__ Gout,
-                                                     const double* __restrict__ bcP) {
+                                                     const double* __restrict__ bcP, const RF* __restrict__ Jnode,
+                                                     const RF* __restrict__ faceNv,
+                                                     const double* __restrict__ faceSe) {
   constexpr int n = D<N>::n, nf = D<N>::nf, np = D<N>::np, NT = D<N>::NT, NF = D<N>::NF;
   using L = LdsB<N>;
   // LDS holds the working precision RF: the values are rounded to RF where they are stored, as
@@ -76,6 +81,7 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
   const int e = blockIdx.x, t = threadIdx.x;
   const bool act = t < np;
   const size_t gid = (size_t)np * e + (act ? t : 0);
+  const RF* Je = Jnode + (size_t)9 * np * e;
   // the basis, with the DVolSurf block halved (exact) for the split-flux loop
   for (int x = t; x < 3 * n * n + 4 * n; x += NT) {
     const double b = m.basis[x];
@@ -110,25 +116,10 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
     RF gn[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) gn[c] = FG[4 * (size_t)nb + c];
-    // (the same arithmetic as face_frame, written out: the register allocation of this kernel
-    // stays within 128 VGPRs this way)
-    double se;
-    RF nv[3];  // master normal
-    if (m.ownFaceMetric) {
-      // own outward normal times SurfElem from the own metric terms at the boundary node
-      const int dir = dir_of(ls);
-      const double sgn = normal_sign(ls);
-      const double* Jd = (dir == 0 ? m.Mf : (dir == 1 ? m.Mg : m.Mh)) + 3 * ((size_t)np * e + id);
-      const double ns0 = sgn * Jd[0], ns1 = sgn * Jd[1], ns2 = sgn * Jd[2];
-      se = sqrt(ns0 * ns0 + ns1 * ns1 + ns2 * ns2);
-      const double mse = ms / se;
-      nv[0] = (RF)(ns0 * mse); nv[1] = (RF)(ns1 * mse); nv[2] = (RF)(ns2 * mse);
-    } else {
-      // the side's normal and surface element, shared by master and slave as in FLEXI
-      const size_t sp = slot_side_point<N>(own);
-      se = m.SurfElem[sp];
-      nv[0] = (RF)m.NormVec[3 * sp]; nv[1] = (RF)m.NormVec[3 * sp + 1]; nv[2] = (RF)m.NormVec[3 * sp + 2];
-    }
+    // master normal and SurfElem of the own face point
+    const double se = faceSe[(size_t)NF * e + x];
+    const RF* fn = faceNv + (size_t)3 * NF * e + x;
+    const RF nv[3] = {fn[0], fn[NF], fn[2 * NF]};
     // tangential basis: Gram-Schmidt of the coordinate axis least aligned with n
     RF t1[3], t2[3];
     {
@@ -182,7 +173,9 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
   double sjd = 0.0;
   if (act) {
     RF Ja[9], sj;
-    load_metrics<RF>(m, gid, Ja, sj);
+#pragma unroll
+    for (int r = 0; r < 9; ++r) Ja[r] = Je[r * np + t];
+    sj = (RF)m.sJ[gid];
     RF g[12];
     lift_node<N, RF>(t, sA + 3 * np, sB, sNb, Ja, sj, g);  // u,v,w,T rows
     if (Gout) {  // (np, 12, nElems) like the four-kernel path
@@ -235,8 +228,8 @@ __attribute__((amdgpu_waves_per_eu(N == 7 && !LAM ? 8 : 6))) void k_dg_fused(con
   for (int d = 0; d < 3; ++d) {
     RF* sM = sJa;
     if (act) {
-      const double* Jg = (d == 0 ? m.Mf : (d == 1 ? m.Mg : m.Mh)) + 3 * gid;
-      sM[t] = (RF)Jg[0]; sM[np + t] = (RF)Jg[1]; sM[2 * np + t] = (RF)Jg[2];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) sM[c * np + t] = Je[(3 * d + c) * np + t];
 #pragma unroll
       for (int c = 0; c < 4; ++c) sF[c * np + t] = fv[4 * d + c];
       if (d == 2 && st.mode != 0) {
@@ -429,7 +422,7 @@ hipError_t fused_n(const DevMesh& m, const FusedWork& w, const Gas& gas, int rie
       const RF* FG = (const RF*)w.FG;
 #define FXG_LAUNCH2(SOLV, BCV, LAM)                                                                              \
       hipLaunchKernelGGL((k_dg_fused<N, RF, SOLV, BCV, LAM>), dim3(K), dim3(NT), 0, s, U, m, FUc, FUn, FG, gas, \
-                         Ut, st, (RF*)G, w.bcP)
+                         Ut, st, (RF*)G, w.bcP, w.Jnode, w.faceNv, w.faceSe)
 #define FXG_LAUNCH(SOLV, BCV)                                                                                   \
       do {                                                                                                      \
         if (st.lamSum) FXG_LAUNCH2(SOLV, BCV, true); else FXG_LAUNCH2(SOLV, BCV, false);                         \
@@ -449,24 +442,42 @@ hipError_t fused_n(const DevMesh& m, const FusedWork& w, const Gas& gas, int rie
 }
 
 // Packs the metric terms of the boundary nodes, (3,np,K) x 3 and sJ (np,K), into rows of NB
-// per element in boundary-node order (bnd_rank).
-template <int N>
-__global__ __launch_bounds__(256) void k_pack_metrics(DevMesh m, size_t nNodes, double* __restrict__ J) {
+// per element in boundary-node order (bnd_rank); in FP32-bulk Ja of every node into rows of np too.
+template <int N, class RF>
+__global__ __launch_bounds__(256) void k_pack_metrics(DevMesh m, size_t nNodes, RF* __restrict__ J, RF* __restrict__ Jnode) {
   constexpr int n = N + 1, np = D<N>::np, NB = Bnd<N>::NB;
   const size_t x = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (x >= nNodes) return;
   const size_t e = x / np;
   const int t = (int)(x - e * np);
   const int i = t % n, j = (t / n) % n, k = t / (n * n);
-  if (!node_sides<N>(i, j, k)) return;
-  double* Je = J + 10 * NB * e + bnd_rank<N>(i, j, k);
+  RF Ja[9], sj;
+  load_metrics<RF>(m, x, Ja, sj);
+  if constexpr (sizeof(RF) == 4)
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    Je[(0 + c) * NB] = m.Mf[3 * x + c];
-    Je[(3 + c) * NB] = m.Mg[3 * x + c];
-    Je[(6 + c) * NB] = m.Mh[3 * x + c];
-  }
-  Je[9 * NB] = m.sJ[x];
+    for (int r = 0; r < 9; ++r) Jnode[(9 * e + r) * np + t] = Ja[r];
+  if (!node_sides<N>(i, j, k)) return;
+  RF* Je = J + 10 * NB * e + bnd_rank<N>(i, j, k);
+#pragma unroll
+  for (int r = 0; r < 9; ++r) Je[r * NB] = Ja[r];
+  Je[9 * NB] = sj;
+}
+
+// Master normal and SurfElem of every own face point (face_frame in FP64, the normal rounded).
+template <int N>
+__global__ __launch_bounds__(256) void k_pack_faces(DevMesh m, size_t total, float* __restrict__ faceNv,
+                                                  double* __restrict__ faceSe) {
+  constexpr int n = N + 1, nf = n * n, NF = 6 * nf;
+  const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (g >= total) return;
+  const size_t e = g / NF;
+  const int x = (int)(g - e * NF), ls = x / nf + 1, ab = x - (ls - 1) * nf, dir = dir_of(ls);
+  const double* Jd = (dir == 0 ? m.Mf : (dir == 1 ? m.Mg : m.Mh)) + 3 * ((size_t)(n * nf) * e + vidx<N>(ls, ab % n, ab / n));
+  const unsigned own = m.slotTab[g];
+  float nv[3], t1[3], t2[3];
+  faceSe[g] = face_frame<N, float>(m, Jd, ls, own, slot_is_master<N>(own), nv, t1, t2);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) faceNv[3 * NF * e + c * NF + x] = nv[c];
 }
 
 template <int N>
@@ -544,13 +555,21 @@ size_t packed_metrics_size(int N, int nElems) {
   return (size_t)10 * (2 * n * n + (N - 1) * 4 * N) * nElems;
 }
 
-hipError_t launch_pack_metrics(const DevMesh& m, double* Jsoa, hipStream_t s) {
-  const int np = (m.N + 1) * (m.N + 1) * (m.N + 1);
-  const size_t nNodes = (size_t)np * m.nElems;
-  const dim3 g((unsigned)((nNodes + 255) / 256)), b(256);
+hipError_t launch_pack_metrics(const DevMesh& m, const FusedWork& w, int fp32, hipStream_t s) {
+  if (!m.slotTab) return hipErrorInvalidValue;
+  const int nf = (m.N + 1) * (m.N + 1), np = nf * (m.N + 1);
+  const size_t nNodes = (size_t)np * m.nElems, points = (size_t)6 * nf * m.nElems;
+  const dim3 g((unsigned)((nNodes + 255) / 256)), gf((unsigned)((points + 255) / 256)), b(256);
   switch (m.N) {
-#define FXG_CASE(NN) \
-  case NN: hipLaunchKernelGGL((k_pack_metrics<NN>), g, b, 0, s, m, nNodes, Jsoa); break;
+#define FXG_CASE(NN)                                                                                                     \
+  case NN:                                                                                                               \
+    if (fp32) {                                                                                                          \
+      hipLaunchKernelGGL((k_pack_metrics<NN, float>), g, b, 0, s, m, nNodes, (float*)w.Jsoa, w.Jnode);                    \
+      hipLaunchKernelGGL((k_pack_faces<NN>), gf, b, 0, s, m, points, w.faceNv, w.faceSe);                                \
+    } else {                                                                                                             \
+      hipLaunchKernelGGL((k_pack_metrics<NN, double>), g, b, 0, s, m, nNodes, (double*)w.Jsoa, (double*)nullptr);         \
+    }                                                                                                                    \
+    break;
     FXG_CASE(2) FXG_CASE(3) FXG_CASE(4) FXG_CASE(5) FXG_CASE(6) FXG_CASE(7)
 #undef FXG_CASE
     default: return hipErrorInvalidValue;

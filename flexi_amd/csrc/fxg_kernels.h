@@ -113,18 +113,25 @@ hipError_t launch_rhs(const DevMesh& m, const DevWork& w, const Gas& gas, int no
 struct FusedWork {
   double* FU[2];  // face states, 5 per side point and slot, double-buffered across stages
   void* FG;       // viscous normal face fluxes f_v.(n SurfElem), 4 per side point and slot
-  double* Jsoa;   // metric terms of the boundary nodes, rows of NB per element: Ja^1..3 x,y,z, sJ
+  // metric terms of the boundary nodes, rows of NB per element: Ja^1..3 x,y,z, sJ (float in FP32-bulk)
+  void* Jsoa = nullptr;
+  // FP32-bulk: Ja^1..3 x,y,z of every node as the kernel uses them, rows of (N+1)^3 per element, and master
+  // normal (3 rows) and SurfElem of every own face point, rows of 6 (N+1)^2 per element
+  float* Jnode = nullptr;
+  float* faceNv = nullptr;
+  double* faceSe = nullptr;
   // per boundary side point, (4,0:N,0:N,nBC): walls the pressure (PRESSURE_RIEMANN) first, Riemann-type
   // boundaries the boundary state's velocity in 1..3
   double* bcP = nullptr;
   void* gBC = nullptr;    // lifted gradients at the boundary side points, 12 per point (gradient type)
 };
-// Doubles of FusedWork::Jsoa.
+// Values of FusedWork::Jsoa.
 size_t packed_metrics_size(int N, int nElems);
 // Face states of U into a face array laid out like FusedWork::FU (Gauss-Lobatto).
 hipError_t launch_faces_of(const DevMesh& m, const double* U, double* FU, hipStream_t s);
-// Fills FusedWork::Jsoa (boundary-node metric terms) from the FLEXI-layout metric arrays of `m`.
-hipError_t launch_pack_metrics(const DevMesh& m, double* Jsoa, hipStream_t s);
+// Fills FusedWork::Jsoa (boundary-node metric terms) from the FLEXI-layout metric arrays of `m`, in FP32-bulk
+// also Jnode, faceNv and faceSe (m.slotTab set).
+hipError_t launch_pack_metrics(const DevMesh& m, const FusedWork& w, int fp32, hipStream_t s);
 // Fills slot(6*(N+1)^2, nElems) with face_slot of every own face point (m.slotTab must be null).
 hipError_t launch_slot_table(const DevMesh& m, unsigned* slot, hipStream_t s);
 // Fills nbNode(6*(N+1)^2, nElems) (m.slotTab set, no boundary sides); slotNode is scratch of 2*(N+1)^2*nSides.
@@ -136,7 +143,7 @@ bool fused_supported(int N, int nodeType, int split, long long nSides);
 // Kernel A of the fused stage (fxg_visc.hip): viscous normal face fluxes into FG (float if fp32). Unless
 // faces_fresh (FU holds the face states of U) it reads the neighbours' states from U and fills FU; that form
 // needs m.nbNode.
-hipError_t launch_visc_faces(const DevMesh& m, bool fp32, bool faces_fresh, const double* U, const double* Jsoa,
+hipError_t launch_visc_faces(const DevMesh& m, bool fp32, bool faces_fresh, const double* U, const void* Jsoa,
                              double* FU, void* FG, const Gas& gas, void* gBC, const double* bcP, hipStream_t s);
 // Boundary sides on the fused path (fxg_visc.hip): the outer slot of each boundary side point gets a
 // face state whose BR1 lifting difference with the inner state is the boundary lifting flux (and,

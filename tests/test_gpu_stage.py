@@ -85,3 +85,22 @@ def test_stage_constant_metrics_against_oracle(N, how):
         assert gpu.CalcTimeStep() == dt_stage
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("N", [2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("how", ["own", "host", "reference"])
+def test_bulk_stage_against_oracle(N, how):
+    """FP32-bulk: packed metric terms of the nodes and the face points, from either side's own face
+    metric or the side's normals. Bound: sums of up to 48 products rounded to 2^-24 whose terms are up to
+    16 times the sum, 48 * 2^-24 * 16 = 4.6e-5."""
+    from flexi_amd.solver import DGSolver
+    mesh = periodic_box(3, 2, 4, NGeo=2, deform=sine_deform(0.1))
+    m = orc.calc_metrics(N, orc.NODE_GL, mesh)
+    U = testcase.tgv_density_perturbed(m["Elem_xGP"], amplitude=1e-2, Ma=1.0)
+    ref = orc.Solver(orc.params(N, orc.NODE_GL, 1, orc.RIEMANN_ROE), mesh, m)
+    kw = dict(metrics=m) if how == "host" else dict(metric_order=how)
+    gpu = DGSolver(mesh, N, node_type="gauss-lobatto", split_dg="pi", riemann="roe", precision="fp32-bulk", **kw)
+    try:
+        assert rel(gpu.rhs(U), ref.rhs(U)) <= 4.6e-5
+    finally:
+        gpu.close()
