@@ -164,7 +164,7 @@ struct fxg_ctx {
   bool weak = false;
   fxg::FusedWork fw{};
   int cur = 0;
-  // the state whose face values FU[cur] holds (only trusted for the context's own state, which
+  // the state whose face values FU[cur] (four-kernel path: w.Uf_m, w.Uf_s) holds (only trusted for the context's own state, which
   // changes only through fxg_set_state and the library's own updates)
   const double* faces_of = nullptr;
   // Ut and the lifted gradients (G) of the context's last right-hand side. After an LSERK step on
@@ -425,8 +425,8 @@ void ctx_free(fxg_ctx* c) {
   delete c;
 }
 
-// One right-hand side (st.mode 0) or LSERK stage. On the fused path `faces_fresh` says that
-// FU[cur] already holds the face states of U (written by the previous stage). `keep_grads`: the fused
+// One right-hand side (st.mode 0) or LSERK stage. `faces_fresh` says that FU[cur] (four-kernel path: Uf_m and
+// Uf_s) already holds the face states of U (written by the previous stage). `keep_grads`: the fused
 // path's right-hand side also stores the lifted gradients in G (96 bytes per node; only the context's
 // own right-hand side is ever asked for them), and so does the weak form's. The four-kernel path goes
 // through G in any case.
@@ -450,18 +450,12 @@ int rhs(fxg_ctx* c, const double* U, double* Ut, const fxg::RKStage& st, hipStre
     return 0;
   }
   HIPCHECK(fxg::launch_rhs(c->m, c->w, c->gas, c->p.nodeType, c->p.splitDG == FXG_SPLITDG_PI, c->p.riemann,
-                           c->p.precision == FXG_PREC_FP32_BULK, U, Ut, st, s, c->timer));
+                           c->p.precision == FXG_PREC_FP32_BULK, U, Ut, st, faces_fresh, s, c->timer));
+  c->faces_of = U;
   return 0;
 }
 
-// One LSERK stage (st = 0 .. nStages-1) of TimeStepByLSERKW2 on (U, R).
-int lserk_stage(fxg_ctx* c, double dt, int st, const double* RKA, const double* RKb, double* U, double* R,
-                hipStream_t s) {
-  fxg::RKStage stage{st == 0 ? 1 : 2, st == 0 ? 0.0 : -RKA[st - 1], RKb[st] * dt, U, R};
-  return rhs(c, U, nullptr, stage, s, st > 0);
-}
-
-// One TimeStepByLSERKW2 step. `faces_known`: FU[cur] already holds the face values of U (the
+// One TimeStepByLSERKW2 step. `faces_known`: the face arrays already hold the face values of U (the
 // previous step of the same call, or of the context's own state), so the first stage reuses them.
 // `want_lambda`: the fused last stage also stores CALCTIMESTEP's per-element spectral radii of the
 // new state (used by the next fxg_calc_timestep on the context's state).
@@ -735,6 +729,7 @@ int fxg_get_gradients(fxg_ctx* c, int nVarLifting, double* gx, double* gy, doubl
       return fail("fxg_get_gradients: no right-hand side has been evaluated for the current state");
     if (!c->rhoG && alloc_owned(c, &c->rhoG, 3 * nodes)) return 1;
     HIPCHECK(fxg::launch_lift_density(c->m, c->w, c->gas, c->p.nodeType, c->grads_state, c->rhoG, c->stream));
+    if (!c->fused && !c->weak) c->faces_of = nullptr;  // it prolongs that state into the same face arrays
   }
   double* host[3] = {gx, gy, gz};
   for (int d = 0; d < 3; ++d) {
@@ -837,7 +832,7 @@ int fxg_timestep_lserkw2(fxg_ctx* c, double t, double dt, int nStages, const dou
   if (!c) return fail("ctx is NULL");
   c->lam_of = nullptr;
   c->grads_state = nullptr;
-  if (lserk(c, dt, nStages, RKA, RKb, c->U, c->R, c->stream, (c->fused || c->weak) && c->faces_of == c->U, true)) return 1;
+  if (lserk(c, dt, nStages, RKA, RKb, c->U, c->R, c->stream, c->faces_of == c->U, true)) return 1;
   // Ut of the last stage is not kept by either pipeline, the gradients not by the fused one
   c->rhs_stale = true;
   c->last_rhs = 2;
@@ -968,7 +963,7 @@ int fxg_forward_n_steps(fxg_ctx* c, int nSteps, const double* dt, int nStages, c
     if (ckpt && it % checkpointEvery == 0)
       HIPCHECK(hipMemcpyAsync(ckpt + (size_t)(it / checkpointEvery) * vol5, U, vol5 * sizeof(double),
                               hipMemcpyDeviceToDevice, s));
-    if (lserk(c, dt[it], nStages, RKA, RKb, U, c->R, s, it > 0 && (c->fused || c->weak))) {
+    if (lserk(c, dt[it], nStages, RKA, RKb, U, c->R, s, it > 0)) {
       c->faces_of = nullptr;
       return 1;
     }

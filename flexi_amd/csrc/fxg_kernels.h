@@ -104,9 +104,10 @@ struct KernelTimer {
 };
 
 // Runs prolongation, lifting, fluxes and the volume/surface integrals for one RHS.
-// Ut may be null when stage.mode != 0. `timer` may be null.
+// Ut may be null when stage.mode != 0. `timer` may be null. With faces_fresh Uf_m and Uf_s hold the face values of
+// U (a stage leaves those of its new state there), and the prolongation is left out.
 hipError_t launch_rhs(const DevMesh& m, const DevWork& w, const Gas& gas, int nodeType, int split,
-                      int riemann, int fp32, const double* U, double* Ut, const RKStage& stage,
+                      int riemann, int fp32, const double* U, double* Ut, const RKStage& stage, bool faces_fresh,
                       hipStream_t s, KernelTimer* timer);
 // Work arrays of the fused Gauss-Lobatto split-form stage (fxg_fused.hip). Face arrays are
 // indexed ((side*2 + slot)*(N+1)^2 + pq) with slot 0 = master, 1 = slave.

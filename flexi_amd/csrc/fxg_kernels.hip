@@ -67,6 +67,53 @@ __device__ __forceinline__ void stage_u_basis(const double* __restrict__ Ue, dou
   if (t < NBAS) sB[t] = b;
 }
 
+// Side point of own face point x = (ls-1)*nf + a + n*b of element e: its index pq + nf*side, negative (its
+// complement) where the element is the side's slave.
+template <int N>
+__device__ __forceinline__ int side_point(const DevMesh& m, int e, int x) {
+  constexpr int n = N + 1, nf = n * n;
+  const int ls = x / nf + 1, ab = x - (ls - 1) * nf;
+  const int side = m.E2S[2 * (ls - 1) + 12 * e] - 1;
+  const int flip = m.E2S[2 * (ls - 1) + 1 + 12 * e];
+  const int* pq = m.v2s2 + 2 * (ab + nf * (flip + 5 * (ls - 1)));
+  const int fp = pq[0] + n * pq[1] + nf * side;
+  return flip == 0 ? fp : ~fp;
+}
+
+// Values of the element's state sU (5 per node, LDS) at its own face points, into the face arrays; sp: side_point
+// of the lane's face points.
+template <int N, bool GL>
+__device__ __forceinline__ void prolong_faces(const double* sU, const double* sB, const int* sp, double* __restrict__ Um,
+                                            double* __restrict__ Us, int t) {
+  constexpr int n = Dim<N>::n, nf = Dim<N>::nf, NT = Dim<N>::NT, RS = (6 * nf + NT - 1) / NT;
+  const BasisLayout B{n};
+#pragma unroll
+  for (int r = 0; r < RS; ++r) {
+    const int x = t + r * NT;
+    if (x >= 6 * nf) break;
+    const int ls = x / nf + 1, ab = x - (ls - 1) * nf;
+    double out[5];
+    if (GL) {
+      const int id = vol_index<N>(ls, ab % n, ab / n, is_minus(ls) ? 0 : N);
+#pragma unroll
+      for (int v = 0; v < 5; ++v) out[v] = sU[5 * id + v];
+    } else {
+      const double* L = sB + (is_minus(ls) ? B.L_Minus() : B.L_Plus());
+      const int id0 = vol_index<N>(ls, ab % n, ab / n, 0);
+#pragma unroll
+      for (int v = 0; v < 5; ++v) out[v] = sU[5 * id0 + v] * L[0];
+      for (int l = 1; l <= N; ++l) {
+        const int id = vol_index<N>(ls, ab % n, ab / n, l);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) out[v] = out[v] + sU[5 * id + v] * L[l];
+      }
+    }
+    double* dst = sp[r] >= 0 ? Um + 5 * (size_t)sp[r] : Us + 5 * (size_t)~sp[r];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) dst[v] = out[v];
+  }
+}
+
 // ---------------------------------------------------------------------------------------------
 // ProlongToFace of the conservative state (prolongtoface.t90:21-144): every element writes the
 // face values of its six sides into the master or slave face array of the side, reordered into
@@ -77,64 +124,73 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_prolong_u(const double* __restri
   constexpr int n = Dim<N>::n, nf = Dim<N>::nf, np = Dim<N>::np, NT = Dim<N>::NT;
   __shared__ double sU[5 * np];
   __shared__ double sB[3 * n * n + 4 * n];
+  constexpr int RS = (6 * nf + NT - 1) / NT;
   const int e = blockIdx.x;
   const int t = threadIdx.x;
   const double* Ue = U + (size_t)5 * np * e;
+  int sp[RS];
+#pragma unroll
+  for (int r = 0; r < RS; ++r) sp[r] = t + r * NT < 6 * nf ? side_point<N>(m, e, t + r * NT) : 0;
   stage_u_basis<N, NT>(Ue, sU, m.basis, sB, t);
   __syncthreads();
-  const BasisLayout B{n};
-  for (int x = t; x < 6 * nf; x += NT) {
-    const int ls = x / nf + 1, pq = x - (ls - 1) * nf;
-    const int side = m.E2S[2 * (ls - 1) + 12 * e] - 1;
-    const int flip = m.E2S[2 * (ls - 1) + 1 + 12 * e];
-    const int* ab = m.s2v2 + 2 * (pq + nf * (flip + 5 * (ls - 1)));
-    double out[5];
-    if (GL) {
-      const int id = vol_index<N>(ls, ab[0], ab[1], is_minus(ls) ? 0 : N);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) out[v] = sU[5 * id + v];
-    } else {
-      const double* L = sB + (is_minus(ls) ? B.L_Minus() : B.L_Plus());
-      const int id0 = vol_index<N>(ls, ab[0], ab[1], 0);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) out[v] = sU[5 * id0 + v] * L[0];
-      for (int l = 1; l <= N; ++l) {
-        const int id = vol_index<N>(ls, ab[0], ab[1], l);
-#pragma unroll
-        for (int v = 0; v < 5; ++v) out[v] = out[v] + sU[5 * id + v] * L[l];
-      }
-    }
-    double* dst = (flip == 0 ? Um : Us) + 5 * ((size_t)pq + (size_t)nf * side);
-#pragma unroll
-    for (int v = 0; v < 5; ++v) dst[v] = out[v];
-  }
+  prolong_faces<N, GL>(sU, sB, sp, Um, Us, t);
 }
 
 // ---------------------------------------------------------------------------------------------
 // BR1 lifting (Lifting_BR1, lifting_br1.t90:48-181; strong form, non-conservative volume
 // integral lifting_volint.t90:26-118; surface flux lifting_fillflux.t90:40-239), Jacobian,
-// and prolongation of the lifted gradients to the element's six sides.
+// and prolongation of the lifted gradients to the element's six sides. The lifting flux of a face point is
+// formed once, by the lane of that point, and read from LDS by the N+1 nodes of its line (they each formed it
+// from the face states: twelve divisions per node behind three dependent loads, six times over). Gauss, N=3,
+// 20^3, FP32-bulk: 52 -> 33 us, 410 bytes per node at 6 TB/s from the memory-side cache.
 template <int N, bool GL, class RF>
 __global__ __launch_bounds__(Dim<N>::NT) void k_lift(const double* __restrict__ U, DevMesh m,
                                                    const double* __restrict__ Um, const double* __restrict__ Us,
                                                    const double* __restrict__ bcLift, Gas gas, RF* __restrict__ G,
                                                    RF* __restrict__ Gm, RF* __restrict__ Gs) {
   constexpr int n = Dim<N>::n, nf = Dim<N>::nf, np = Dim<N>::np, NT = Dim<N>::NT;
-  __shared__ double sA[12 * np];
+  constexpr int NF = 6 * nf, RS = (NF + NT - 1) / NT;
+  constexpr int LIFT = 5 * np * 8 + 7 * NF * (int)sizeof(RF), GRAD = 12 * np * (int)sizeof(RF);
+  __shared__ double sA[((LIFT > GRAD ? LIFT : GRAD) + 7) / 8];  // U, then the lifting variables (u,v,w,T), SoA
+  RF* sP = reinterpret_cast<RF*>(sA);
+  RF* sS = reinterpret_cast<RF*>(sA + 5 * np);  // own face points: 0.5*(U_slave-U_master)*SurfElem (4 rows), n (3)
   __shared__ double sB[3 * n * n + 4 * n];
   const BasisLayout B{n};
   const int e = blockIdx.x;
   const int t = threadIdx.x;
   const double* Ue = U + (size_t)5 * np * e;
+  int sp[RS];
+#pragma unroll
+  for (int r = 0; r < RS; ++r) sp[r] = t + r * NT < NF ? side_point<N>(m, e, t + r * NT) : 0;
   stage_u_basis<N, NT>(Ue, sA, m.basis, sB, t);
+#pragma unroll
+  for (int r = 0; r < RS; ++r) {
+    const int x = t + r * NT;
+    if (x >= NF) break;
+    const size_t fp = sp[r] >= 0 ? sp[r] : ~sp[r];
+    const RF se = (RF)m.SurfElem[fp];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) sS[(4 + d) * NF + x] = (RF)m.NormVec[3 * fp + d];
+    if (fp < (size_t)m.nBC * nf) {  // boundary side: Lifting_GetBoundaryFlux (k_bc_lift) times SurfElem
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sS[v * NF + x] = (RF)bcLift[4 * fp + v] * se;
+    } else {
+      const Prim pm = cons_to_prim(Um + 5 * fp, gas);
+      const Prim ps = cons_to_prim(Us + 5 * fp, gas);
+      const RF dq[4] = {(RF)ps.u - (RF)pm.u, (RF)ps.v - (RF)pm.v, (RF)ps.w - (RF)pm.w, (RF)ps.T - (RF)pm.T};
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sS[v * NF + x] = RF(0.5) * dq[v] * se;
+    }
+  }
   __syncthreads();
-  double* sP = sA + 5 * np;  // lifting variables (u,v,w,T), SoA
+  Prim q{};
+  if (t < np) q = cons_to_prim(sA + 5 * t, gas);
+  __syncthreads();
   if (t < np) {
-    const Prim q = cons_to_prim(sA + 5 * t, gas);
-    sP[t] = q.u;
-    sP[np + t] = q.v;
-    sP[2 * np + t] = q.w;
-    sP[3 * np + t] = q.T;
+    sP[t] = (RF)q.u;
+    sP[np + t] = (RF)q.v;
+    sP[2 * np + t] = (RF)q.w;
+    sP[3 * np + t] = (RF)q.T;
   }
   __syncthreads();
   RF g[12];
@@ -144,17 +200,17 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_lift(const double* __restrict__ 
     RF gxi[4], geta[4], gzeta[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      gxi[v] = (RF)DT[0 + n * i] * (RF)sP[v * np + (0 + n * (j + n * k))];
-      geta[v] = (RF)DT[0 + n * j] * (RF)sP[v * np + (i + n * (0 + n * k))];
-      gzeta[v] = (RF)DT[0 + n * k] * (RF)sP[v * np + (i + n * (j + n * 0))];
+      gxi[v] = (RF)DT[0 + n * i] * sP[v * np + (0 + n * (j + n * k))];
+      geta[v] = (RF)DT[0 + n * j] * sP[v * np + (i + n * (0 + n * k))];
+      gzeta[v] = (RF)DT[0 + n * k] * sP[v * np + (i + n * (j + n * 0))];
     }
     for (int l = 1; l <= N; ++l) {
       const RF dxi = (RF)DT[l + n * i], deta = (RF)DT[l + n * j], dzeta = (RF)DT[l + n * k];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        gxi[v] = gxi[v] + dxi * (RF)sP[v * np + (l + n * (j + n * k))];
-        geta[v] = geta[v] + deta * (RF)sP[v * np + (i + n * (l + n * k))];
-        gzeta[v] = gzeta[v] + dzeta * (RF)sP[v * np + (i + n * (j + n * l))];
+        gxi[v] = gxi[v] + dxi * sP[v * np + (l + n * (j + n * k))];
+        geta[v] = geta[v] + deta * sP[v * np + (i + n * (l + n * k))];
+        gzeta[v] = gzeta[v] + dzeta * sP[v * np + (i + n * (j + n * l))];
       }
     }
     const size_t gid = (size_t)np * e + t;
@@ -175,65 +231,50 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_lift(const double* __restrict__ 
       int a, b, l;
       face_coords(ls, i, j, k, a, b, l);
       if (GL && l != (is_minus(ls) ? 0 : N)) continue;
-      const int side = m.E2S[2 * (ls - 1) + 12 * e] - 1;
-      const int flip = m.E2S[2 * (ls - 1) + 1 + 12 * e];
-      const int* pq2 = m.v2s2 + 2 * ((a + n * b) + nf * (flip + 5 * (ls - 1)));
-      const size_t fp = (size_t)(pq2[0] + n * pq2[1]) + (size_t)nf * side;
-      const RF se = (RF)m.SurfElem[fp];
-      const RF nv[3] = {(RF)m.NormVec[3 * fp], (RF)m.NormVec[3 * fp + 1], (RF)m.NormVec[3 * fp + 2]};
       const RF lh = GL ? (RF)(is_minus(ls) ? sB[B.L_HatMinus()] : sB[B.L_HatPlus() + N])
                        : (RF)(is_minus(ls) ? sB[B.L_HatMinus() + l] : sB[B.L_HatPlus() + l]);
-      RF f[4];
-      if (side < m.nBC) {  // boundary side: Lifting_GetBoundaryFlux (k_bc_lift) times SurfElem
-#pragma unroll
-        for (int v = 0; v < 4; ++v) f[v] = (RF)bcLift[4 * fp + v] * se;
-      } else {
-        const Prim pm = cons_to_prim(Um + 5 * fp, gas);
-        const Prim ps = cons_to_prim(Us + 5 * fp, gas);
-        const RF dq[4] = {(RF)ps.u - (RF)pm.u, (RF)ps.v - (RF)pm.v, (RF)ps.w - (RF)pm.w, (RF)ps.T - (RF)pm.T};
-#pragma unroll
-        for (int v = 0; v < 4; ++v) f[v] = RF(0.5) * dq[v] * se;
-      }
+      const RF* f = sS + (ls - 1) * nf + a + n * b;
 #pragma unroll
       for (int v = 0; v < 4; ++v)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) g[4 * d + v] = g[4 * d + v] + f[v] * nv[d] * lh;
+        for (int d = 0; d < 3; ++d) g[4 * d + v] = g[4 * d + v] + f[v * NF] * f[(4 + d) * NF] * lh;
     }
     const RF sj = (RF)m.sJ[gid];
 #pragma unroll
     for (int c = 0; c < 12; ++c) g[c] = g[c] * sj;
   }
-  __syncthreads();  // all reads of sP are done before sA is overwritten
+  __syncthreads();  // all reads of sP and sS are done before the gradients take their place
+  RF* sG = sP;
   if (t < np) {
     RF* Ge = G + (size_t)12 * np * e;
 #pragma unroll
     for (int c = 0; c < 12; ++c) {
       Ge[c * np + t] = g[c];
-      sA[c * np + t] = (double)g[c];
+      sG[c * np + t] = g[c];
     }
   }
   __syncthreads();
   // ProlongToFaceLifting of the gradients into the side arrays (12 values per side point)
-  for (int x = t; x < 6 * nf; x += NT) {
-    const int ls = x / nf + 1, pq = x - (ls - 1) * nf;
-    const int side = m.E2S[2 * (ls - 1) + 12 * e] - 1;
-    const int flip = m.E2S[2 * (ls - 1) + 1 + 12 * e];
-    const int* ab = m.s2v2 + 2 * (pq + nf * (flip + 5 * (ls - 1)));
-    RF* dst = (flip == 0 ? Gm : Gs) + 12 * ((size_t)pq + (size_t)nf * side);
-    if (GL) {
-      const int id = vol_index<N>(ls, ab[0], ab[1], is_minus(ls) ? 0 : N);
 #pragma unroll
-      for (int c = 0; c < 12; ++c) dst[c] = (RF)sA[c * np + id];
+  for (int r = 0; r < RS; ++r) {
+    const int x = t + r * NT;
+    if (x >= NF) break;
+    const int ls = x / nf + 1, ab = x - (ls - 1) * nf;
+    RF* dst = sp[r] >= 0 ? Gm + 12 * (size_t)sp[r] : Gs + 12 * (size_t)~sp[r];
+    if (GL) {
+      const int id = vol_index<N>(ls, ab % n, ab / n, is_minus(ls) ? 0 : N);
+#pragma unroll
+      for (int c = 0; c < 12; ++c) dst[c] = sG[c * np + id];
     } else {
       const double* L = sB + (is_minus(ls) ? B.L_Minus() : B.L_Plus());
-      const int id0 = vol_index<N>(ls, ab[0], ab[1], 0);
+      const int id0 = vol_index<N>(ls, ab % n, ab / n, 0);
       RF out[12];
 #pragma unroll
-      for (int c = 0; c < 12; ++c) out[c] = (RF)sA[c * np + id0] * (RF)L[0];
+      for (int c = 0; c < 12; ++c) out[c] = sG[c * np + id0] * (RF)L[0];
       for (int l = 1; l <= N; ++l) {
-        const int id = vol_index<N>(ls, ab[0], ab[1], l);
+        const int id = vol_index<N>(ls, ab % n, ab / n, l);
 #pragma unroll
-        for (int c = 0; c < 12; ++c) out[c] = out[c] + (RF)sA[c * np + id] * (RF)L[l];
+        for (int c = 0; c < 12; ++c) out[c] = out[c] + sG[c * np + id] * (RF)L[l];
       }
 #pragma unroll
       for (int c = 0; c < 12; ++c) dst[c] = out[c];
@@ -404,21 +445,32 @@ __global__ __launch_bounds__(256) void k_bc_flux(DevMesh m, const double* __rest
 // The split flux is evaluated in contravariant form: with m = (Ja_i + Ja_l)/2 and the sums
 // rho_s, v_s, p_s, H_s of the two states, F = (rho_s m.v_s/2, rho_s m.v_s v_s/4 + p_s m,
 // rho_s m.v_s H_s/4), algebraically identical to the reference's m.(f,g,h).
+//
+// The face points' fluxes are loaded once, by the lanes of these points, during the volume integral, and
+// shared through LDS. An LSERK stage then prolongs its new state to the faces for the next stage. Gauss, N=3,
+// 20^3, FP32-bulk: 38 -> 45 us with the prolongation, whose own kernel took 17.
 template <int N, bool GL, bool SPLIT, class RF>
 __global__ __launch_bounds__(Dim<N>::NT) void k_volint(const double* __restrict__ U, DevMesh m,
                                                      const RF* __restrict__ G, const double* __restrict__ Flux,
                                                      const double* __restrict__ FluxS, Gas gas,
-                                                     double* __restrict__ Ut, RKStage st) {
+                                                     double* __restrict__ Ut, RKStage st, double* __restrict__ Um,
+                                                     double* __restrict__ Us) {
   constexpr int n = Dim<N>::n, nf = Dim<N>::nf, np = Dim<N>::np, NT = Dim<N>::NT;
   constexpr int NPRIM = SPLIT ? 6 : 5;   // split: rho,u,v,w,p,H ; weak: staging of f~ (5 comps)
   constexpr int NDIR = SPLIT ? 7 : 0;    // split: Ja^d (3) + viscous contravariant flux (4)
-  __shared__ double sA[(NPRIM + NDIR) * np > 5 * np ? (NPRIM + NDIR) * np : 5 * np];
+  // own face points' fluxes after the direction loop (5 rows of NF, working precision)
+  constexpr int NF = 6 * nf, RS = (NF + NT - 1) / NT;
+  constexpr int FACE = 5 * NF * (int)sizeof(RF) / 8, VOL = (NPRIM + NDIR) * np;
+  __shared__ double sA[VOL > FACE ? VOL : FACE];
   __shared__ double sB[3 * n * n + 4 * n];
   const BasisLayout B{n};
   const GasT<RF> g(gas);
   const int e = blockIdx.x;
   const int t = threadIdx.x;
   const double* Ue = U + (size_t)5 * np * e;
+  int sp[RS];
+#pragma unroll
+  for (int r = 0; r < RS; ++r) sp[r] = t + r * NT < NF ? side_point<N>(m, e, t + r * NT) : 0;
   stage_u_basis<N, NT>(Ue, sA, m.basis, sB, t);
   __syncthreads();
   const bool act = t < np;
@@ -429,6 +481,13 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_volint(const double* __restrict_
 #pragma unroll
     for (int v = 0; v < 5; ++v) Uown[v] = sA[5 * t + v];
     q = cons_to_prim(Uown, gas);
+  }
+  double ff[RS][5];  // the fluxes of the lane's face points, in flight during the volume integral
+#pragma unroll
+  for (int r = 0; r < RS; ++r) {
+    const double* F = sp[r] >= 0 ? Flux + 5 * (size_t)sp[r] : (FluxS ? FluxS : Flux) + 5 * (size_t)~sp[r];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) ff[r][v] = F[v];
   }
   // viscous Cartesian fluxes at the own node (EvalDiffFlux3D_Point)
   RF fvx[4] = {0, 0, 0, 0}, fvy[4] = {0, 0, 0, 0}, fvz[4] = {0, 0, 0, 0};
@@ -507,6 +566,7 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_volint(const double* __restrict_
   } else {
     // weak form: per direction stage the contravariant flux Ja^d.(f_euler + f_visc) (5 comps)
     const double* DH = sB + B.D_Hat_T();
+    RF* sC = reinterpret_cast<RF*>(sA);
     RF fe[5], ge[5], he[5];
     if (act) {
       const RF Ep = (RF)(Uown[4] + q.p);
@@ -527,7 +587,7 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_volint(const double* __restrict_
       if (act) {
         const RF* Jd = Ja + 3 * d;
 #pragma unroll
-        for (int v = 0; v < 5; ++v) sA[v * np + t] = (double)(fe[v] * Jd[0] + ge[v] * Jd[1] + he[v] * Jd[2]);
+        for (int v = 0; v < 5; ++v) sC[v * np + t] = fe[v] * Jd[0] + ge[v] * Jd[1] + he[v] * Jd[2];
       }
       __syncthreads();
       if (act) {
@@ -539,29 +599,31 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_volint(const double* __restrict_
           const RF dh = (RF)DH[l + n * me];
           const int id = base + l * stride;
 #pragma unroll
-          for (int v = 0; v < 5; ++v) acc[v] = acc[v] + dh * (RF)sA[v * np + id];
+          for (int v = 0; v < 5; ++v) acc[v] = acc[v] + dh * sC[v * np + id];
         }
       }
       __syncthreads();
     }
   }
-  if (!act) return;  // no barrier follows
   // surface integral: master sides +Flux, slave sides -Flux (surfint.t90:21-239, 471-616)
-#pragma unroll 1
+  RF* sS = reinterpret_cast<RF*>(sA);
+#pragma unroll
+  for (int r = 0; r < RS; ++r)
+#pragma unroll
+    for (int v = 0; v < 5; ++v)
+      if (t + r * NT < NF) sS[v * NF + t + r * NT] = sp[r] >= 0 ? (RF)ff[r][v] : -(RF)ff[r][v];
+  __syncthreads();
+  if (st.mode == 0 && !act) return;  // no barrier follows
+#pragma unroll
   for (int ls = 1; ls <= 6; ++ls) {
     int a, b, l;
     face_coords(ls, i, j, k, a, b, l);
     if (GL && l != (is_minus(ls) ? 0 : N)) continue;
-    const int side = m.E2S[2 * (ls - 1) + 12 * e] - 1;
-    const int flip = m.E2S[2 * (ls - 1) + 1 + 12 * e];
-    const int* pq2 = m.v2s2 + 2 * ((a + n * b) + nf * (flip + 5 * (ls - 1)));
-    const size_t fp = (size_t)(pq2[0] + n * pq2[1]) + (size_t)nf * side;
-    const double lh = GL ? (is_minus(ls) ? sB[B.L_HatMinus()] : sB[B.L_HatPlus() + N])
-                         : (is_minus(ls) ? sB[B.L_HatMinus() + l] : sB[B.L_HatPlus() + l]);
-    const RF sl = (RF)(flip == 0 ? lh : -lh);
-    const double* Fs = (flip != 0 && FluxS) ? FluxS : Flux;
+    const RF sl = (RF)(GL ? (is_minus(ls) ? sB[B.L_HatMinus()] : sB[B.L_HatPlus() + N])
+                          : (is_minus(ls) ? sB[B.L_HatMinus() + l] : sB[B.L_HatPlus() + l]));
+    const RF* f = sS + (ls - 1) * nf + a + n * b;
 #pragma unroll
-    for (int v = 0; v < 5; ++v) acc[v] = acc[v] + (RF)Fs[5 * fp + v] * sl;
+    for (int v = 0; v < 5; ++v) acc[v] = acc[v] + f[v * NF] * sl;
   }
   const double sj = m.sJ[gid];
   double ut[5];
@@ -571,15 +633,23 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_volint(const double* __restrict_
   if (st.mode == 0) {
 #pragma unroll
     for (int v = 0; v < 5; ++v) Ut[o + v] = ut[v];
-  } else {
-    // VCopy / VAXPBY of TimeStepByLSERKW2 (vector.f90:74-125)
+    return;
+  }
+  // VCopy / VAXPBY of TimeStepByLSERKW2 (vector.f90:74-125), and the new state's face values for the next stage
+  // (a pass of its own over U otherwise: 20^3, N=3 Gauss, FP32-bulk: 16 us a stage)
+  __syncthreads();
+  if (act) {
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
       const double r = (st.mode == 1) ? ut[v] : st.R[o + v] * st.minusA + ut[v];
+      const double un = Uown[v] + r * st.b_dt;
       st.R[o + v] = r;
-      st.U[o + v] = Uown[v] + r * st.b_dt;
+      st.U[o + v] = un;
+      sA[5 * t + v] = un;
     }
   }
+  __syncthreads();
+  prolong_faces<N, GL>(sA, sB, sp, Um, Us, t);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -776,10 +846,11 @@ struct TimedScope {
 
 template <int N, bool GL, class RF>
 static hipError_t rhs_n(const DevMesh& m, const DevWork& w, const Gas& gas, int split, int riemann,
-                        const double* U, double* Ut, const RKStage& st, hipStream_t s, KernelTimer* tm) {
+                        const double* U, double* Ut, const RKStage& st, bool faces_fresh, hipStream_t s,
+                        KernelTimer* tm) {
   const int K = m.nElems;
   constexpr int NT = Dim<N>::NT;
-  {
+  if (!faces_fresh) {
     TimedScope ts(tm, K_PROLONG, s);
     hipLaunchKernelGGL((k_prolong_u<N, GL>), dim3(K), dim3(NT), 0, s, U, m, w.Uf_m, w.Uf_s);
   }
@@ -810,39 +881,39 @@ static hipError_t rhs_n(const DevMesh& m, const DevWork& w, const Gas& gas, int 
     TimedScope ts(tm, K_VOLINT, s);
     if (split)
       hipLaunchKernelGGL((k_volint<N, GL, true, RF>), dim3(K), dim3(NT), 0, s, U, m, (const RF*)w.G, w.Flux, w.FluxS,
-                         gas, Ut, st);
+                         gas, Ut, st, w.Uf_m, w.Uf_s);
     else
       hipLaunchKernelGGL((k_volint<N, GL, false, RF>), dim3(K), dim3(NT), 0, s, U, m, (const RF*)w.G, w.Flux,
-                         w.FluxS, gas, Ut, st);
+                         w.FluxS, gas, Ut, st, w.Uf_m, w.Uf_s);
   }
   return hipGetLastError();
 }
 
 template <int N>
 static hipError_t rhs_dispatch(const DevMesh& m, const DevWork& w, const Gas& gas, int nodeType, int split,
-                               int riemann, int fp32, const double* U, double* Ut, const RKStage& st, hipStream_t s,
-                               KernelTimer* tm) {
+                               int riemann, int fp32, const double* U, double* Ut, const RKStage& st,
+                               bool faces_fresh, hipStream_t s, KernelTimer* tm) {
   if (nodeType == 2) {
-    if (fp32) return rhs_n<N, true, float>(m, w, gas, split, riemann, U, Ut, st, s, tm);
-    return rhs_n<N, true, double>(m, w, gas, split, riemann, U, Ut, st, s, tm);
+    if (fp32) return rhs_n<N, true, float>(m, w, gas, split, riemann, U, Ut, st, faces_fresh, s, tm);
+    return rhs_n<N, true, double>(m, w, gas, split, riemann, U, Ut, st, faces_fresh, s, tm);
   }
   if (split) return hipErrorInvalidValue;  // Gauss split form (entropy variables) is not built
-  if (fp32) return rhs_n<N, false, float>(m, w, gas, split, riemann, U, Ut, st, s, tm);
-  return rhs_n<N, false, double>(m, w, gas, split, riemann, U, Ut, st, s, tm);
+  if (fp32) return rhs_n<N, false, float>(m, w, gas, split, riemann, U, Ut, st, faces_fresh, s, tm);
+  return rhs_n<N, false, double>(m, w, gas, split, riemann, U, Ut, st, faces_fresh, s, tm);
 }
 
 bool supported_degree(int N) { return N >= 1 && N <= 7; }
 
 hipError_t launch_rhs(const DevMesh& m, const DevWork& w, const Gas& gas, int nodeType, int split, int riemann,
-                      int fp32, const double* U, double* Ut, const RKStage& st, hipStream_t s, KernelTimer* tm) {
+                      int fp32, const double* U, double* Ut, const RKStage& st, bool faces_fresh, hipStream_t s, KernelTimer* tm) {
   switch (m.N) {
-    case 1: return rhs_dispatch<1>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, s, tm);
-    case 2: return rhs_dispatch<2>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, s, tm);
-    case 3: return rhs_dispatch<3>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, s, tm);
-    case 4: return rhs_dispatch<4>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, s, tm);
-    case 5: return rhs_dispatch<5>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, s, tm);
-    case 6: return rhs_dispatch<6>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, s, tm);
-    case 7: return rhs_dispatch<7>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, s, tm);
+    case 1: return rhs_dispatch<1>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, faces_fresh, s, tm);
+    case 2: return rhs_dispatch<2>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, faces_fresh, s, tm);
+    case 3: return rhs_dispatch<3>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, faces_fresh, s, tm);
+    case 4: return rhs_dispatch<4>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, faces_fresh, s, tm);
+    case 5: return rhs_dispatch<5>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, faces_fresh, s, tm);
+    case 6: return rhs_dispatch<6>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, faces_fresh, s, tm);
+    case 7: return rhs_dispatch<7>(m, w, gas, nodeType, split, riemann, fp32, U, Ut, st, faces_fresh, s, tm);
     default: return hipErrorInvalidValue;
   }
 }
