@@ -340,7 +340,7 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
   if (alloc_owned(c, &c->w.Uf_m, 5 * face) || alloc_owned(c, &c->w.Uf_s, 5 * face) ||
       alloc_owned(c, &G, 12 * vol * gsz) || alloc_owned(c, &Gm, 12 * face * gsz) || alloc_owned(c, &Gs, 12 * face * gsz) ||
       alloc_owned(c, &c->w.Flux, 5 * face) || alloc_owned(c, &c->w.dtElem, 2 * (size_t)K) ||
-      alloc_owned(c, &c->w.errElem, (size_t)K) || alloc_owned(c, &c->w.dtOut, 2) || alloc_owned(c, &c->w.errOut, 1) ||
+      alloc_owned(c, &c->w.errElem, (size_t)K) ||
       alloc_owned(c, &c->w.bcLift, 4 * (size_t)c->nf * nBC))
     return 1;
   c->w.G = G; c->w.Gf_m = Gm; c->w.Gf_s = Gs;
@@ -354,7 +354,8 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
             !(pipe && std::strcmp(pipe, "classic") == 0);
   if (c->weak) {
     double* FG;
-    if (alloc_owned(c, &c->fw.FU[0], 10 * face) || alloc_owned(c, &c->fw.FU[1], 10 * face) || alloc_owned(c, &FG, 8 * face))
+    if (alloc_owned(c, &c->fw.FU[0], 10 * face) || alloc_owned(c, &c->fw.FU[1], 10 * face) || alloc_owned(c, &FG, 8 * face) ||
+        alloc_owned(c, &c->lamSum, 2 * (size_t)K) || alloc_owned(c, &c->lamNan, (size_t)K))
       return 1;
     c->fw.FG = FG;
   }
@@ -372,6 +373,8 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
   }
   HIPCHECK(hipHostMalloc((void**)&c->dtHost, 2 * sizeof(double), hipHostMallocDefault));
   HIPCHECK(hipHostMalloc((void**)&c->errHost, sizeof(int), hipHostMallocDefault));
+  c->w.dtOut = c->dtHost;
+  c->w.errOut = c->errHost;
   c->m = fxg::DevMesh{c->N, K, S, c->E2S, c->s2v2, c->v2s2, c->Mf, c->Mg, c->Mh, c->sJ,
                       c->NV, c->T1, c->T2, c->SE, c->basis, 0};
   return 0;
@@ -396,7 +399,7 @@ int finish_setup(fxg_ctx* c) {
       double* aff = nullptr;
       bool all = false;
       if (alloc_owned(c, &aff, (size_t)10 * c->K)) return 1;
-      HIPCHECK(fxg::find_const_metrics(c->m, aff, c->w.errOut, all, c->stream));
+      HIPCHECK(fxg::find_const_metrics(c->m, aff, c->w.errElem, all, c->stream));
       c->m.aff = all ? aff : nullptr;
     }
     if (c->fused && !c->m.aff) {  // the boundary nodes' metric terms, packed for the viscous face kernel
@@ -457,7 +460,7 @@ int rhs(fxg_ctx* c, const double* U, double* Ut, const fxg::RKStage& st, hipStre
 
 // One TimeStepByLSERKW2 step. `faces_known`: the face arrays already hold the face values of U (the
 // previous step of the same call, or of the context's own state), so the first stage reuses them.
-// `want_lambda`: the fused last stage also stores CALCTIMESTEP's per-element spectral radii of the
+// `want_lambda`: the last stage of the fused path and of the weak form's line kernels also stores CALCTIMESTEP's per-element spectral radii of the
 // new state (used by the next fxg_calc_timestep on the context's state).
 int lserk(fxg_ctx* c, double dt, int nStages, const double* RKA, const double* RKb, double* U, double* R,
           hipStream_t s, bool faces_known = false, bool want_lambda = false) {
@@ -465,7 +468,7 @@ int lserk(fxg_ctx* c, double dt, int nStages, const double* RKA, const double* R
   if (!RKb || (nStages > 1 && !RKA)) return fail("RK coefficient arrays are NULL");
   for (int st = 0; st < nStages; ++st) {
     fxg::RKStage stage{st == 0 ? 1 : 2, st == 0 ? 0.0 : -RKA[st - 1], RKb[st] * dt, U, R};
-    if (want_lambda && c->fused && st == nStages - 1) {
+    if (want_lambda && (c->fused || c->weak) && st == nStages - 1) {
       stage.lamSum = c->lamSum;
       stage.lamNan = c->lamNan;
     }
@@ -836,7 +839,7 @@ int fxg_timestep_lserkw2(fxg_ctx* c, double t, double dt, int nStages, const dou
   // Ut of the last stage is not kept by either pipeline, the gradients not by the fused one
   c->rhs_stale = true;
   c->last_rhs = 2;
-  if (c->fused) c->lam_of = c->U;
+  if (c->fused || c->weak) c->lam_of = c->U;
   c->last_b_dt = RKb[nStages - 1] * dt;
   HIPCHECK(hipStreamSynchronize(c->stream));
   return 0;
@@ -1072,12 +1075,11 @@ int fxg_adjoint_n_steps(fxg_ctx* c, int nSteps, const double* dt, int nStages, c
 
 int fxg_calc_timestep(fxg_ctx* c, double CFL, double DFL, double* dt, int* errType, double* dtElem) {
   if (!c || !dt || !errType) return fail("NULL argument");
-  if (c->fused && c->lam_of == c->U)
-    HIPCHECK(fxg::launch_calc_timestep_from_sums(c->m, c->w, c->lamSum, c->lamNan, CFL, DFL, c->stream, c->timer));
+  if (c->lam_of == c->U)
+    HIPCHECK(fxg::launch_calc_timestep_from_sums(c->m, c->w, c->lamSum, c->lamNan, CFL, DFL, dtElem != nullptr, c->stream,
+                                                     c->timer));
   else
     HIPCHECK(fxg::launch_calc_timestep(c->m, c->w, c->gas, c->U, CFL, DFL, c->stream, c->timer));
-  HIPCHECK(hipMemcpyAsync(c->dtHost, c->w.dtOut, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(hipMemcpyAsync(c->errHost, c->w.errOut, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   if (dtElem) {
     // dtElem = MIN(convective, viscous) per element, as CALCTIMESTEP stores it
     std::vector<double> tmp(2 * (size_t)c->K);

@@ -74,8 +74,8 @@ struct DevWork {
   double* bcLift;  // lifting flux of the boundary sides before SurfElem, (4,0:N,0:N,nBC)
   double* dtElem;  // (nElems)
   int* errElem;    // (nElems)
-  double* dtOut;   // [2]: convective and viscous minima
-  int* errOut;     // [1]
+  double* dtOut;   // [2]: convective and viscous minima (of a context: pinned host memory)
+  int* errOut;     // [1], likewise
 };
 
 struct RKStage {
@@ -200,9 +200,9 @@ hipError_t launch_axpy(size_t n, double a, const double* x, double* y, hipStream
 
 hipError_t launch_calc_timestep(const DevMesh& m, const DevWork& w, const Gas& gas, const double* U,
                                 double CFL, double DFL, hipStream_t s, KernelTimer* timer);
-// CALCTIMESTEP from the spectral-radius sums a fused last stage stored for the current state.
+// CALCTIMESTEP from the spectral-radius sums a last stage stored for the current state; `elements`: w.dtElem too.
 hipError_t launch_calc_timestep_from_sums(const DevMesh& m, const DevWork& w, const double* lamSum, const int* lamNan,
-                                          double CFL, double DFL, hipStream_t s, KernelTimer* timer);
+                                          double CFL, double DFL, bool elements, hipStream_t s, KernelTimer* timer);
 // Copies a (12, np, nElems) gradient array of type float/double into three FLEXI-layout
 // FP64 arrays (4,0:N,0:N,0:N,nElems).
 hipError_t launch_unpack_gradients(const DevMesh& m, const void* G, int fp32, double* gx, double* gy,

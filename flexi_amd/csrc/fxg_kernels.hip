@@ -655,6 +655,14 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_volint(const double* __restrict_
 // ---------------------------------------------------------------------------------------------
 // CALCTIMESTEP (calctimestep.f90:89-227): per element the maxima of the convective and viscous
 // eigenvalue sums, then dtElem; a second kernel reduces over elements.
+// The convective and viscous step of an element from its eigenvalue sums, and its error code.
+__device__ __forceinline__ int dt_of_sums(double conv, double visc, bool nan_rho, double CFL, double DFL, double& dc,
+                                          double& dv) {
+  dc = CFL * 2. / conv;
+  dv = (visc > 0.0) ? DFL * 4. / visc : 1.79769313486231571e308;
+  return nan_rho ? 1 : (dc != dc ? 2 : (dv != dv ? 3 : 0));
+}
+
 template <int N>
 __global__ __launch_bounds__(Dim<N>::NT) void k_dt_elem(const double* __restrict__ U, DevMesh m, Gas gas, double CFL,
                                                       double DFL, double* __restrict__ dtConv,
@@ -673,46 +681,20 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_dt_elem(const double* __restrict
   int nanr = 0;
   block_lambda_max<NT>(lam, isnan_rho, red, nanflag, t, mx, nanr);
   if (t == 0) {
-    const double dc = CFL * 2. / (mx[0] + mx[1] + mx[2]);
-    const double sv = mx[3] + mx[4] + mx[5];
-    const double dv = (sv > 0.0) ? DFL * 4. / sv : 1.79769313486231571e308;
+    double dc, dv;
+    err[e] = dt_of_sums(mx[0] + mx[1] + mx[2], mx[3] + mx[4] + mx[5], nanr != 0, CFL, DFL, dc, dv);
     dtConv[e] = dc;
     dtVisc[e] = dv;
-    err[e] = nanr ? 1 : (dc != dc ? 2 : (dv != dv ? 3 : 0));
   }
 }
 
-// Per-element steps from the spectral-radius sums the fused last LSERK stage stored
-// (lamSum[2e]: convective, lamSum[2e+1]: viscous), as k_dt_elem finishes them.
-__global__ __launch_bounds__(256) void k_dt_finish(const double* __restrict__ lamSum, const int* __restrict__ lamNan,
-                                                 int K, double CFL, double DFL, double* __restrict__ dtConv,
-                                                 double* __restrict__ dtVisc, int* __restrict__ err) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= K) return;
-  const double dc = CFL * 2. / lamSum[2 * e];
-  const double sv = lamSum[2 * e + 1];
-  const double dv = (sv > 0.0) ? DFL * 4. / sv : 1.79769313486231571e308;
-  dtConv[e] = dc;
-  dtVisc[e] = dv;
-  err[e] = lamNan[e] ? 1 : (dc != dc ? 2 : (dv != dv ? 3 : 0));
-}
-
-// Minimum over elements of the convective and viscous steps and the error code.
-__global__ __launch_bounds__(1024) void k_dt_reduce(const double* __restrict__ dtConv, const double* __restrict__ dtVisc,
-                                                  const int* __restrict__ err, int K, double* __restrict__ out,
-                                                  int* __restrict__ errOut) {
+// Minimum over the workgroup's lanes of the convective and viscous steps and the error code (priority to the
+// root cause: 1 (NaN density) over 2 (convective) over 3 (viscous)); lane 0 stores them. The context's own
+// calls have them stored in pinned host memory, which saves two copies of a few bytes.
+__device__ __forceinline__ void dt_min(double c, double v, int ec, double* __restrict__ out, int* __restrict__ errOut) {
   __shared__ double sc[16], sv[16];
   __shared__ int se[16];
   const int t = threadIdx.x;
-  double c = 1.79769313486231571e308, v = 1.79769313486231571e308;
-  int ec = 0;
-  for (int x = t; x < K; x += 1024) {
-    c = fmin(c, dtConv[x]);
-    v = fmin(v, dtVisc[x]);
-    const int ex = err[x];
-    // priority to the root cause: 1 (NaN density) over 2 (convective) over 3 (viscous)
-    if (ex != 0 && (ec == 0 || ex < ec)) ec = ex;
-  }
   for (int off = 32; off > 0; off >>= 1) {
     c = fmin(c, __shfl_down(c, off, 64));
     v = fmin(v, __shfl_down(v, off, 64));
@@ -731,6 +713,41 @@ __global__ __launch_bounds__(1024) void k_dt_reduce(const double* __restrict__ d
     out[1] = v;
     errOut[0] = ec;
   }
+}
+
+// Time step from the spectral-radius sums a last LSERK stage stored (lamSum[2e]: convective, lamSum[2e+1]:
+// viscous); with dtConv also the elements' own steps.
+__global__ __launch_bounds__(1024) void k_dt_sums(const double* __restrict__ lamSum, const int* __restrict__ lamNan, int K,
+                                                double CFL, double DFL, double* __restrict__ dtConv,
+                                                double* __restrict__ dtVisc, double* __restrict__ out,
+                                                int* __restrict__ errOut) {
+  double c = 1.79769313486231571e308, v = 1.79769313486231571e308;
+  int ec = 0;
+#pragma unroll 4
+  for (int x = threadIdx.x; x < K; x += 1024) {
+    double dc, dv;
+    const int ex = dt_of_sums(lamSum[2 * x], lamSum[2 * x + 1], lamNan[x] != 0, CFL, DFL, dc, dv);
+    if (dtConv) { dtConv[x] = dc; dtVisc[x] = dv; }
+    c = fmin(c, dc);
+    v = fmin(v, dv);
+    if (ex != 0 && (ec == 0 || ex < ec)) ec = ex;
+  }
+  dt_min(c, v, ec, out, errOut);
+}
+
+// The same from the elements' steps.
+__global__ __launch_bounds__(1024) void k_dt_reduce(const double* __restrict__ dtConv, const double* __restrict__ dtVisc,
+                                                  const int* __restrict__ err, int K, double* __restrict__ out,
+                                                  int* __restrict__ errOut) {
+  double c = 1.79769313486231571e308, v = 1.79769313486231571e308;
+  int ec = 0;
+  for (int x = threadIdx.x; x < K; x += 1024) {
+    c = fmin(c, dtConv[x]);
+    v = fmin(v, dtVisc[x]);
+    const int ex = err[x];
+    if (ex != 0 && (ec == 0 || ex < ec)) ec = ex;
+  }
+  dt_min(c, v, ec, out, errOut);
 }
 
 template <class RF>
@@ -937,19 +954,12 @@ static hipError_t dt_n(const DevMesh& m, const DevWork& w, const Gas& gas, const
 }
 
 hipError_t launch_calc_timestep_from_sums(const DevMesh& m, const DevWork& w, const double* lamSum, const int* lamNan,
-                                          double CFL, double DFL, hipStream_t s, KernelTimer* tm) {
+                                          double CFL, double DFL, bool elements, hipStream_t s, KernelTimer* tm) {
   const int K = m.nElems;
-  double* dtConv = w.dtElem;
-  double* dtVisc = w.dtElem + K;
-  {
-    TimedScope ts(tm, K_DT_ELEM, s);
-    hipLaunchKernelGGL(k_dt_finish, dim3((K + 255) / 256), dim3(256), 0, s, lamSum, lamNan, K, CFL, DFL, dtConv, dtVisc,
-                       w.errElem);
-  }
-  {
-    TimedScope ts(tm, K_DT_REDUCE, s);
-    hipLaunchKernelGGL(k_dt_reduce, dim3(1), dim3(1024), 0, s, dtConv, dtVisc, w.errElem, K, w.dtOut, w.errOut);
-  }
+  double* dtConv = elements ? w.dtElem : nullptr;
+  TimedScope ts(tm, K_DT_REDUCE, s);
+  hipLaunchKernelGGL(k_dt_sums, dim3(1), dim3(1024), 0, s, lamSum, lamNan, K, CFL, DFL, dtConv, w.dtElem + K, w.dtOut,
+                     w.errOut);
   return hipGetLastError();
 }
 

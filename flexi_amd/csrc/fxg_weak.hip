@@ -316,8 +316,9 @@ __global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(N == 7
   }
 }
 
-// Kernel B.
-template <int N, int SOLVER, bool GL, bool AFF>
+// Kernel B. LAM: the last stage of a step, which also forms CALCTIMESTEP's spectral radii of the new state (a kernel
+// of its own over U and the metric terms otherwise, 8 us of a step's 90 at 8^3, N=3).
+template <int N, int SOLVER, bool GL, bool AFF, bool LAM>
 __global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(N == 7 ? 2 : 3))) void k_weak_stage(
     const double* U, DevMesh m, const double* __restrict__ basis, const double* __restrict__ FU,
     double* __restrict__ FUnext, const double* __restrict__ FG, Gas gas, double* Ut, RKStage st,
@@ -495,6 +496,8 @@ __global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(N == 7
         sum[r][v0 + w] = s[0] + s[2 * RS] + s[4 * RS];
       }
   }
+  double lam[6] = {0, 0, 0, 0, 0, 0};
+  int nan_rho = 0;
   // Ut = -Ut*sJ, the register update, and the new state in rows 0..3 and 9 for its face values
 #pragma unroll
   for (int r = 0; r < RN; ++r) {
@@ -519,8 +522,29 @@ __global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(N == 7
       st.U[o + v] = c[r][v];
       sL[(v < 4 ? v : 9) * RS + place[r]] = c[r][v];
     }
+    if constexpr (LAM) {
+      double ln6[6];
+      int nr;
+      if constexpr (AFF) dt_node_lambda(c[r], gas, je[9], je, je + 3, je + 6, ln6, nr);
+      else dt_node_lambda(c[r], gas, sj[r], m.Mf + 3 * (e0 + nd), m.Mg + 3 * (e0 + nd), m.Mh + 3 * (e0 + nd), ln6, nr);
+      nan_rho |= nr;
+#pragma unroll
+      for (int x = 0; x < 6; ++x) lam[x] = (ln6[x] > lam[x] || ln6[x] != ln6[x]) ? ln6[x] : lam[x];
+    }
   }
   if (st.mode == 0) return;
+  if constexpr (LAM) {
+    __shared__ double red[6 * (NT / 64)];
+    __shared__ int flag[NT / 64];
+    double mx[6];
+    int nanr = 0;
+    block_lambda_max<NT>(lam, nan_rho, red, flag, threadIdx.x, mx, nanr);
+    if (threadIdx.x == 0) {
+      st.lamSum[2 * e] = mx[0] + mx[1] + mx[2];
+      st.lamSum[2 * e + 1] = mx[3] + mx[4] + mx[5];
+      st.lamNan[e] = nanr;
+    }
+  }
   __syncthreads();
   if (!line) return;
   lp.again();
@@ -571,10 +595,15 @@ hipError_t weak_n(const DevMesh& m, const FusedWork& w, const Gas& gas, int riem
   {
     Scope sc(tm, K_VOLINT, s);
 #define FXG_LAUNCH(SOLV)                                                                                               \
-  hipLaunchKernelGGL((k_weak_stage<N, SOLV, GL, AFF>), g, b, 0, s, U, m, m.basis, FU, w.FU[1 - cur], FG, gas, Ut, st, G)
-    if (riemann == 1) FXG_LAUNCH(1);
-    else if (riemann == 3) FXG_LAUNCH(3);
-    else FXG_LAUNCH(33);
+  if (st.lamSum)                                                                                                       \
+    hipLaunchKernelGGL((k_weak_stage<N, SOLV, GL, AFF, true>), g, b, 0, s, U, m, m.basis, FU, w.FU[1 - cur], FG, gas, \
+                       Ut, st, G);                                                                                     \
+  else                                                                                                                 \
+    hipLaunchKernelGGL((k_weak_stage<N, SOLV, GL, AFF, false>), g, b, 0, s, U, m, m.basis, FU, w.FU[1 - cur], FG, gas, \
+                       Ut, st, G)
+    if (riemann == 1) { FXG_LAUNCH(1); }
+    else if (riemann == 3) { FXG_LAUNCH(3); }
+    else { FXG_LAUNCH(33); }
 #undef FXG_LAUNCH
   }
   return hipGetLastError();
