@@ -24,3 +24,29 @@ def test_vjp_is_the_transpose(N, riemann, curved):
         assert abs(np.sum(lam * jd) - np.sum(vjp(s, U, lam) * d)) <= 1e-7 * np.sum(np.abs(lam * jd))
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("N", [2, 5, 7])
+def test_runs_of_different_sizes_share_a_context(N):
+    """The workspace of an adjoint run stays with its context: runs that need less of it or more give, bit for
+    bit, what a context of their own gives."""
+    import torch
+
+    def grad(s, U, steps, every):
+        x = torch.from_numpy(np.ascontiguousarray(U.ravel(order="K"))).cuda()
+        ubar = torch.ones_like(x)
+        torch.cuda.synchronize()
+        s.adjoint_n_steps_dev(x.data_ptr(), ubar.data_ptr(), [1e-3] * steps, checkpoint_every=every)
+        return ubar.cpu().numpy()
+
+    _, s = make(N, "roe", shape=(2, 3, 2))
+    try:
+        U = perturbed_tgv(s, 1)
+        for steps, every in ((4, 2), (6, 6), (3, 1), (5, 3), (4, 2)):
+            _, own = make(N, "roe", shape=(2, 3, 2))
+            try:
+                assert np.array_equal(grad(s, U, steps, every), grad(own, U, steps, every))
+            finally:
+                own.close()
+    finally:
+        s.close()
