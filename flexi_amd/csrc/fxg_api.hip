@@ -659,6 +659,7 @@ int fxg_set_boundaries(fxg_ctx* c, int nBCs, const int* BC, const int* BoundaryT
                        const double* RefStatePrim) {
   if (!c) return fail("ctx is NULL");
   if (c->nBC == 0) return 0;
+  c->faces_of = nullptr;  // the kept boundary states follow the conditions
   if (!BC || !BoundaryType || nBCs < 1) return fail("BC and BoundaryType are required for a mesh with boundary sides");
   if (nRefState < 0 || (nRefState > 0 && !RefStatePrim)) return fail("RefStatePrim is NULL");
   std::vector<int> info(2 * (size_t)c->nBC);
@@ -713,6 +714,7 @@ int fxg_set_boundary_data(fxg_ctx* c, const double* BCDataPrim) {
   if (!c) return fail("ctx is NULL");
   if (c->nBC == 0) return 0;
   if (!BCDataPrim) return fail("BCDataPrim is NULL");
+  c->faces_of = nullptr;  // the kept boundary states follow the conditions
   const size_t n = 6 * (size_t)c->nf * c->nBC;
   for (size_t x = 0; x < n; x += 6)
     if (!(BCDataPrim[x] > 0.0) || !(BCDataPrim[x + 4] > 0.0) || !(BCDataPrim[x + 5] > 0.0))

@@ -397,6 +397,7 @@ hipError_t fused_n(const DevMesh& m, const FusedWork& w, const Gas& gas, int rie
   const int K = m.nElems;
   constexpr int NT = D<N>::NT;
   const bool bc = m.nBC > 0;
+  const bool ghosts = bc && (sizeof(RF) == 4 || !faces_fresh);  // (FP64 stages leave them with the face states)
   if (!faces_fresh && (bc || !m.nbNode)) {
     Scope sc(tm, K_FACES, s);
     hipLaunchKernelGGL((k_faces_of<N>), dim3(K), dim3(NT), 0, s, U, m, w.FU[cur]);
@@ -404,7 +405,7 @@ hipError_t fused_n(const DevMesh& m, const FusedWork& w, const Gas& gas, int rie
   }
   {
     Scope sc(tm, K_VISC_FACES, s);
-    if (bc) {
+    if (ghosts) {
       const hipError_t err = launch_bc_ghost(m, w.FU[cur], w.bcP, gas, s);
       if (err != hipSuccess) return err;
     }

@@ -4,7 +4,7 @@
 // LSERK register update, the new state's face values and, in the last stage of a step, CALCTIMESTEP's
 // spectral radii. The face arrays and the conventions at a face are those described in fxg_fused.hip,
 // which holds the FP32-bulk form of this kernel.
-#include "fxg_bc.h"
+#include "fxg_bcface.h"
 #include "fxg_line.h"
 
 namespace fxg {
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(S<N>::NT)
 __attribute__((amdgpu_waves_per_eu(AFF || N <= 5 ? 3 : 2))) void k_stage(const double* U, DevMesh m, const double* __restrict__ basis, const double* __restrict__ FU,
                                                 double* __restrict__ FUnext, const double* __restrict__ FG, Gas gas,
                                                 double* Ut, RKStage st, double* __restrict__ Gout,
-                                                const double* __restrict__ bcP) {
+                                                double* __restrict__ bcP) {
   constexpr int n = S<N>::n, nf = S<N>::nf, np = S<N>::np, NL = S<N>::NL, NT = S<N>::NT, RN = S<N>::RN, RS = S<N>::RS;
   using L = Lds<N, AFF>;
   __shared__ double sL[L::SIZE];
@@ -482,10 +482,18 @@ __attribute__((amdgpu_waves_per_eu(AFF || N <= 5 ? 3 : 2))) void k_stage(const d
   if (line) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      double* dst = FUnext + 5 * (size_t)m.slotTab[(size_t)6 * nf * e + ((s ? lsp : lsm) - 1) * nf + ln];
+      const unsigned own = m.slotTab[(size_t)6 * nf * e + ((s ? lsp : lsm) - 1) * nf + ln];
+      double* dst = FUnext + 5 * (size_t)own;
       const double* src = lp.at(sL, s ? N : 0);
+      double u[5];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) dst[v] = src[v * RS];
+      for (int v = 0; v < 5; ++v) dst[v] = u[v] = src[v * RS];
+      if constexpr (BC) {
+        // a boundary side: its outer slot of the next stage too (a kernel of its own otherwise). bcP of this
+        // point was last read above, by this lane
+        const int side = (int)(own / (2u * (unsigned)nf));
+        if (side < m.nBC) bc_ghost_point(m, u, dst + 5 * nf, bcP, gas, slot_side_point<N>(own), side);
+      }
     }
   }
 }

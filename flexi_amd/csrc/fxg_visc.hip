@@ -3,7 +3,7 @@
 // normal flux f_v . (n SurfElem) seen from that element (4 values per face point, momentum and
 // energy) into the side array FG (lifting_br1.t90:48-181, flux.f90:149-241). A translation unit
 // of its own, so that its code does not change the register allocation of k_dg_fused.
-#include "fxg_bc.h"
+#include "fxg_bcface.h"
 #include "fxg_line.h"
 
 namespace fxg {
@@ -131,7 +131,8 @@ __attribute__((amdgpu_waves_per_eu(N == 7 ? 8 : 6))) void k_visc_faces(
 template <int N, bool BC, bool AFF, bool FIRST>
 __global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(3))) void k_visc_lines(
     const double* __restrict__ U, DevMesh m, const double* __restrict__ basis, const double* __restrict__ Jsoa,
-    double* __restrict__ FU, double* __restrict__ FG, Gas gas, double* __restrict__ gBC) {
+    double* __restrict__ FU, double* __restrict__ FG, Gas gas, double* __restrict__ gBC,
+    const double* __restrict__ bcP) {
   constexpr int n = S<N>::n, nf = S<N>::nf, np = S<N>::np, NL = S<N>::NL, NT = S<N>::NT, RN = S<N>::RN, RS = S<N>::RS;
   constexpr int X = 4, NF = 6 * nf;
   __shared__ double sL[10 * RS];
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(3))) v
       for (int v = 0; v < 4; ++v)
         p[4 * x + v] = (Ja[x] * g[r][v] + Ja[3 + x] * g[r][4 + v] + Ja[6 + x] * g[r][8 + v]) * sj;
     if constexpr (BC) {
-      // boundary sides: keep the gradients at their face points for k_bc_visc
+      // boundary sides: the gradients at their face points, for the ends of the lines below
       if (t + r * NT < np) {
         const int i = nd % n, j = (nd / n) % n, k = nd / nf, sides = node_sides<N>(i, j, k);
 #pragma unroll 1
@@ -308,101 +309,46 @@ __global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(3))) v
     FG[4 * (size_t)own0 + v] = f[0][v];
     FG[4 * (size_t)own1 + v] = f[1][v];
   }
+  if constexpr (BC) {
+    // the outer slots of boundary sides (a kernel of its own over the boundary points otherwise); the gradients
+    // were stored by this workgroup, before the barriers above
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const unsigned own = s ? own1 : own0;
+      const int side = (int)(own / (2u * (unsigned)nf));
+      if (side >= m.nBC) continue;
+      const size_t fp = slot_side_point<N>(own);
+      double q[12];
+#pragma unroll
+      for (int x = 0; x < 12; ++x) q[x] = gBC[12 * fp + x];
+      bc_visc_point<double>(m, FU + 5 * (size_t)own, q, f[s], FG + 4 * ((size_t)own + nf), bcP, gas, fp, side);
+    }
+  }
 }
 
-// One lane per boundary side point, after k_visc_faces: the outer slot's viscous flux, so that with
-// the inner element's half it makes the boundary's viscous flux (getboundaryflux.f90:561-776):
-// Riemann type 0.5 (f_in + f_b).n with the boundary state's velocity, walls f_wall.n with the
-// wall's velocity (none, or the tangential part at a slip wall) and the inner gradients (slip walls:
-// as slip_wall_gradients leaves them; no heat flux at an adiabatic wall). n SurfElem is the side's.
-template <class RF>
-__global__ __launch_bounds__(256) void k_bc_visc(DevMesh m, const double* __restrict__ FU, const RF* __restrict__ gBC,
-                                               RF* __restrict__ FG, const double* __restrict__ bcP, Gas gas, int nf,
+// FP32-bulk: one lane per boundary side point, after k_visc_faces (k_visc_lines forms these fluxes itself).
+__global__ __launch_bounds__(256) void k_bc_visc(DevMesh m, const double* __restrict__ FU, const float* __restrict__ gBC,
+                                               float* __restrict__ FG, const double* __restrict__ bcP, Gas gas, int nf,
                                                int nPts) {
   const int fp = blockIdx.x * blockDim.x + threadIdx.x;
   if (fp >= nPts) return;
   const int side = fp / nf, pq = fp - side * nf;
   const size_t in = ((size_t)side * 2) * nf + pq, out = in + nf;
-  const int type = m.bcInfo[2 * side];
-  const GasT<RF> gt(gas);
-  const RF se = (RF)m.SurfElem[fp];
-  const RF nh[3] = {(RF)m.NormVec[3 * (size_t)fp], (RF)m.NormVec[3 * (size_t)fp + 1], (RF)m.NormVec[3 * (size_t)fp + 2]};
-  RF q[12];
+  float q[12];
 #pragma unroll
   for (int c = 0; c < 12; ++c) q[c] = gBC[12 * (size_t)fp + c];
-  RF ub[3] = {RF(0), RF(0), RF(0)};
-  const bool riemann = bc_riemann_type(type);
-  if (type == BC_DIRICHLET) {
-    const double* ref = m.refPrim + 6 * m.bcInfo[2 * side + 1];
-    ub[0] = (RF)ref[1]; ub[1] = (RF)ref[2]; ub[2] = (RF)ref[3];
-  } else if (riemann) {  // the boundary state's velocity, as k_bc_ghost formed it
-    ub[0] = (RF)bcP[4 * (size_t)fp + 1]; ub[1] = (RF)bcP[4 * (size_t)fp + 2]; ub[2] = (RF)bcP[4 * (size_t)fp + 3];
-  } else if (bc_slip_wall(type)) {
-    const Prim p = cons_to_prim(FU + 5 * in, gas);
-    const RF vn = (RF)p.u * nh[0] + (RF)p.v * nh[1] + (RF)p.w * nh[2];
-    ub[0] = (RF)p.u - vn * nh[0]; ub[1] = (RF)p.v - vn * nh[1]; ub[2] = (RF)p.w - vn * nh[2];
-    const RF t1[3] = {(RF)m.TangVec1[3 * (size_t)fp], (RF)m.TangVec1[3 * (size_t)fp + 1],
-                      (RF)m.TangVec1[3 * (size_t)fp + 2]};
-    const RF t2[3] = {(RF)m.TangVec2[3 * (size_t)fp], (RF)m.TangVec2[3 * (size_t)fp + 1],
-                      (RF)m.TangVec2[3 * (size_t)fp + 2]};
-    slip_wall_gradients<RF>(type, nh, t1, t2, q);
-  }
-  RF bx[4], by[4], bz[4];
-  diff_flux<RF>(gt, ub[0], ub[1], ub[2], q, q + 4, q + 8, bx, by, bz);
-  if (type == BC_WALL_ADIABATIC) bx[3] = by[3] = bz[3] = RF(0);
-  const RF* fi = FG + 4 * in;
-  RF* fo = FG + 4 * out;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const RF fb = (bx[c] * nh[0] + by[c] * nh[1] + bz[c] * nh[2]) * se;
-    fo[c] = riemann ? -fb : fi[c] - RF(2) * fb;
-  }
+  bc_visc_point<float>(m, FU + 5 * in, q, FG + 4 * in, FG + 4 * out, bcP, gas, fp, side);
 }
 
-// One lane per boundary side point: the outer slot of the boundary side, from the inner face
-// state and GetBoundaryState (getboundaryflux.f90:224-472). Riemann type: the boundary state itself
-// (the Riemann solver and the lifting then see it as FLEXI's boundary flux does); its velocity also
-// goes to bcP for k_bc_visc. Walls: a state whose lifting variables are 2 f - q_in, f the boundary
-// lifting value (Lifting_GetBoundaryFlux, :855-939), so that the BR1 difference (q_out - q_in)/2 is
-// FLEXI's f - q_in; their inviscid flux (0, p_wall n, 0) is formed by the stage kernel from bcP.
+// One lane per boundary side point: the outer slots from the inner face states (in FP64 a stage leaves those of its
+// new state, and this kernel serves the first stage of a state without face states).
 __global__ __launch_bounds__(256) void k_bc_ghost(DevMesh m, double* __restrict__ FU, double* __restrict__ bcP,
                                                 Gas gas, int nf, int nPts) {
   const int fp = blockIdx.x * blockDim.x + threadIdx.x;
   if (fp >= nPts) return;
   const int side = fp / nf, pq = fp - side * nf;
-  const size_t in = ((size_t)side * 2) * nf + pq, out = in + nf;
-  const Prim q = cons_to_prim(FU + 5 * in, gas);
-  const double Pm[6] = {q.rho, q.u, q.v, q.w, q.p, q.T};
-  double nv[3], t1[3], t2[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    nv[c] = m.NormVec[3 * (size_t)fp + c];
-    t1[c] = m.TangVec1[3 * (size_t)fp + c];
-    t2[c] = m.TangVec2[3 * (size_t)fp + c];
-  }
-  const int type = m.bcInfo[2 * side], st = m.bcInfo[2 * side + 1];
-  double Pb[6];
-  boundary_state(gas, type, st >= 0 ? m.refPrim + 6 * st : nullptr, m.bcData ? m.bcData + 6 * (size_t)fp : nullptr,
-                 Pm, nv, t1, t2, Pb);
-  double G[6];
-  double* bp = bcP + 4 * (size_t)fp;
-  if (bc_riemann_type(type)) {
-#pragma unroll
-    for (int v = 0; v < 6; ++v) G[v] = Pb[v];
-    bp[0] = Pb[4]; bp[1] = Pb[1]; bp[2] = Pb[2]; bp[3] = Pb[3];
-  } else {
-    double F[4];
-    boundary_lifting_flux(type, Pm, Pb, F);
-    G[0] = Pm[0];
-    G[1] = Pm[1] + 2.0 * F[0]; G[2] = Pm[2] + 2.0 * F[1]; G[3] = Pm[3] + 2.0 * F[2];
-    G[5] = Pm[5] + 2.0 * F[3];
-    G[4] = G[0] * gas.R * G[5];
-    bp[0] = Pb[4];
-  }
-  double* o = FU + 5 * out;
-  o[0] = G[0];
-  o[1] = G[1] * G[0]; o[2] = G[2] * G[0]; o[3] = G[3] * G[0];
-  o[4] = gas.sKappaM1 * G[4] + 0.5 * (o[1] * G[1] + o[2] * G[2] + o[3] * G[3]);
+  const size_t in = ((size_t)side * 2) * nf + pq;
+  bc_ghost_point(m, FU + 5 * in, FU + 5 * (in + nf), bcP, gas, fp, side);
 }
 
 }  // namespace
@@ -426,7 +372,7 @@ hipError_t launch_visc_faces(const DevMesh& m, bool fp32, bool faces_fresh, cons
                          (const float*)Jsoa, FU, (float*)FG, gas, (float*)gBC);                                                  \
     else                                                                                                           \
       hipLaunchKernelGGL((k_visc_lines<NN, BC, AFF, FIRST>), dim3(m.nElems), dim3(S<NN>::NT), 0, s, U, m, m.basis, \
-                         (const double*)Jsoa, FU, (double*)FG, gas, (double*)gBC);                                                      \
+                         (const double*)Jsoa, FU, (double*)FG, gas, (double*)gBC, bcP);                                                      \
   } while (0)
 #define FXG_CASE(NN)                                                                                               \
   case NN:                                                                                                         \
@@ -439,14 +385,10 @@ hipError_t launch_visc_faces(const DevMesh& m, bool fp32, bool faces_fresh, cons
 #undef FXG_LAUNCH2
     default: return hipErrorInvalidValue;
   }
-  if (bc) {
+  if (bc && fp32) {
     const int nf = (m.N + 1) * (m.N + 1), nPts = m.nBC * nf;
-    if (fp32)
-      hipLaunchKernelGGL((k_bc_visc<float>), dim3((nPts + 255) / 256), dim3(256), 0, s, m, FU, (const float*)gBC,
-                         (float*)FG, bcP, gas, nf, nPts);
-    else
-      hipLaunchKernelGGL((k_bc_visc<double>), dim3((nPts + 255) / 256), dim3(256), 0, s, m, FU, (const double*)gBC,
-                         (double*)FG, bcP, gas, nf, nPts);
+    hipLaunchKernelGGL(k_bc_visc, dim3((nPts + 255) / 256), dim3(256), 0, s, m, FU, (const float*)gBC, (float*)FG, bcP,
+                       gas, nf, nPts);
   }
   return hipGetLastError();
 }
