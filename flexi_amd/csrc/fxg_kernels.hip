@@ -721,16 +721,32 @@ __global__ __launch_bounds__(1024) void k_dt_sums(const double* __restrict__ lam
                                                 double CFL, double DFL, double* __restrict__ dtConv,
                                                 double* __restrict__ dtVisc, double* __restrict__ out,
                                                 int* __restrict__ errOut) {
-  double c = 1.79769313486231571e308, v = 1.79769313486231571e308;
+  const double big = 1.79769313486231571e308;
+  double c = big, v = big;
   int ec = 0;
+  if (!dtConv && CFL > 0.0 && CFL <= big && DFL >= 0.0 && DFL <= big) {
+    // the smallest step is that of the largest sum (the quotient is monotonic, also as rounded): two divisions
+    // per lane instead of two per element (32768 elements: 28 -> 15 us)
+    double mc = -1.0, mv = -1.0;
 #pragma unroll 4
-  for (int x = threadIdx.x; x < K; x += 1024) {
-    double dc, dv;
-    const int ex = dt_of_sums(lamSum[2 * x], lamSum[2 * x + 1], lamNan[x] != 0, CFL, DFL, dc, dv);
-    if (dtConv) { dtConv[x] = dc; dtVisc[x] = dv; }
-    c = fmin(c, dc);
-    v = fmin(v, dv);
-    if (ex != 0 && (ec == 0 || ex < ec)) ec = ex;
+    for (int x = threadIdx.x; x < K; x += 1024) {
+      const double conv = lamSum[2 * x];
+      mc = fmax(mc, conv);
+      mv = fmax(mv, lamSum[2 * x + 1]);
+      const int ex = lamNan[x] ? 1 : (conv != conv ? 2 : 0);
+      if (ex != 0 && (ec == 0 || ex < ec)) ec = ex;
+    }
+    if (mc >= 0.0) c = fmin(c, CFL * 2. / mc);
+    if (mv > 0.0) v = fmin(v, DFL * 4. / mv);
+  } else {
+    for (int x = threadIdx.x; x < K; x += 1024) {
+      double dc, dv;
+      const int ex = dt_of_sums(lamSum[2 * x], lamSum[2 * x + 1], lamNan[x] != 0, CFL, DFL, dc, dv);
+      if (dtConv) { dtConv[x] = dc; dtVisc[x] = dv; }
+      c = fmin(c, dc);
+      v = fmin(v, dv);
+      if (ex != 0 && (ec == 0 || ex < ec)) ec = ex;
+    }
   }
   dt_min(c, v, ec, out, errOut);
 }
