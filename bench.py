@@ -32,27 +32,28 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0  # MI355X datasheet HBM3E bandwidth
 # Algorithmic HBM bytes per DOF of each kernel launch (FP64, N=7, Gauss-Lobatto: 512 volume
 # nodes, 296 boundary nodes and 6*64 own face points per element). Face values carry 40 B
-# (5 doubles), viscous face fluxes 32 B, metrics 80 B (Ja^1..3 + sJ).
+# (5 doubles), viscous face fluxes 32 B; the metric terms of a parallelepiped are ten values (80 B
+# per element).
 #   faces      : boundary U read 296*40 + own face states written 384*40       ->  53.1 B/DOF
-#   visc_faces : U 512*40 + boundary metrics 296*80 + neighbour face states 384*40
-#                + own viscous fluxes written 384*32                              -> 140.25 B/DOF
-#   dg_fused   : U 40 + metrics 80 + neighbour states 30 + neighbour fluxes 24 + U written 40
-#                + next face states 30 + register R read 40 (not in stage 1) + written 40
-#                (stage 5 also forms CALCTIMESTEP's spectral radii from the metric terms, no
-#                algorithmic bytes), averaged over the 5 stages: (284 + 4*324)/5  -> 316.0 B/DOF
-# The four-kernel path's figures follow the same counting.
+#   visc_faces : U 512*40 + neighbour face states 384*40 + own viscous fluxes written 384*32
+#                + metrics 80 per element                                       ->  94.2 B/DOF
+#   dg_fused   : U 40 + neighbour states 30 + neighbour fluxes 24 + U written 40 + next face
+#                states 30 + register R read 40 (not in stage 1) + written 40 + metrics 80 per
+#                element (stage 5 also forms CALCTIMESTEP's spectral radii, no algorithmic
+#                bytes), averaged over the 5 stages: (204 + 4*244)/5              -> 236.2 B/DOF
+# The four-kernel path's figures follow the same counting, with 80 B of metric terms per node.
 ALGO_BYTES_PER_DOF = {"prolong_u": 60.0, "lift": 372.0, "flux": 147.0, "volint": 366.0,
-                      "faces": 53.125, "visc_faces": 140.25, "dg_fused": 316.0}
-# Per DOF-stage byte model of the stage (U, Ut/R, metrics and gradient traffic of one stage)
-B_STAGE = 432.0
+                      "faces": 53.125, "visc_faces": 94.2, "dg_fused": 236.2}
+# Per DOF-stage byte model of the stage (U, Ut/R and gradient traffic of one stage)
+B_STAGE = 352.0
 # HBM bytes per DOF of one launch of the fused kernels at this workload (FP64, mean over the 5
 # stages of a step), from rocprofv3 FETCH_SIZE (x2.0, plain-copy calibration) + WRITE_SIZE runs of
 # this benchmark; the summary and the commands are in profiles/fused_stage_tgv32_n7_fp64.md
-MEASURED_BYTES_PER_DOF = {"dg_fused": 364.1, "visc_faces": 143.3, "faces": 64.0}
+MEASURED_BYTES_PER_DOF = {"dg_fused": 281.9, "visc_faces": 97.4, "faces": 64.0}
 # FP64 floating-point operations per DOF of one launch (mean over the 5 stages of a step): rocprofv3
-# SQ_INSTS_VALU_{ADD,MUL,FMA,TRANS}_F64 per dispatch, wave instructions x 64 lanes (every wave of
-# these kernels runs with all 64 lanes or skips a phase as a whole), FMA counted as 2; same summary
-MEASURED_FLOP_PER_DOF = {"dg_fused": 2048.6, "visc_faces": 391.0}
+# SQ_INSTS_VALU_{ADD,MUL,FMA,TRANS}_F64 per dispatch, wave instructions x 64 lanes (an upper bound:
+# lanes without a line or node count too), FMA counted as 2; same summary
+MEASURED_FLOP_PER_DOF = {"dg_fused": 1336.0, "visc_faces": 418.0}
 FP64_PEAK_TFLOPS = 78.6
 RHS_EVALS = 1000
 
