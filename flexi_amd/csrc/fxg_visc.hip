@@ -175,6 +175,13 @@ __global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(3))) v
   }
   const Prim q0 = cons_to_prim(nb[0], gas), q1 = cons_to_prim(nb[1], gas);
   Line<N> lp(d, la, lb);
+  // the element's boundary sides, one bit per local side: uniform, so that interior elements skip what follows for
+  // them (cavity box 32^3, N=7: 0.494 -> 0.457 ms)
+  int walls = 0;
+  if constexpr (BC) {
+#pragma unroll
+    for (int ls = 1; ls <= 6; ++ls) walls |= (m.E2S[2 * (ls - 1) + 12 * (size_t)e] <= m.nBC ? 1 : 0) << (ls - 1);
+  }
   __syncthreads();
   double jq[2][4];  // BR1 jumps with their sign and weight
 #pragma unroll
@@ -258,13 +265,12 @@ __global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(3))) v
         p[4 * x + v] = (Ja[x] * g[r][v] + Ja[3 + x] * g[r][4 + v] + Ja[6 + x] * g[r][8 + v]) * sj;
     if constexpr (BC) {
       // boundary sides: the gradients at their face points, for the ends of the lines below
-      if (t + r * NT < np) {
-        const int i = nd % n, j = (nd / n) % n, k = nd / nf, sides = node_sides<N>(i, j, k);
+      if (walls && t + r * NT < np) {
+        const int i = nd % n, j = (nd / n) % n, k = nd / nf, sides = node_sides<N>(i, j, k) & walls;
 #pragma unroll 1
         for (int ls = 1; ls <= 6; ++ls) {
           if (!(sides & (1 << (ls - 1)))) continue;
           const unsigned own = m.slotTab[(size_t)NF * e + face_point<N>(ls, i, j, k)];
-          if ((int)(own / (2u * (unsigned)nf)) >= m.nBC) continue;
           double* gb = gBC + 12 * slot_side_point<N>(own);
 #pragma unroll
           for (int x = 0; x < 12; ++x) gb[x] = p[x];
@@ -312,16 +318,19 @@ __global__ __launch_bounds__(S<N>::NT) __attribute__((amdgpu_waves_per_eu(3))) v
   if constexpr (BC) {
     // the outer slots of boundary sides (a kernel of its own over the boundary points otherwise); the gradients
     // were stored by this workgroup, before the barriers above
-#pragma unroll
+    if (!walls) return;
+#pragma unroll 1
     for (int s = 0; s < 2; ++s) {
       const unsigned own = s ? own1 : own0;
       const int side = (int)(own / (2u * (unsigned)nf));
       if (side >= m.nBC) continue;
       const size_t fp = slot_side_point<N>(own);
-      double q[12];
+      double q[12], fi[4];
 #pragma unroll
       for (int x = 0; x < 12; ++x) q[x] = gBC[12 * fp + x];
-      bc_visc_point<double>(m, FU + 5 * (size_t)own, q, f[s], FG + 4 * ((size_t)own + nf), bcP, gas, fp, side);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) fi[x] = s ? f[1][x] : f[0][x];
+      bc_visc_point<double>(m, FU + 5 * (size_t)own, q, fi, FG + 4 * ((size_t)own + nf), bcP, gas, fp, side);
     }
   }
 }
