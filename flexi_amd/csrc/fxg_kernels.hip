@@ -614,16 +614,18 @@ __global__ __launch_bounds__(Dim<N>::NT) void k_volint(const double* __restrict_
       if (t + r * NT < NF) sS[v * NF + t + r * NT] = sp[r] >= 0 ? (RF)ff[r][v] : -(RF)ff[r][v];
   __syncthreads();
   if (st.mode == 0 && !act) return;  // no barrier follows
+  if (act) {  // (the lanes beyond the nodes stay for the barriers and the face points below)
 #pragma unroll
-  for (int ls = 1; ls <= 6; ++ls) {
-    int a, b, l;
-    face_coords(ls, i, j, k, a, b, l);
-    if (GL && l != (is_minus(ls) ? 0 : N)) continue;
-    const RF sl = (RF)(GL ? (is_minus(ls) ? sB[B.L_HatMinus()] : sB[B.L_HatPlus() + N])
-                          : (is_minus(ls) ? sB[B.L_HatMinus() + l] : sB[B.L_HatPlus() + l]));
-    const RF* f = sS + (ls - 1) * nf + a + n * b;
+    for (int ls = 1; ls <= 6; ++ls) {
+      int a, b, l;
+      face_coords(ls, i, j, k, a, b, l);
+      if (GL && l != (is_minus(ls) ? 0 : N)) continue;
+      const RF sl = (RF)(GL ? (is_minus(ls) ? sB[B.L_HatMinus()] : sB[B.L_HatPlus() + N])
+                            : (is_minus(ls) ? sB[B.L_HatMinus() + l] : sB[B.L_HatPlus() + l]));
+      const RF* f = sS + (ls - 1) * nf + a + n * b;
 #pragma unroll
-    for (int v = 0; v < 5; ++v) acc[v] = acc[v] + f[v * NF] * sl;
+      for (int v = 0; v < 5; ++v) acc[v] = acc[v] + f[v * NF] * sl;
+    }
   }
   const double sj = m.sJ[gid];
   double ut[5];
