@@ -175,7 +175,7 @@ struct fxg_ctx {
   bool rhs_stale = false;
   int last_rhs = 0;  // 0: none since creation or fxg_set_state; 1: a right-hand side of U; 2: an LSERK step of U
   double last_b_dt = 0.0;
-  double* Uprev = nullptr;
+  double* Uprev = nullptr;  // (and the register of fxg_forward_n_steps, step_register)
   // the state whose lifted gradients G holds (c->U or Uprev), null when unknown
   const double* grads_state = nullptr;
   // fxg_get_gradients: one direction in FLEXI's layout (5 per node) and the density gradient
@@ -569,6 +569,18 @@ int refresh_last_rhs(fxg_ctx* c) {
   c->rhs_stale = false;
   c->grads_state = X;
   return 0;
+}
+
+// The register of steps on a caller's state that brings none: Uprev, since R holds what refresh_last_rhs forms the
+// last stage's input of the context's own step from. What was kept in Uprev, and the gradients in G that these
+// steps overwrite on the four-kernel path, are formed again on request. On a stream other than the context's the
+// caller orders the calls.
+double* step_register(fxg_ctx* c) {
+  if ((!c->fused && !c->weak) || (c->grads_state && c->grads_state == c->Uprev)) {
+    c->rhs_stale = true;
+    c->grads_state = nullptr;
+  }
+  return c->Uprev;
 }
 
 }  // namespace
@@ -986,6 +998,7 @@ int fxg_forward_n_steps(fxg_ctx* c, int nSteps, const double* dt, int nStages, c
     if (ensure_adjoint(c)) return 1;
     c->faces_of = nullptr;
     if (nSteps == 0) return 0;
+    double* R = step_register(c);
     const size_t face10 = (size_t)10 * c->nf * c->S, nTot = (size_t)nSteps * nStages;
     double* S = ckpt;
     double* F = ckpt + nTot * vol5;
@@ -998,17 +1011,18 @@ int fxg_forward_n_steps(fxg_ctx* c, int nSteps, const double* dt, int nStages, c
       fw.FU[0] = F + x * face10;
       fw.FU[1] = last ? c->fw.FU[0] : F + (x + 1) * face10;
       const fxg::RKStage stage{st == 0 ? 1 : 2, st == 0 ? 0.0 : -RKA[st - 1], RKb[st] * dt[it],
-                               last ? U : S + (x + 1) * vol5, c->R};
+                               last ? U : S + (x + 1) * vol5, R};
       HIPCHECK(fxg::launch_rhs_fused(c->m, fw, c->gas, c->p.riemann, 0, S + x * vol5, nullptr, stage, true, 0, nullptr,
                                      s, c->timer));
     }
     return 0;
   }
+  double* R = nSteps > 0 ? step_register(c) : nullptr;
   for (int it = 0; it < nSteps; ++it) {
     if (ckpt && it % checkpointEvery == 0)
       HIPCHECK(hipMemcpyAsync(ckpt + (size_t)(it / checkpointEvery) * vol5, U, vol5 * sizeof(double),
                               hipMemcpyDeviceToDevice, s));
-    if (lserk(c, dt[it], nStages, RKA, RKb, U, c->R, s, it > 0)) {
+    if (lserk(c, dt[it], nStages, RKA, RKb, U, R, s, it > 0)) {
       c->faces_of = nullptr;
       return 1;
     }
