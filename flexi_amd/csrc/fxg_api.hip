@@ -650,9 +650,9 @@ int fxg_create_from_nodes(const fxg_params* p, int nElems, int nSides, const int
     fail(err); ctx_free(c); return 1;
   }
   c->m.slaveNS = slaveNS;
-  // FXG_METRICS_OWN: the curl-form face metric depends only on the face, so each element's own
-  // boundary metric is the face metric; using it on both sides keeps the freestream exact to
-  // flux round-off. FXG_METRICS_REFERENCE: the master's NormVec/SurfElem on both sides, as FLEXI.
+  // FXG_METRICS_OWN: the face metric depends only on the face (curl form), or on the edges of a parallelepiped
+  // that are the face's to rounding, so each element's own boundary metric is the face metric; using it on both
+  // sides keeps the freestream exact to flux round-off. FXG_METRICS_REFERENCE: the master's NormVec/SurfElem on both sides, as FLEXI.
   c->m.ownFaceMetric = own ? 1 : 0;
   if (finish_setup(c)) { ctx_free(c); return 1; }
   *out = c;

@@ -15,7 +15,7 @@ namespace fxg {
 // master's normal. `m` supplies ElemToSide and S2V2. With `reference`, the metrics.f90 operation
 // order (absolute coordinates, one-dimensional basis changes in sequence, no FMA contraction;
 // SlaveNS must be null); otherwise coordinates relative to each element's first node, and with `flat` the
-// terms of a mesh of parallelepipeds exactly constant in each element. Returns nonzero and sets `err` on
+// terms of a mesh whose elements are parallelepipeds to rounding exactly constant in each element. Returns nonzero and sets `err` on
 // failure.
 int compute_metrics_gpu(int N, int nodeType, int NGeo, int nElems, const double* NodeCoords, const DevMesh& m,
                         double* Mf, double* Mg, double* Mh, double* sJ, double* xGP, double* NormVec,

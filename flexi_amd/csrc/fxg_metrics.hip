@@ -7,7 +7,6 @@
 // nodes; surface metrics of each master side from the interpolated face metrics.
 #include "fxg_metrics.h"
 
-#include <algorithm>
 #include <vector>
 
 #include "fxg_basis.h"
@@ -284,46 +283,46 @@ __global__ __launch_bounds__(512) void k_metrics_n(const double* __restrict__ XC
 // from its edges gives every node exactly the same values, without the curl form's rounding, and
 // lets the stage kernels read ten numbers per element instead of ten per node.
 
-// Largest absolute coordinate of the mesh, as the bits of a double (nonnegative doubles order as integers).
-__global__ __launch_bounds__(256) void k_coord_max(const double* __restrict__ NC, size_t count,
-                                                 unsigned long long* __restrict__ out) {
-  double x = 0.0;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (size_t)gridDim.x * 256) x = fmax(x, fabs(NC[i]));
-  for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_down(x, off, 64));
-  if ((threadIdx.x & 63) == 0) atomicMax(out, (unsigned long long)__double_as_longlong(x));
-}
-
-// One lane per element: half the mean edge vectors of the three directions, edge[9]; clears *ok where a node is
-// further from the affine map of these edges through the first corner's position (taken from the mean
-// of the corners) than the rounding of the mesh's coordinates.
+// One lane per element: half the mean edge vectors of the three directions, edge[9]; clears *ok where the element is
+// not affine to the rounding of the curl form, so that neither the terms themselves nor their match across a
+// face are worse than there. Two bounds, both relative to the element:
+//  - each of a direction's four edges within 4 eps of their mean. The face metric is then that of the face
+//    alone to 8 eps, and both elements of a face have it alike (the fluxes through it cancel), as in the curl form,
+//    which is off by 1.5e-15 (N=2) to 2.5e-14 (N=7). Vertices of a sheared box far from the origin are rounded
+//    by more than that (eps |x|/h); those of an axis-aligned one leave the four edges exactly alike;
+//  - every node within 64 eps of an edge of the affine map: the rounding of equidistant nodes of a box
+//    with up to some 64 elements across.
 __global__ __launch_bounds__(256) void k_affine_edges(const double* __restrict__ NC, int ng, int nElems,
-                                                    const unsigned long long* __restrict__ big,
                                                     double* __restrict__ edge, int* __restrict__ ok) {
   const int e = blockIdx.x * 256 + threadIdx.x;
   if (e >= nElems) return;
   const double* x = NC + (size_t)3 * ng * ng * ng * e;
   const int G = ng - 1;
-  double h[3][3], mid[3];
+  const double eps = 2.220446049250313e-16;
+  double h[3][3], len[3] = {0, 0, 0}, off[3] = {0, 0, 0};  // half edges; largest component, largest deviation of an edge
   for (int c = 0; c < 3; ++c) {
     double v[8];
     for (int q = 0; q < 8; ++q) v[q] = x[c + 3 * vol_id(ng, (q & 1) * G, ((q >> 1) & 1) * G, (q >> 2) * G)];
-    h[0][c] = 0.125 * (((v[1] - v[0]) + (v[3] - v[2])) + ((v[5] - v[4]) + (v[7] - v[6])));
-    h[1][c] = 0.125 * (((v[2] - v[0]) + (v[3] - v[1])) + ((v[6] - v[4]) + (v[7] - v[5])));
-    h[2][c] = 0.125 * (((v[4] - v[0]) + (v[5] - v[1])) + ((v[6] - v[2]) + (v[7] - v[3])));
-    mid[c] = 0.125 * (((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
+    for (int d = 0; d < 3; ++d) {
+      const int s = 1 << d, a = 1 << ((d + 1) % 3), b = 1 << ((d + 2) % 3);
+      const double f[4] = {v[s] - v[0], v[a + s] - v[a], v[b + s] - v[b], v[a + b + s] - v[a + b]};
+      const double mean = 0.25 * ((f[0] + f[1]) + (f[2] + f[3]));
+      h[d][c] = 0.5 * mean;
+      len[d] = fmax(len[d], fabs(mean));
+      for (int q = 0; q < 4; ++q) off[d] = fmax(off[d], fabs(f[q] - mean));
+    }
   }
   for (int d = 0; d < 3; ++d)
     for (int c = 0; c < 3; ++c) edge[(size_t)9 * e + 3 * d + c] = h[d][c];
-  // a node's coordinates and the eight corners' are each off by a few units in the last place of the
-  // largest coordinate of the mesh (box vertices are lo + i*h)
-  const double tol = 16.0 * 2.220446049250313e-16 * __longlong_as_double((long long)*big);
-  bool fine = true;
+  bool fine = true;  // (a NaN compares false and clears it; fmax alone would lose it)
+  for (int d = 0; d < 3; ++d) fine = fine && off[d] <= 4.0 * eps * len[d] && len[d] > 0.0;
+  const double tol = 64.0 * eps * fmin(len[0], fmin(len[1], len[2]));
   for (int k = 0; k < ng; ++k)
     for (int j = 0; j < ng; ++j)
       for (int i = 0; i < ng; ++i) {
-        const double a = 2.0 * i / G - 1.0, b = 2.0 * j / G - 1.0, cc = 2.0 * k / G - 1.0;
+        const double a = 2.0 * i / G, b = 2.0 * j / G, cc = 2.0 * k / G;
         for (int c = 0; c < 3; ++c)
-          fine = fine && fabs(x[c + 3 * vol_id(ng, i, j, k)] - (mid[c] + a * h[0][c] + b * h[1][c] + cc * h[2][c])) <= tol;
+          fine = fine && fabs((x[c + 3 * vol_id(ng, i, j, k)] - x[c]) - (a * h[0][c] + b * h[1][c] + cc * h[2][c])) <= tol;
       }
   if (!fine) *ok = 0;
 }
@@ -696,20 +695,14 @@ int compute_metrics_gpu(int N, int nodeType, int NGeo, int nElems, const double*
     return 0;
   }
   double *dm = nullptr, *XCLN = nullptr, *dXCLG = nullptr, *detRef = nullptr, *edge = nullptr;
-  // edge vectors, the largest coordinate and the affine flag
-  hipError_t e = hipMalloc((void**)&edge, ((size_t)9 * nElems + 2) * sizeof(double));
+  // edge vectors and the affine flag
+  hipError_t e = hipMalloc((void**)&edge, ((size_t)9 * nElems + 1) * sizeof(double));
   int affine = flat;
   if (e == hipSuccess && flat) {
-    unsigned long long* big = reinterpret_cast<unsigned long long*>(edge + (size_t)9 * nElems);
-    int* ok = reinterpret_cast<int*>(big + 1);
-    const unsigned long long zero = 0;
-    e = hipMemcpyAsync(big, &zero, sizeof(zero), hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(ok, &affine, sizeof(int), hipMemcpyHostToDevice, s);
+    int* ok = reinterpret_cast<int*>(edge + (size_t)9 * nElems);
+    e = hipMemcpyAsync(ok, &affine, sizeof(int), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
-      const size_t count = (size_t)3 * ngp * nElems;
-      hipLaunchKernelGGL(k_coord_max, dim3((unsigned)std::min<size_t>(1024, (count + 255) / 256)), dim3(256), 0, s,
-                         NodeCoords, count, big);
-      hipLaunchKernelGGL(k_affine_edges, dim3((nElems + 255) / 256), dim3(256), 0, s, NodeCoords, ng, nElems, big, edge, ok);
+      hipLaunchKernelGGL(k_affine_edges, dim3((nElems + 255) / 256), dim3(256), 0, s, NodeCoords, ng, nElems, edge, ok);
       e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(&affine, ok, sizeof(int), hipMemcpyDeviceToHost, s);
