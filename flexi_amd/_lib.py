@@ -98,7 +98,8 @@ EXPORTS = ["fxg_last_error", "fxg_version", "fxg_create", "fxg_create_from_nodes
            "fxg_sync", "fxg_sizes", "fxg_calc_timestep_dev_noalloc",
            "fxg_profile_enable", "fxg_profile_read"]
 
-KERNEL_NAMES = ["prolong_u", "lift", "flux", "volint", "dt_elem", "dt_reduce", "faces", "visc_faces", "dg_fused"]
+KERNEL_NAMES = ["prolong_u", "lift", "flux", "volint", "dt_elem", "dt_reduce", "faces", "visc_faces", "dg_fused",
+                "weak_faces", "weak_visc", "weak_stage"]
 
 
 def check(rc: int) -> None:

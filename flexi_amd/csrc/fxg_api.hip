@@ -159,8 +159,8 @@ struct fxg_ctx {
   EventTimer* timer = nullptr;  // non-null while kernel timing is enabled
   // fused Gauss-Lobatto split-form path: face states double-buffered across LSERK stages
   bool fused = false;
-  // weak form in FP64 without boundary sides: the two line kernels instead of the four (reported as
-  // "classic": the path of every form but the split one); its face states are kept like the fused path's
+  // weak form in FP64 without boundary sides: the two line kernels instead of the four; its face states are kept
+  // like the fused path's
   bool weak = false;
   fxg::FusedWork fw{};
   int cur = 0;
@@ -927,7 +927,7 @@ int fxg_timestep_lserkw2_dev(fxg_ctx* c, double t, double dt, int nStages, const
   return rc;
 }
 
-const char* fxg_pipeline(fxg_ctx* c) { return !c ? "" : (c->fused ? "fused" : "classic"); }
+const char* fxg_pipeline(fxg_ctx* c) { return !c ? "" : (c->fused ? "fused" : (c->weak ? "weak" : "classic")); }
 
 int fxg_sync(fxg_ctx* c) {
   if (!c) return fail("ctx is NULL");

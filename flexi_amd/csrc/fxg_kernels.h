@@ -94,7 +94,7 @@ struct RKStage {
 // 0-3: four-kernel path; 6-8: fused Gauss-Lobatto split-form path.
 enum KernelId {
   K_PROLONG = 0, K_LIFT = 1, K_FLUX = 2, K_VOLINT = 3, K_DT_ELEM = 4, K_DT_REDUCE = 5,
-  K_FACES = 6, K_VISC_FACES = 7, K_DG_FUSED = 8, K_COUNT = 9
+  K_FACES = 6, K_VISC_FACES = 7, K_DG_FUSED = 8, K_WEAK_FACES = 9, K_WEAK_VISC = 10, K_WEAK_STAGE = 11, K_COUNT = 12
 };
 
 // Records a HIP event before (start = true) and after each kernel launch when timing is on.

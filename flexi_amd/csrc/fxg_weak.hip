@@ -585,15 +585,15 @@ hipError_t weak_n(const DevMesh& m, const FusedWork& w, const Gas& gas, int riem
   double* FU = w.FU[cur];
   double* FG = (double*)w.FG;
   if (!faces_fresh) {
-    Scope sc(tm, K_PROLONG, s);
+    Scope sc(tm, K_WEAK_FACES, s);
     hipLaunchKernelGGL((k_weak_faces<N, GL>), g, b, 0, s, U, m, m.basis, FU);
   }
   {
-    Scope sc(tm, K_LIFT, s);
+    Scope sc(tm, K_WEAK_VISC, s);
     hipLaunchKernelGGL((k_weak_visc<N, GL, AFF>), g, b, 0, s, U, m, m.basis, FU, FG, gas);
   }
   {
-    Scope sc(tm, K_VOLINT, s);
+    Scope sc(tm, K_WEAK_STAGE, s);
 #define FXG_LAUNCH(SOLV)                                                                                               \
   if (st.lamSum)                                                                                                       \
     hipLaunchKernelGGL((k_weak_stage<N, SOLV, GL, AFF, true>), g, b, 0, s, U, m, m.basis, FU, w.FU[1 - cur], FG, gas, \

@@ -235,7 +235,7 @@ class DGSolver:
         return n.value
 
     def kernel_pipeline(self) -> str:
-        """'fused' or 'classic' (which stage kernels this context launches)."""
+        """'fused', 'weak' or 'classic' (which stage kernels this context launches, include/fxg.h)."""
         return _lib.lib().fxg_pipeline(self.ctx).decode()
 
     def sync(self) -> None:

@@ -231,8 +231,9 @@ int fxg_adjoint_storage(fxg_ctx* ctx, int nSteps, int nStages, int checkpointEve
 int fxg_calc_timestep_dev_noalloc(fxg_ctx* ctx, const double* U_dev, double CFLScale, double DFLScale,
                                   double* dt_dev, int* errType_dev, void* stream);
 /* Which stage kernels the context runs: "fused" (Gauss-Lobatto split form, N 2..7: two
- * kernels per stage, face states carried between LSERK stages) or "classic" (prolongation,
- * lifting, side fluxes, integrals). No counterpart in the reference; FXG_PIPELINE=classic in
+ * kernels per stage, face states carried between LSERK stages), "weak" (the same for the weak form
+ * in FP64, N 2..7, without boundary sides, on either node type) or "classic" (prolongation, lifting, side
+ * fluxes, integrals). No counterpart in the reference; FXG_PIPELINE=classic in
  * the environment at fxg_create time selects the classic path everywhere. */
 const char* fxg_pipeline(fxg_ctx* ctx);
 /* Synchronise the context's stream. */
@@ -247,8 +248,9 @@ int fxg_sizes(fxg_ctx* ctx, int* N, int* nElems, int* nSides);
  * and returns the summed duration and launch count of one kernel since enabling.
  * Kernel ids: 0 prolongation, 1 lifting, 2 side fluxes, 3 volume/surface integral (+RK update),
  * 4 per-element time step, 5 time-step reduction; on the fused Gauss-Lobatto split-form path
- * 6 face states of the first stage, 7 viscous face fluxes, 8 fused stage. Enabling again resets
- * the counters. */
+ * 6 face states of the first stage, 7 viscous face fluxes, 8 fused stage; on the weak form's
+ * two-kernel path 9, 10 and 11 likewise. A time step from the sums of the last stage is one launch of 5.
+ * Enabling again resets the counters. */
 int fxg_profile_enable(fxg_ctx* ctx, int enable);
 int fxg_profile_read(fxg_ctx* ctx, int kernel, double* total_ms, int* launches);
 
