@@ -502,7 +502,7 @@ int ensure_adjoint(fxg_ctx* c) {
 
 // Device workspace of one adjoint run. Up to kKeepAdjoint bytes it stays with the context for the next run
 // (its hipMalloc and hipFree took 1.8 ms of the 19.3 ms of a gradient through ten steps at 16^3, N=5) until a
-// larger one replaces it or the context is destroyed; a larger one is released at the end of the run. A run that
+// larger one replaces it, a run of no steps or the end of the context; a larger one is released at the end of the run. A run that
 // fails releases it in any case: hipFree waits for what is still in flight.
 constexpr size_t kKeepAdjoint = (size_t)4 << 30;
 struct AdjointBuffer {
@@ -1043,7 +1043,12 @@ int fxg_adjoint_n_steps(fxg_ctx* c, int nSteps, const double* dt, int nStages, c
   if (check_rk(nStages, RKA, RKb)) return 1;
   if (ensure_adjoint(c)) return 1;
   c->faces_of = nullptr;  // the recomputation below runs on scratch states
-  if (nSteps == 0) return 0;
+  if (nSteps == 0) {
+    if (c->adjRun) HIPCHECK(hipFree(c->adjRun));
+    c->adjRun = nullptr;
+    c->adjRunSize = 0;
+    return 0;
+  }
   const hipStream_t s = stream ? (hipStream_t)stream : c->stream;
   const size_t vol5 = (size_t)5 * c->np * c->K, bytes = vol5 * sizeof(double);
   const size_t face10 = (size_t)10 * c->nf * c->S;  // both slots of every side, 5 per point

@@ -234,6 +234,12 @@ class DGSolver:
                                                   C.byref(n)))
         return n.value
 
+    def release_workspace(self) -> None:
+        """Frees the device memory (up to 4 GiB) that adjoint runs of this solver keep for the next one, for a
+        program that needs it elsewhere (a run of no steps: its pointers are not used)."""
+        p = self._dt_array(np.zeros(1))[0].ctypes.data
+        self.adjoint_n_steps_dev(p, p, [], 1)
+
     def kernel_pipeline(self) -> str:
         """'fused', 'weak' or 'classic' (which stage kernels this context launches, include/fxg.h)."""
         return _lib.lib().fxg_pipeline(self.ctx).decode()

@@ -203,8 +203,10 @@ int fxg_timestep_lserkw2_dev(fxg_ctx* ctx, double t, double dt, int nStages, con
  *   U(0) -> U(T) of fxg_forward_n_steps started from U0_dev. The stage states are recomputed
  *   segment by segment from the checkpoints: those of a forward call with the same
  *   checkpointEvery (ckpt_dev), or, with ckpt_dev NULL, from a forward sweep of its own. Device
- *   memory allocated for the call: checkpointEvery*nStages + 3 states (+ the checkpoints when it
- *   takes them itself). With checkpointEvery = 0, ckpt_dev must be the trajectory of a forward
+ *   memory allocated for the call: checkpointEvery*nStages states with their face states + 3 states (+ the
+ *   checkpoints when it takes them itself). Up to 4 GiB of it stay with the context for its next run, until a
+ *   larger run, a run of no steps (nSteps = 0, which only gives it back; the pointers are not used) or
+ *   fxg_destroy; more is freed at the end of the call. With checkpointEvery = 0, ckpt_dev must be the trajectory of a forward
  *   call with checkpointEvery = 0 and the same steps; only the reverse stages run (one state of
  *   scratch). Synchronous.
  * fxg_adjoint_storage: the number of doubles ckpt_dev needs for nSteps steps and checkpointEvery
