@@ -176,6 +176,9 @@ struct fxg_ctx {
   int last_rhs = 0;  // 0: none since creation or fxg_set_state; 1: a right-hand side of U; 2: an LSERK step of U
   double last_b_dt = 0.0;
   double* Uprev = nullptr;  // (and the register of fxg_forward_n_steps, step_register)
+  // a call on a caller's state was captured into a graph (note_capture): its replays write the face states, G and
+  // Uprev unseen, so these are never taken for the context's own again
+  bool captured = false;
   // the state whose lifted gradients G holds (c->U or Uprev), null when unknown
   const double* grads_state = nullptr;
   // fxg_get_gradients: one direction in FLEXI's layout (5 per node) and the density gradient
@@ -556,7 +559,7 @@ struct AdjointBuffer {
 // round-off), and one right-hand side there restores them; after a right-hand side of U, or with
 // none yet, the right-hand side of U.
 int refresh_last_rhs(fxg_ctx* c) {
-  if (!c->rhs_stale) return 0;
+  if (!c->rhs_stale && !(c->captured && c->last_rhs != 0)) return 0;
   const double* X = c->U;
   if (c->last_rhs == 2) {
     const size_t vol5 = (size_t)5 * c->np * c->K;
@@ -581,6 +584,11 @@ double* step_register(fxg_ctx* c) {
     c->grads_state = nullptr;
   }
   return c->Uprev;
+}
+
+void note_capture(fxg_ctx* c, hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone) c->captured = true;
 }
 
 }  // namespace
@@ -889,7 +897,7 @@ int fxg_timestep_lserkw2(fxg_ctx* c, double t, double dt, int nStages, const dou
   if (!c) return fail("ctx is NULL");
   c->lam_of = nullptr;
   c->grads_state = nullptr;
-  if (lserk(c, dt, nStages, RKA, RKb, c->U, c->R, c->stream, c->faces_of == c->U, true)) return 1;
+  if (lserk(c, dt, nStages, RKA, RKb, c->U, c->R, c->stream, c->faces_of == c->U && !c->captured, true)) return 1;
   // Ut of the last stage is not kept by either pipeline, the gradients not by the fused one
   c->rhs_stale = true;
   c->last_rhs = 2;
@@ -903,8 +911,10 @@ int fxg_dg_time_derivative_dev(fxg_ctx* c, double t, const double* U, double* Ut
   (void)t;
   if (!c || !U || !Ut) return fail("NULL argument");
   fxg::RKStage st{0, 0.0, 0.0, nullptr, nullptr};
+  const hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+  note_capture(c, s);
   // the gradients of the caller's state cannot be asked for
-  const int rc = rhs(c, U, Ut, st, stream ? (hipStream_t)stream : c->stream, false, false);
+  const int rc = rhs(c, U, Ut, st, s, false, false);
   c->faces_of = nullptr;  // the caller's buffer may change before the next call
   // on the four-kernel path G now holds the gradients of the caller's state: the context's are recomputed
   // on request
@@ -918,7 +928,9 @@ int fxg_timestep_lserkw2_dev(fxg_ctx* c, double t, double dt, int nStages, const
   (void)t;
   (void)RKc;
   if (!c || !U || !R) return fail("NULL argument");
-  const int rc = lserk(c, dt, nStages, RKA, RKb, U, R, stream ? (hipStream_t)stream : c->stream);
+  const hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+  note_capture(c, s);
+  const int rc = lserk(c, dt, nStages, RKA, RKb, U, R, s);
   c->faces_of = nullptr;
   if (!c->fused) {  // the four-kernel stages wrote the caller's gradients into G
     c->rhs_stale = true;
@@ -991,6 +1003,7 @@ int fxg_forward_n_steps(fxg_ctx* c, int nSteps, const double* dt, int nStages, c
   if (ckpt && checkpointEvery < 0) return fail("checkpointEvery must not be negative");
   if (check_rk(nStages, RKA, RKb)) return 1;
   const hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+  note_capture(c, s);
   const size_t vol5 = (size_t)5 * c->np * c->K;
   if (ckpt && checkpointEvery == 0) {
     // trajectory: every stage's input state and its face states, written by the stages themselves

@@ -180,7 +180,9 @@ int fxg_calc_timestep(fxg_ctx* ctx, double CFLScale, double DFLScale, double* dt
  * uses the context's scratch arrays (face states, face fluxes, gradients), so calls on one
  * context must be serialised: with a stream other than the context's, the caller orders the
  * calls itself (e.g. synchronises before switching streams). Afterwards fxg_get_ut and
- * fxg_get_gradients recompute those of the context's own state. */
+ * fxg_get_gradients recompute those of the context's own state. The calls launch kernels and device copies only,
+ * so they can be captured into a HIP graph (after one eager call, which loads the kernels); a context that
+ * had a call captured keeps nothing of its own state in the arrays that a replay writes. */
 int fxg_dg_time_derivative_dev(fxg_ctx* ctx, double t, const double* U_dev, double* Ut_dev,
                                void* stream);
 int fxg_timestep_lserkw2_dev(fxg_ctx* ctx, double t, double dt, int nStages, const double* RKA,
