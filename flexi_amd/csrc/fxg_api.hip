@@ -341,14 +341,11 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
   HIPCHECK(hipMemsetAsync(c->Ut, 0, 5 * vol * sizeof(double), c->stream));
   HIPCHECK(hipMemsetAsync(c->R, 0, 5 * vol * sizeof(double), c->stream));
   const size_t gsz = p->precision == FXG_PREC_FP32_BULK ? sizeof(float) : sizeof(double);
-  char *G, *Gm, *Gs;
-  if (alloc_owned(c, &c->w.Uf_m, 5 * face) || alloc_owned(c, &c->w.Uf_s, 5 * face) ||
-      alloc_owned(c, &G, 12 * vol * gsz) || alloc_owned(c, &Gm, 12 * face * gsz) || alloc_owned(c, &Gs, 12 * face * gsz) ||
-      alloc_owned(c, &c->w.Flux, 5 * face) || alloc_owned(c, &c->w.dtElem, 2 * (size_t)K) ||
-      alloc_owned(c, &c->w.errElem, (size_t)K) ||
-      alloc_owned(c, &c->w.bcLift, 4 * (size_t)c->nf * nBC))
+  char* G;
+  if (alloc_owned(c, &G, 12 * vol * gsz) || alloc_owned(c, &c->w.dtElem, 2 * (size_t)K) ||
+      alloc_owned(c, &c->w.errElem, (size_t)K))
     return 1;
-  c->w.G = G; c->w.Gf_m = Gm; c->w.Gf_s = Gs;
+  c->w.G = G;
   HIPCHECK(hipMemsetAsync(G, 0, 12 * vol * gsz, c->stream));
   // FXG_PIPELINE=classic keeps the four-kernel path for cases the fused one covers
   const char* pipe = std::getenv("FXG_PIPELINE");
@@ -357,6 +354,14 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
   c->weak = !c->fused && fxg::weak_supported(c->N, p->nodeType, p->splitDG == FXG_SPLITDG_PI,
                                              p->precision == FXG_PREC_FP32_BULK, nBC, S) &&
             !(pipe && std::strcmp(pipe, "classic") == 0);
+  if (!c->fused && !c->weak) {
+    char *Gm, *Gs;
+    if (alloc_owned(c, &c->w.Uf_m, 5 * face) || alloc_owned(c, &c->w.Uf_s, 5 * face) ||
+        alloc_owned(c, &Gm, 12 * face * gsz) || alloc_owned(c, &Gs, 12 * face * gsz) ||
+        alloc_owned(c, &c->w.Flux, 5 * face) || alloc_owned(c, &c->w.bcLift, 4 * (size_t)c->nf * nBC))
+      return 1;
+    c->w.Gf_m = Gm; c->w.Gf_s = Gs;
+  }
   if (c->weak) {
     double* FG;
     if (alloc_owned(c, &c->fw.FU[0], 10 * face) || alloc_owned(c, &c->fw.FU[1], 10 * face) || alloc_owned(c, &FG, 8 * face) ||
@@ -648,7 +653,7 @@ int fxg_create_from_nodes(const fxg_params* p, int nElems, int nSides, const int
   double* slaveNS = nullptr;
   if (own && !c->fused) {
     const size_t face = (size_t)c->nf * nSides;
-    if (alloc_owned(c, &slaveNS, 3 * face) || alloc_owned(c, &c->w.FluxS, 5 * face)) { ctx_free(c); return 1; }
+    if (alloc_owned(c, &slaveNS, 3 * face) || (!c->weak && alloc_owned(c, &c->w.FluxS, 5 * face))) { ctx_free(c); return 1; }
   }
   // (FP32-bulk keeps each node's own rounding of the terms: any other would change which of its sums round
   // up, and with that its results by an ulp of FP32 at some nodes)
@@ -793,8 +798,14 @@ int fxg_get_gradients(fxg_ctx* c, int nVarLifting, double* gx, double* gy, doubl
     if (!c->grads_state)
       return fail("fxg_get_gradients: no right-hand side has been evaluated for the current state");
     if (!c->rhoG && alloc_owned(c, &c->rhoG, 3 * nodes)) return 1;
-    HIPCHECK(fxg::launch_lift_density(c->m, c->w, c->gas, c->p.nodeType, c->grads_state, c->rhoG, c->stream));
-    if (!c->fused && !c->weak) c->faces_of = nullptr;  // it prolongs that state into the same face arrays
+    fxg::DevWork w = c->w;
+    if (c->fused || c->weak) {  // the face states' buffer that the next stage writes
+      w.Uf_m = c->fw.FU[1 - c->cur];
+      w.Uf_s = w.Uf_m + (size_t)5 * c->nf * c->S;
+    } else {
+      c->faces_of = nullptr;  // it prolongs that state into the same face arrays
+    }
+    HIPCHECK(fxg::launch_lift_density(c->m, w, c->gas, c->p.nodeType, c->grads_state, c->rhoG, c->stream));
   }
   double* host[3] = {gx, gy, gz};
   for (int d = 0; d < 3; ++d) {
