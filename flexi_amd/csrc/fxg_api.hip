@@ -351,7 +351,7 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
   const char* pipe = std::getenv("FXG_PIPELINE");
   c->fused = fxg::fused_supported(c->N, p->nodeType, p->splitDG == FXG_SPLITDG_PI, S) &&
              !(pipe && std::strcmp(pipe, "classic") == 0);
-  c->weak = !c->fused && fxg::weak_supported(c->N, p->nodeType, p->splitDG == FXG_SPLITDG_PI,
+  c->weak = !c->fused && fxg::weak_supported(c->N, p->splitDG == FXG_SPLITDG_PI,
                                              p->precision == FXG_PREC_FP32_BULK, nBC, S) &&
             !(pipe && std::strcmp(pipe, "classic") == 0);
   if (!c->fused && !c->weak) {

@@ -144,16 +144,6 @@ __device__ __forceinline__ void load_metrics(const DevMesh& m, size_t gid, RF* J
   sj = (RF)m.sJ[gid];
 }
 
-// Metric terms of node t from the element's block of the packed array (rows of np: Ja^1 x,y,z,
-// Ja^2 x,y,z, Ja^3 x,y,z, sJ), so that consecutive lanes load consecutive doubles.
-template <int N, class RF>
-__device__ __forceinline__ void load_metrics(const double* Je, int t, RF* Ja, RF& sj) {
-  constexpr int np = D<N>::np;
-#pragma unroll
-  for (int r = 0; r < 9; ++r) Ja[r] = (RF)Je[r * np + t];
-  sj = (RF)Je[9 * np + t];
-}
-
 // Geometry of own face point (local side ls, Jd: the metric terms Ja^dir of its node), the same arithmetic as the surface
 // phase of the fused stage kernel: the master normal nv, SurfElem (returned) and a tangential
 // basis (Gram-Schmidt of the coordinate axis least aligned with n, t2 = n x t1). With

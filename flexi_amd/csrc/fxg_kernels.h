@@ -156,7 +156,7 @@ hipError_t launch_stage(const DevMesh& m, const FusedWork& w, const Gas& gas, in
                         const RKStage& st, int cur, double* G, hipStream_t s);
 // One right-hand side or stage of the weak form by the two line kernels (fxg_weak.hip), with FU and FG of
 // FusedWork used as on the fused path. G (optional, (np,12,nElems)) receives the lifted gradients.
-bool weak_supported(int N, int nodeType, int split, int fp32, int nBC, long long nSides);
+bool weak_supported(int N, int split, int fp32, int nBC, long long nSides);
 hipError_t launch_rhs_weak(const DevMesh& m, const FusedWork& w, const Gas& gas, int nodeType, int riemann,
                            const double* U, double* Ut, const RKStage& st, bool faces_fresh, int cur, double* G,
                            hipStream_t s, KernelTimer* timer);
@@ -203,10 +203,6 @@ hipError_t launch_calc_timestep(const DevMesh& m, const DevWork& w, const Gas& g
 // CALCTIMESTEP from the spectral-radius sums a last stage stored for the current state; `elements`: w.dtElem too.
 hipError_t launch_calc_timestep_from_sums(const DevMesh& m, const DevWork& w, const double* lamSum, const int* lamNan,
                                           double CFL, double DFL, bool elements, hipStream_t s, KernelTimer* timer);
-// Copies a (12, np, nElems) gradient array of type float/double into three FLEXI-layout
-// FP64 arrays (4,0:N,0:N,0:N,nElems).
-hipError_t launch_unpack_gradients(const DevMesh& m, const void* G, int fp32, double* gx, double* gy,
-                                   double* gz, hipStream_t s);
 // Lifted density gradient rhoG(np, 3, nElems) of U (PP_OPTLIFT=0's LIFT_DENS), through the face
 // states written into w.Uf_m/Uf_s (overwritten).
 hipError_t launch_lift_density(const DevMesh& m, const DevWork& w, const Gas& gas, int nodeType, const double* U,

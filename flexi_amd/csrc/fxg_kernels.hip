@@ -768,20 +768,6 @@ __global__ __launch_bounds__(1024) void k_dt_reduce(const double* __restrict__ d
   dt_min(c, v, ec, out, errOut);
 }
 
-template <class RF>
-__global__ __launch_bounds__(256) void k_unpack_grad(const RF* __restrict__ G, int np, int nNodes, double* __restrict__ gx,
-                                                   double* __restrict__ gy, double* __restrict__ gz) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= nNodes) return;
-  const int e = x / np, t = x - e * np;
-  const RF* Ge = G + (size_t)12 * np * e;
-  for (int v = 0; v < 4; ++v) {
-    gx[4 * (size_t)x + v] = (double)Ge[v * np + t];
-    gy[4 * (size_t)x + v] = (double)Ge[(4 + v) * np + t];
-    gz[4 * (size_t)x + v] = (double)Ge[(8 + v) * np + t];
-  }
-}
-
 // ---------------------------------------------------------------------------------------------
 // Lifted density gradient, the first lifting variable of FLEXI's default build (PP_OPTLIFT=0,
 // LIFT_DENS, idealgas/eos.h:108-117): the BR1 lifting of k_lift applied to rho (strong form,
@@ -1029,19 +1015,6 @@ hipError_t launch_unpack_gradient_dir(const DevMesh& m, const void* G, int fp32,
   else
     hipLaunchKernelGGL(k_unpack_grad_dir<double>, dim3((nNodes + 255) / 256), dim3(256), 0, s, (const double*)G, rhoG,
                        np, nNodes, nVar, dir, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_unpack_gradients(const DevMesh& m, const void* G, int fp32, double* gx, double* gy, double* gz,
-                                   hipStream_t s) {
-  const int n = m.N + 1, np = n * n * n;
-  const int nNodes = np * m.nElems;
-  if (fp32)
-    hipLaunchKernelGGL(k_unpack_grad<float>, dim3((nNodes + 255) / 256), dim3(256), 0, s, (const float*)G, np, nNodes,
-                       gx, gy, gz);
-  else
-    hipLaunchKernelGGL(k_unpack_grad<double>, dim3((nNodes + 255) / 256), dim3(256), 0, s, (const double*)G, np, nNodes,
-                       gx, gy, gz);
   return hipGetLastError();
 }
 

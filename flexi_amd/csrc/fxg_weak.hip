@@ -634,8 +634,7 @@ hipError_t launch_rhs_weak(const DevMesh& m, const FusedWork& w, const Gas& gas,
 }
 
 // Side slots are 32-bit, as on the split form's path. N = 1 has too few nodes on a line to gain.
-bool weak_supported(int N, int nodeType, int split, int fp32, int nBC, long long nSides) {
-  (void)nodeType;
+bool weak_supported(int N, int split, int fp32, int nBC, long long nSides) {
   return !split && !fp32 && nBC == 0 && N >= 2 && N <= 7 && nSides * 2LL * (N + 1) * (N + 1) < (1LL << 32);
 }
 
