@@ -1,5 +1,5 @@
 // Discrete adjoint of the Gauss-Lobatto split-form right-hand side (the fused stage's arithmetic):
-// out = (dUt/dU)^T lam at a state U, written as three element kernels and the face-state kernel.
+// out = (dUt/dU)^T lam at a state U, written as three element kernels.
 //
 // Forward, per element and node i (mu_i = -sJ_i lam_i is the adjoint of the accumulated terms):
 //   Ut_i = -sJ_i [ sum_d sum_l DVolSurf(l,i) F#(P_i,P_l; Ja^d_i,Ja^d_l)            split Euler part
@@ -305,8 +305,11 @@ __device__ __forceinline__ void rot_state_adjoint(const double* c, const Gas& g,
 // Both element kernels give each lane a line of nodes, as the forward stage kernel does (fxg_stage.hip): a
 // pair's Jacobian serves both of its nodes, so evaluating it once per pair halves it, and the LDS reads
 // per node fall from about 330 to 90 (k_adj_euler) and from 290 to 110 (k_adj_visc), which bound the forms with
-// one lane per node. TGV 16^3, N=5, Roe, parallelepipeds: 134 -> 112 us and 90 -> 61 us per reverse stage (about 430 and 310
-// bytes per node at 3.4 and 4.5 TB/s). Two waves per SIMD: at three the Riemann reverse spills (143 and 88 us).
+// one lane per node. TGV 16^3, N=5, Roe, parallelepipeds: 134 -> 110 us and 90 -> 58 us per reverse stage (491 and 321
+// bytes per node at 4.0 and 4.9 TB/s). Two waves per SIMD: at three the Riemann reverse spills (143 and 88 us); with
+// Roe-entropy-fix 3 to 11 VGPRs spill at two as well. At N = 7 with general metric terms k_adj_euler's 93 KB of
+// LDS leave one workgroup per CU, one wave per SIMD: vjp at 12^3, Roe 0.241 -> 0.206 ms all the same
+// (parallelepipeds 0.248 -> 0.161).
 
 // The lane's line: direction, end nodes (offset in the element), local sides and side slots of its ends.
 template <int N>

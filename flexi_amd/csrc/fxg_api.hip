@@ -164,8 +164,8 @@ struct fxg_ctx {
   bool weak = false;
   fxg::FusedWork fw{};
   int cur = 0;
-  // the state whose face values FU[cur] (four-kernel path: w.Uf_m, w.Uf_s) holds (only trusted for the context's own state, which
-  // changes only through fxg_set_state and the library's own updates)
+  // the state whose face values FU[cur] (four-kernel path: w.Uf_m, w.Uf_s) holds (only trusted for the context's own
+  // state, which changes only through fxg_set_state and the library's own updates)
   const double* faces_of = nullptr;
   // Ut and the lifted gradients (G) of the context's last right-hand side. After an LSERK step on
   // the context's state that is the last stage's, at the state before the last update,
@@ -510,8 +510,8 @@ int ensure_adjoint(fxg_ctx* c) {
 
 // Device workspace of one adjoint run. Up to kKeepAdjoint bytes it stays with the context for the next run
 // (its hipMalloc and hipFree took 1.8 ms of the 19.3 ms of a gradient through ten steps at 16^3, N=5) until a
-// larger one replaces it, a run of no steps or the end of the context; a larger one is released at the end of the run. A run that
-// fails releases it in any case: hipFree waits for what is still in flight.
+// larger one replaces it, a run of no steps or the end of the context; a larger one is released at the end of the
+// run. A run that fails releases it in any case: hipFree waits for what is still in flight.
 constexpr size_t kKeepAdjoint = (size_t)4 << 30;
 struct AdjointBuffer {
   fxg_ctx* c;
@@ -665,7 +665,8 @@ int fxg_create_from_nodes(const fxg_params* p, int nElems, int nSides, const int
   c->m.slaveNS = slaveNS;
   // FXG_METRICS_OWN: the face metric depends only on the face (curl form), or on the edges of a parallelepiped
   // that are the face's to rounding, so each element's own boundary metric is the face metric; using it on both
-  // sides keeps the freestream exact to flux round-off. FXG_METRICS_REFERENCE: the master's NormVec/SurfElem on both sides, as FLEXI.
+  // sides keeps the freestream exact to flux round-off. FXG_METRICS_REFERENCE: the master's NormVec/SurfElem on
+  // both sides, as FLEXI.
   c->m.ownFaceMetric = own ? 1 : 0;
   if (finish_setup(c)) { ctx_free(c); return 1; }
   *out = c;

@@ -63,6 +63,7 @@ struct DevMesh {
 
 // Work arrays of one right-hand side evaluation. Face arrays of U are FP64 (U(5,p,q,side));
 // gradient arrays hold T = double or float (FP32-bulk).
+// On the two-kernel paths a context holds neither these face arrays nor the fluxes.
 struct DevWork {
   double* Uf_m;    // (5,0:N,0:N,nSides)
   double* Uf_s;

@@ -26,7 +26,7 @@ namespace {
 // AFF: where every element's metric terms are the same at all of its nodes (parallelepipeds: m.aff, checked
 // bitwise at set-up) they are ten uniform values: no metric rows in LDS (13 rows instead of 15, three
 // workgroups per CU instead of two at N = 7), 80 bytes per node less to read, and the pair flux needs only the
-// sum of the contravariant velocities. N = 7, 32^3: 1.31 -> 1.01 ms (278 bytes per node, 4.6 TB/s); N = 4, 32^3
+// sum of the contravariant velocities. N = 7, 32^3: 1.31 -> 1.05 ms (282 bytes per node, 4.5 TB/s); N = 4, 32^3
 // 0.381 -> 0.333, N = 5, 24^3 0.268 -> 0.224, N = 6, 24^3 0.475 -> 0.337.
 
 // LDS rows: 0 u, 1 v, 2 w, 3 rho/4, 4 p, 5 H, 6 T; 7..12 exchange between line and node phases

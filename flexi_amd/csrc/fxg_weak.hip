@@ -11,11 +11,13 @@
 // double-buffered across stages as on the split form's path; k_weak_faces fills them where no stage has.
 //
 // The four-kernel path (fxg_kernels.hip) stores the gradients (96 bytes per node written and read again) and
-// reads the metric terms and U in two more passes: about 950 bytes per node at N = 5 against 720 here (560 on
-// meshes of parallelepipeds), and its element kernels, one lane per node, are bound by LDS reads. A stage
+// reads the metric terms and U in two more passes: about 950 bytes per node at N = 5 against 742 here (on
+// parallelepipeds 558 at N = 3, 402 at N = 7), and its element kernels, one lane per node, are bound by LDS reads. A stage
 // (all kernels) on Gauss nodes, Roe: N = 3, 32^3 0.67 -> 0.29 ms; N = 5, 24^3 0.85 -> 0.36 (curved 0.86 -> 0.51);
 // N = 7, 32^3 4.75 -> 1.70. At 8^3, N = 3 two kernels of 13 us together instead of four of 31.
-// N = 7 is held to two waves per SIMD: at three both kernels spill, at the same time.
+// N = 7 is held to two waves per SIMD: at three both kernels spill, at the same time. Below, Roe-entropy-fix
+// spills 2 to 24 VGPRs at three (Roe at most 4); a step at 17^3, N = 5: 1.57 -> 1.03 ms curved, 1.58 -> 0.77 straight
+// (Roe 1.57 -> 0.97 and 1.58 -> 0.68).
 #include "fxg_line.h"
 
 namespace fxg {
@@ -633,7 +635,8 @@ hipError_t launch_rhs_weak(const DevMesh& m, const FusedWork& w, const Gas& gas,
   }
 }
 
-// Side slots are 32-bit, as on the split form's path. N = 1 has too few nodes on a line to gain.
+// Side slots are 32-bit, as on the split form's path. N = 1 has too few nodes on a line to gain, FP32-bulk keeps the
+// order of its sums, and boundary sides have no form of these kernels yet (fxg_bcface.h holds what one would need).
 bool weak_supported(int N, int split, int fp32, int nBC, long long nSides) {
   return !split && !fp32 && nBC == 0 && N >= 2 && N <= 7 && nSides * 2LL * (N + 1) * (N + 1) < (1LL << 32);
 }
