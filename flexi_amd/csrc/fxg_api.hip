@@ -274,6 +274,14 @@ int upload(fxg_ctx* c, T** dst, const T* src, size_t count) {
 template <class T>
 int alloc_owned(fxg_ctx* c, T** dst, size_t count) { return upload<T>(c, dst, nullptr, count); }
 
+template <class T>
+void free_owned(fxg_ctx* c, T** p) {
+  if (!*p) return;
+  (void)hipFree(*p);
+  c->owned.erase(std::remove(c->owned.begin(), c->owned.end(), (void*)*p), c->owned.end());
+  *p = nullptr;
+}
+
 // ---------------------------------------------------------------------------------------------
 // Scratch of fxg_calc_timestep_dev_noalloc: a file-scope device array, so that entry point
 // allocates nothing. Each GPU holds its own copy until the process ends; its address on a device
@@ -354,7 +362,11 @@ int ctx_setup(fxg_ctx* c, const fxg_params* p, int K, int S, const int* S2E, con
   c->weak = !c->fused && fxg::weak_supported(c->N, p->splitDG == FXG_SPLITDG_PI,
                                              p->precision == FXG_PREC_FP32_BULK, nBC, S) &&
             !(pipe && std::strcmp(pipe, "classic") == 0);
-  if (!c->fused && !c->weak) {
+  // The four kernels' face arrays. The weak form's two kernels and FP32-bulk, whose own arrays would come on top, do
+  // without them. The FP64 split form uses none either, but its contexts have always held them, and where they end decides
+  // where a caller's arrays come to lie: a step at 32^3, N=7 took 6.97 or 7.12 ms with the same kernels, depending
+  // on what else the process had allocated, and without them more often the latter.
+  if (!c->weak && !(c->fused && p->precision == FXG_PREC_FP32_BULK)) {
     char *Gm, *Gs;
     if (alloc_owned(c, &c->w.Uf_m, 5 * face) || alloc_owned(c, &c->w.Uf_s, 5 * face) ||
         alloc_owned(c, &Gm, 12 * face * gsz) || alloc_owned(c, &Gs, 12 * face * gsz) ||
@@ -411,6 +423,10 @@ int finish_setup(fxg_ctx* c) {
       if (alloc_owned(c, &aff, (size_t)10 * c->K)) return 1;
       HIPCHECK(fxg::find_const_metrics(c->m, aff, c->w.errElem, all, c->stream));
       c->m.aff = all ? aff : nullptr;
+      if (!all) {
+        free_owned(c, &aff);
+        if (c->fused) free_owned(c, &c->w.Flux);  // general terms: more than the neighbours' nodes take
+      }
     }
     if (c->fused && !c->m.aff) {  // the boundary nodes' metric terms, packed for the viscous face kernel
       const bool bulk = c->p.precision == FXG_PREC_FP32_BULK;
@@ -722,11 +738,7 @@ int fxg_set_boundaries(fxg_ctx* c, int nBCs, const int* BC, const int* BoundaryT
   HIPCHECK(hipStreamSynchronize(c->stream));
   if (!c->bcInfo && alloc_owned(c, &c->bcInfo, info.size())) return 1;
   HIPCHECK(hipMemcpy(c->bcInfo, info.data(), info.size() * sizeof(int), hipMemcpyHostToDevice));
-  if (c->refPrim) {
-    (void)hipFree(c->refPrim);
-    c->owned.erase(std::remove(c->owned.begin(), c->owned.end(), (void*)c->refPrim), c->owned.end());
-    c->refPrim = nullptr;
-  }
+  free_owned(c, &c->refPrim);
   if (upload(c, &c->refPrim, nRefState > 0 ? RefStatePrim : nullptr, 6 * (size_t)std::max(1, nRefState))) return 1;
   c->m.nBC = c->nBC;
   c->m.bcInfo = c->bcInfo;
@@ -800,12 +812,11 @@ int fxg_get_gradients(fxg_ctx* c, int nVarLifting, double* gx, double* gy, doubl
       return fail("fxg_get_gradients: no right-hand side has been evaluated for the current state");
     if (!c->rhoG && alloc_owned(c, &c->rhoG, 3 * nodes)) return 1;
     fxg::DevWork w = c->w;
-    if (c->fused || c->weak) {  // the face states' buffer that the next stage writes
+    if (!w.Uf_m) {  // the face states' buffer that the next stage writes
       w.Uf_m = c->fw.FU[1 - c->cur];
       w.Uf_s = w.Uf_m + (size_t)5 * c->nf * c->S;
-    } else {
-      c->faces_of = nullptr;  // it prolongs that state into the same face arrays
     }
+    if (!c->fused && !c->weak) c->faces_of = nullptr;  // it prolongs that state into the same face arrays
     HIPCHECK(fxg::launch_lift_density(c->m, w, c->gas, c->p.nodeType, c->grads_state, c->rhoG, c->stream));
   }
   double* host[3] = {gx, gy, gz};

@@ -63,9 +63,10 @@ struct DevMesh {
 
 // Work arrays of one right-hand side evaluation. Face arrays of U are FP64 (U(5,p,q,side));
 // gradient arrays hold T = double or float (FP32-bulk).
-// On the two-kernel paths a context holds neither these face arrays nor the fluxes.
+// The weak form's two kernels and the split form in FP32-bulk use neither these face arrays nor the fluxes, and their
+// contexts hold none.
 struct DevWork {
-  double* Uf_m;    // (5,0:N,0:N,nSides)
+  double* Uf_m = nullptr;  // (5,0:N,0:N,nSides)
   double* Uf_s;
   void* G;         // volume gradients: (0:N^3, 12, nElems), components gx(u,v,w,T),gy(..),gz(..)
   void* Gf_m;      // face gradients (12,0:N,0:N,nSides)
